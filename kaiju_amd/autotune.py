@@ -26,8 +26,8 @@ CANDIDATES: Dict[str, list] = {
     "emf_j": [(256, 1, 1, LINEAR | NOXCD), (32, 1, 8, 2), (64, 1, 4, 2), (32, 2, 4, NOXCD)],
     "emf_k": [(32, 8, 1, 1), (64, 4, 1, 1), (32, 8, 1, 1 | NOXCD), (256, 1, 1, LINEAR | NOXCD)],
     "flux_i": [(256, 1, 1, LINEAR | NOXCD), (256, 1, 1, LINEAR), (32, 8, 1, 0), (64, 4, 1, NOXCD)],
-    "flux_j": [(32, 8, 1, 0), (32, 8, 1, NOXCD), (16, 16, 1, 1), (64, 4, 1, 1)],
-    "flux_k": [(64, 1, 4, 2), (32, 1, 8, 2), (64, 1, 4, 2 | NOXCD), (16, 1, 16, 2)],
+    "flux_j": [(256, 1, 1, LINEAR), (256, 1, 1, LINEAR | NOXCD), (64, 1, 4, 0), (64, 4, 1, 0)],
+    "flux_k": [(256, 1, 1, LINEAR), (256, 1, 1, LINEAR | NOXCD), (64, 4, 1, 0), (64, 1, 4, 0)],
     "update": [(256, 1, 1, LINEAR | NOXCD), (256, 1, 1, LINEAR), (64, 4, 1, NOXCD), (32, 8, 1, NOXCD)],
 }
 

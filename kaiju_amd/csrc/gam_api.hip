@@ -301,8 +301,8 @@ static bool tiled_stage(int st) {
 }
 static void default_tiles(gam_handle *h) {
     // measured best on MI355X for the 256^3 blast wave (ms per launch, stage
-    // timers): flux_j/flux_k/emf bricks halve their HBM traffic against
-    // row-shaped blocks; the full-box kernels keep plain row-major blocks
+    // timers): emf bricks halve their HBM traffic against row-shaped blocks; the
+    // full-box kernels keep plain row-major blocks
     h->tile[ST_BHALF] = {256, 1, 1, TILE_LINEAR | TILE_NOXCD};
     h->tile[ST_BPOST] = {256, 1, 1, TILE_LINEAR | TILE_NOXCD};
     h->tile[ST_MOM2FACE] = {256, 1, 1, TILE_LINEAR};
@@ -311,8 +311,8 @@ static void default_tiles(gam_handle *h) {
     h->tile[ST_EMF_K] = {32, 8, 1, 1};
     h->tile[ST_UPDATE] = {256, 1, 1, TILE_LINEAR | TILE_NOXCD};
     h->tile[ST_FLUX_I] = {256, 1, 1, TILE_LINEAR | TILE_NOXCD};
-    h->tile[ST_FLUX_J] = {32, 8, 1, 0};
-    h->tile[ST_FLUX_K] = {64, 1, 4, 2};
+    h->tile[ST_FLUX_J] = {256, 1, 1, TILE_LINEAR};   // columns: 64 x 4 bricks within 2%
+    h->tile[ST_FLUX_K] = {256, 1, 1, TILE_LINEAR};
 }
 static inline dim3 tgrid(const gam_handle *h, int st, int nx, int ny, int nz) {
     return dim3((unsigned)tile_blocks(h->tile[st], nx, ny, nz));
@@ -1005,49 +1005,30 @@ static void launch_cpr(gam_handle *h) {
     if (h->prec) launch_cpr_t<float>(h); else launch_cpr_t<double>(h);
 }
 
-// the flux launches with the learned correction added at the store (a block
-// with a correction is periodic, no ring average, so never packed)
-template <int RM, int BO, int MH, int BG, typename R>
-static void launch_flux_corr(gam_handle *h, int d, dim3 gr, dim3 gr2, Tile tl, const WKT<R> &w, const R *nB, const R *hB,
-                             const R *hmag, const R *hGas, R *Flx) {
-    const GVT<R> &g = view<R>(h);
-#define FLUX_CORR(KERN, GRID) hipLaunchKernelGGL(HIP_KERNEL_NAME KERN, (GRID), 256, 0, h->stream, g, tl, h->mp, h->bgv, h->clk, \
-                                                 w.Wn, nB, w.Wh, hB, hmag, hGas, Flx, h->corr, h->corr_scale)
-    if (d == 0) FLUX_CORR((k_flux<0, RM, BO, MH, BG, R, 1>), gr);
-    else if (sizeof(R) == sizeof(float)) {
-        if (d == 1) FLUX_CORR((k_flux<1, RM, BO, MH, BG, R, 1>), gr);
-        else FLUX_CORR((k_flux<2, RM, BO, MH, BG, R, 1>), gr);
-    }
-    else if (d == 1) {   // the plain pairs, then the correction on its own
-        FLUX_CORR((k_flux2<1, RM, BO, MH, BG, R, 0>), gr2);
-        const long n = (long)g.Nip * (g.Njp + 1) * (h->mp.do25D ? 1 : g.Nkp);
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_corr_flux<1, R>), grid1(n), 256, 0, h->stream, g, h->mp, h->clk, Flx, h->corr,
-                           h->corr_scale);
-    }
-    else FLUX_CORR((k_flux2<2, RM, BO, MH, BG, R, 1>), gr2);
-#undef FLUX_CORR
-}
-
 template <int RM, int BO, int MH, int BG, typename R>
 static void launch_flux_bg(gam_handle *h, int d) {
     const GVT<R> &g = view<R>(h);
     const int S = h->s;
-    long nx = g.Nip + (d == 0), ny = g.Njp + (d == 1), nz = (h->mp.do25D ? 1 : g.Nkp) + (d == 2);
+    const int nx = g.Nip + (d == 0), ny = g.Njp, nz = h->mp.do25D ? 1 : g.Nkp;
     const Tile tl = h->tile[ST_FLUX_I + d];
-    dim3 gr = tgrid(h, ST_FLUX_I + d, (int)nx, (int)ny, (int)nz);
-    const dim3 gr2 = tgrid(h, ST_FLUX_I + d, (int)(nx + 1) / 2, (int)ny, (int)nz);   // j, k: interface pairs along i
     const WKT<R> w = wkt<R>(h);
     const R *nB = P<R>(h->B[S]), *hB = P<R>(h->hB), *hmag = P<R>(h->hmag), *hGas = P<R>(h->hGas);
     R *Flx = P<R>(h->Flx);
     StageTimer t(h, ST_FLUX_I + d);
-    if (h->corr) launch_flux_corr<RM, BO, MH, BG, R>(h, d, gr, gr2, tl, w, nB, hB, hmag, hGas, Flx);
-    else if (d == 0) PLAUNCH(h, (k_flux<0, RM, BO, MH, BG, R>), (b_flux<0, RM, BO, MH, BG, R>), gr, 256, g, tl, h->mp, h->bgv, h->clk, w.Wn, nB, w.Wh, hB, hmag, hGas, Flx, h->corr, h->corr_scale);
-    else if (sizeof(R) == sizeof(float)) {   // FP32 bulk: one interface per thread measured as fast as pairs
-        if (d == 1) PLAUNCH(h, (k_flux<1, RM, BO, MH, BG, R>), (b_flux<1, RM, BO, MH, BG, R>), gr, 256, g, tl, h->mp, h->bgv, h->clk, w.Wn, nB, w.Wh, hB, hmag, hGas, Flx, h->corr, h->corr_scale);
-        else PLAUNCH(h, (k_flux<2, RM, BO, MH, BG, R>), (b_flux<2, RM, BO, MH, BG, R>), gr, 256, g, tl, h->mp, h->bgv, h->clk, w.Wn, nB, w.Wh, hB, hmag, hGas, Flx, h->corr, h->corr_scale);
+    const int L = (d == 1 ? ny : nz) + 1;   // interfaces along a j or k column
+    const int kc = d == 0 ? 0 : flux_col_kc(L, (long)nx * (d == 1 ? nz : ny));
+    const dim3 gr = d == 0 ? tgrid(h, ST_FLUX_I, nx, ny, nz)
+                           : tgrid(h, ST_FLUX_I + d, nx, d == 1 ? cdiv(L, kc) : ny, d == 1 ? nz : cdiv(L, kc));
+#define FLUX_ARGS g, tl, h->mp, h->bgv, h->clk, w.Wn, nB, w.Wh, hB, hmag, hGas, Flx, h->corr, h->corr_scale
+    if (h->corr) {   // a block with a correction is periodic, no ring average, so never packed
+        if (d == 0) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_flux<0, RM, BO, MH, BG, R, 1>), gr, 256, 0, h->stream, FLUX_ARGS);
+        else if (d == 1) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_flux_col<1, RM, BO, MH, BG, R, 1>), gr, 256, 0, h->stream, FLUX_ARGS, kc);
+        else hipLaunchKernelGGL(HIP_KERNEL_NAME(k_flux_col<2, RM, BO, MH, BG, R, 1>), gr, 256, 0, h->stream, FLUX_ARGS, kc);
     }
-    else if (d == 1) PLAUNCH(h, (k_flux2<1, RM, BO, MH, BG, R>), (b_flux2<1, RM, BO, MH, BG, R>), gr2, 256, g, tl, h->mp, h->bgv, h->clk, w.Wn, nB, w.Wh, hB, hmag, hGas, Flx, h->corr, h->corr_scale);
-    else PLAUNCH(h, (k_flux2<2, RM, BO, MH, BG, R>), (b_flux2<2, RM, BO, MH, BG, R>), gr2, 256, g, tl, h->mp, h->bgv, h->clk, w.Wn, nB, w.Wh, hB, hmag, hGas, Flx, h->corr, h->corr_scale);
+    else if (d == 0) PLAUNCH(h, (k_flux<0, RM, BO, MH, BG, R>), (b_flux<0, RM, BO, MH, BG, R>), gr, 256, FLUX_ARGS);
+    else if (d == 1) PLAUNCH(h, (k_flux_col<1, RM, BO, MH, BG, R>), (b_flux_col<1, RM, BO, MH, BG, R>), gr, 256, FLUX_ARGS, kc);
+    else PLAUNCH(h, (k_flux_col<2, RM, BO, MH, BG, R>), (b_flux_col<2, RM, BO, MH, BG, R>), gr, 256, FLUX_ARGS, kc);
+#undef FLUX_ARGS
 }
 
 template <int RM, int BO, int MH, typename R>

@@ -187,15 +187,13 @@ __device__ __forceinline__ void pdmlr(R pdmb, R v0, R v1, R v2, R v3, R Qi, R &Q
     Qr = vN + s1 * rmax(R(0.0), rabs(dvR) - q1 * rabs(dv2));
 }
 
-// GetLRs for one variable: recon.F90:125-158 (Cen8LRs) / 162-198 (Up7LRs).
+// GetLRs for one variable: recon.F90:125-158 (Cen8LRs) / 162-198 (Up7LRs),
+// from the volume-weighted points QdV[n] = dV[n] * Q[n].
 // rVi = 1/Vi, formed once per interface by the caller: the reference divides
 // each interpolant by Vi; multiplying by the reciprocal differs by at most
 // an ulp and saves two divisions per variable.
 template <int RM, typename R>
-__device__ __forceinline__ void get_lrs(R pdmb, const R *dV, const R *nQ, const R *Q, R rVi, R &Ql, R &Qr) {
-    R QdV[8];
-#pragma unroll
-    for (int n = 0; n < 8; n++) QdV[n] = dV[n] * Q[n];
+__device__ __forceinline__ void get_lrs_w(R pdmb, const R *QdV, const R *nQ, R rVi, R &Ql, R &Qr) {
     if (RM == 1) {
         R l = up7(QdV[0], QdV[1], QdV[2], QdV[3], QdV[4], QdV[5], QdV[6]) * rVi;
         R r = up7(QdV[7], QdV[6], QdV[5], QdV[4], QdV[3], QdV[2], QdV[1]) * rVi;
@@ -205,6 +203,13 @@ __device__ __forceinline__ void get_lrs(R pdmb, const R *dV, const R *nQ, const 
         R Qi = c8(QdV) * rVi;
         pdmlr(pdmb, nQ[0], nQ[1], nQ[2], nQ[3], Qi, Ql, Qr);
     }
+}
+template <int RM, typename R>
+__device__ __forceinline__ void get_lrs(R pdmb, const R *dV, const R *nQ, const R *Q, R rVi, R &Ql, R &Qr) {
+    R QdV[8];
+#pragma unroll
+    for (int n = 0; n < 8; n++) QdV[n] = dV[n] * Q[n];
+    get_lrs_w<RM>(pdmb, QdV, nQ, rVi, Ql, Qr);
 }
 
 // gamutils.F90:301-321 CellC2P

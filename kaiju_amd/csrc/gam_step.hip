@@ -7,7 +7,7 @@
 //   k_b2f       (G)   H.Bxyz = bFlux2Fld(H.magFlux)  gridutils.F90:281-301,648-680
 //   k_vf        (G)   Mom2Face for the 3 sweeps      fields.F90:110-179,235-285
 //   k_emf<d>    (E)   edge EMFs, one direction each  fields.F90:186-226,288-517
-//   k_flux<d>   (I)   interface fluxes, 3 launches   stress.F90:84-128,204-599
+//   k_flux, k_flux_col (I)  interface fluxes, 3 launches  stress.F90:84-128,204-599
 //   k_ct        (F)   O.magFlux = E2Flux(S.magFlux)  fields.F90:18-51
 //   k_update    (G)   Flux2Deltas + Reynolds + Bxyz + Maxwell/Boris + CellDT min
 //                                                    stress.F90:152-194, mhdgroup.F90:79-442,
@@ -26,7 +26,24 @@
 // CFL bound stay FP64 (values are promoted on load).
 #include "gam_common.h"
 
+// k_flux_col's register budget: two waves per SIMD (see there)
+#ifdef GAM_EMU
+#define FLUX_COL_WAVES
+#else
+#define FLUX_COL_WAVES __attribute__((amdgpu_waves_per_eu(2)))
+#endif
+
 // ----------------------------------------------------------------- helpers
+// p[i], i >= 0, with the byte offset formed in 32 bits: the load takes p from
+// scalar registers and one offset register shared by all slabs, where a 64-bit
+// index costs an address add and a register pair per slab.  One slab stays
+// below 4 GB: a block of 2^29 points would need over 370 GB in either precision.
+template <typename T> __device__ __forceinline__ T &at32(T *p, int i) {
+    return *(T *)((char *)p + (unsigned)i * (unsigned)sizeof(T));
+}
+template <typename T> __device__ __forceinline__ T at32(const T *p, int i) {
+    return *(const T *)((const char *)p + (unsigned)i * (unsigned)sizeof(T));
+}
 // Streaming (non-temporal) store, used where it measured faster: the Mom2Face
 // and update outputs, which later stages read back from HBM anyway.
 template <typename T> __device__ __forceinline__ void st_nt(T *p, T v) {
@@ -639,15 +656,15 @@ __device__ __forceinline__ void lr_flux(const GVT<R> &g, const MP &m, const BGV 
     const int st = cstride(g, DN);
     R T[9];
 #pragma unroll
-    for (int q = 0; q < 9; q++) T[q] = g.Tf[nf * (q + 9 * DN) + f];
-    const R faB = g.face[nf * DN + f];
-    const R Bn = MHD ? hmag[nf * DN + f] / faB : R(0.0);
+    for (int q = 0; q < 9; q++) T[q] = at32(g.Tf + nf * (q + 9 * DN), f);
+    const R faB = at32(g.face + nf * DN, f);
+    const R Bn = MHD ? at32(hmag + nf * DN, f) / faB : R(0.0);
     R B0f[3] = {0, 0, 0}, B0n = R(0.0);
     const bool bgon = MHD && BG;
     if (bgon) {   // stress.F90:302-305
 #pragma unroll
-        for (int x = 0; x < 3; x++) B0f[x] = R(bg.fcB0[nc * (x + 3 * DN) + c]);
-        B0n = R(bg.bFlux0[nc * DN + c]) / faB;
+        for (int x = 0; x < 3; x++) B0f[x] = R(at32(bg.fcB0 + nc * (x + 3 * DN), c));
+        B0n = R(at32(bg.bFlux0 + nc * DN, c)) / faB;
     }
     const R Ca = R(m.Ca);
     R VaD = R(0.0);
@@ -678,7 +695,7 @@ __device__ __forceinline__ void lr_flux(const GVT<R> &g, const MP &m, const BGV 
         if (Vn >= R(1.5) * Ca) {
 #pragma unroll
             for (int v = 0; v < 5; v++) {
-                R dCon = hGas[nc * v + c] - hGas[nc * v + c - st];
+                R dCon = at32(hGas + nc * v, c) - at32(hGas + nc * v, c - st);
                 gF[v] = gF[v] - Ca * dCon;
             }
         }
@@ -726,64 +743,9 @@ __device__ __forceinline__ void face_flux(const GVT<R> &g, const MP &m, const BG
     lr_flux<DN, BORIS, MHD, BG>(g, m, bg, hmag, hGas, c, f, PL, PR, MagL, MagR, out);
 }
 
-// The same for the two interfaces at cells c and c + 1 (adjacent along i),
-// for a j or k stencil: every stencil point is one 2-wide load.  B's results
-// are formed whether or not the caller keeps them (c + 1 is always a cell of
-// the array: at most the first ghost past the active range).
-#ifdef GAM_EMU
-template <typename R> __device__ __forceinline__ void ld2(const R *p, R &a, R &b) { a = p[0]; b = p[1]; }
-#else
-template <typename R> struct P2 { typedef R T __attribute__((ext_vector_type(2), aligned(sizeof(R)))); };
-template <typename R> __device__ __forceinline__ void ld2(const R *p, R &a, R &b) {
-    const typename P2<R>::T v = *(const typename P2<R>::T *)p;
-    a = v.x;
-    b = v.y;
-}
-#endif
-template <int DN, int RM, int BORIS, int MHD, int BG, typename R>
-__device__ __forceinline__ void face_flux2(const GVT<R> &g, const MP &m, const BGV &bg,
-                                           const R *__restrict__ Wn, const R *__restrict__ nB,
-                                           const R *__restrict__ Wh, const R *__restrict__ hB,
-                                           const R *__restrict__ hmag, const R *__restrict__ hGas,
-                                           int c, int f, R *outA, R *outB) {
-    const size_t nc = g.nc;
-    const int st = cstride(g, DN);
-    const R pdmb = R(m.pdmb);
-    R VA[8], VB[8];
-#pragma unroll
-    for (int n = 0; n < 8; n++) ld2(g.vol + c + (n - 4) * st, VA[n], VB[n]);
-    const R rVA = R(1) / c8(VA), rVB = R(1) / c8(VB);
-    R PLA[5], PRA[5], PLB[5], PRB[5];
-    R MLA[3] = {0, 0, 0}, MRA[3] = {0, 0, 0}, MLB[3] = {0, 0, 0}, MRB[3] = {0, 0, 0};
-    if (MHD) {
-        const R *limB = m.doLFMLim ? nB : hB;
-#pragma unroll
-        for (int d = 0; d < 3; d++) {
-            R QA[8], QB[8], nA[4], nBq[4];
-#pragma unroll
-            for (int n = 0; n < 8; n++) ld2(hB + nc * d + c + (n - 4) * st, QA[n], QB[n]);
-#pragma unroll
-            for (int n = 0; n < 4; n++) ld2(limB + nc * d + c + (n - 2) * st, nA[n], nBq[n]);
-            get_lrs<RM>(pdmb, VA, nA, QA, rVA, MLA[d], MRA[d]);
-            get_lrs<RM>(pdmb, VB, nBq, QB, rVB, MLB[d], MRB[d]);
-        }
-    }
-#pragma unroll
-    for (int v = 0; v < 5; v++) {
-        R QA[8], QB[8], nA[4], nBq[4];
-#pragma unroll
-        for (int n = 0; n < 8; n++) ld2(Wh + nc * v + c + (n - 4) * st, QA[n], QB[n]);
-#pragma unroll
-        for (int n = 0; n < 4; n++) ld2(Wn + nc * v + c + (n - 2) * st, nA[n], nBq[n]);
-        get_lrs<RM>(pdmb, VA, nA, QA, rVA, PLA[v], PRA[v]);
-        get_lrs<RM>(pdmb, VB, nBq, QB, rVB, PLB[v], PRB[v]);
-    }
-    lr_flux<DN, BORIS, MHD, BG>(g, m, bg, hmag, hGas, c, f, PLA, PRA, MLA, MRA, outA);
-    lr_flux<DN, BORIS, MHD, BG>(g, m, bg, hmag, hGas, c + 1, f + 1, PLB, PRB, MLB, MRB, outB);
-}
-
-// Interface fluxes in direction DN for the interface box
-// DN=I: [is,ie+1]x[js,je]x[ks,ke]  (k range a single slice in 2.5D)
+// Fluxes of the i interfaces, box [is,ie+1]x[js,je]x[ks,ke] (k a single slice
+// in 2.5D), one interface per thread: the 8 points of a stencil lie in the
+// cache lines its neighbouring lanes load.
 // Output slabs Flx[(8*DN + v)*nc + c], v = 0..4 gas, 5..7 magnetic.  CORR = 1:
 // with the learned correction (corr, cs) added to the gas fluxes (corr_add); a
 // separate instantiation, so the plain kernels keep their registers.
@@ -793,15 +755,15 @@ __device__ __forceinline__ void b_flux(const unsigned vb, GVT<R> g, Tile t, MP m
                                               const R *__restrict__ Wh, const R *__restrict__ hB,
                                               const R *__restrict__ hmag, const R *__restrict__ hGas,
                                               R *__restrict__ Flx, const float *__restrict__ corr, double cs) {
-    const int nx = g.Nip + (DN == 0), ny = g.Njp + (DN == 1), nz = (m.do25D ? 1 : g.Nkp) + (DN == 2);
+    static_assert(DN == 0, "the j and k interfaces go through b_flux_col");
     int a, b, cz;
-    if (!tile_pos(vb, t, nx, ny, nz, a, b, cz) || clk->halt) return;
+    if (!tile_pos(vb, t, g.Nip + 1, g.Njp, m.do25D ? 1 : g.Nkp, a, b, cz) || clk->halt) return;
     const int i = a + g.nG, j = b + g.nG, k = cz + g.nG;
     const size_t nc = g.nc;
     const int c = ci(g, i, j, k);
     R o[8];
     face_flux<DN, RM, BORIS, MHD, BG>(g, m, bg, Wn, nB, Wh, hB, hmag, hGas, c, fi(g, i, j, k), o);
-    if (CORR && !(DN == 2 && m.do25D)) {   // CORR instantiations run with a correction set only
+    if (CORR) {   // CORR instantiations run with a correction set only
         const double A = (double)g.face[(size_t)g.nf * DN + fi(g, i, j, k)];
         const float *oc = corr + pimg(g, i, j, k) * 8;
 #pragma unroll
@@ -819,67 +781,122 @@ __global__ void __launch_bounds__(256) k_flux(GVT<R> g, Tile t, MP m, BGV bg, co
     b_flux<DN, RM, BORIS, MHD, BG, R, CORR>(blockIdx.x, g, t, m, bg, clk, Wn, nB, Wh, hB, hmag, hGas, Flx, corr, cs);
 }
 
-// j or k interfaces two at a time along i (face_flux2): thread (a, b, c) of
-// the box ceil(nx/2) x ny x nz owns interfaces i = 2a and 2a + 1.
+// Fluxes of the j or k interfaces.  A thread walks up to kc interfaces along
+// DN, lanes along i: the 8-point windows of the volume-weighted variables stay
+// in registers and move by one point per interface, so each point is loaded and
+// weighted once instead of 8 times (104 loads per interface become 17).  The
+// windows of the volume (8 points) and of the limiter state (4) live in LDS
+// rings private to the thread (no barrier): in registers they cost the FP64
+// kernel its second wave per SIMD.  The next interface's points are loaded ahead
+// of this one's flux arithmetic and land during it; where the FP64 flux itself
+// needs the registers (Boris, background, correction: they would spill), after
+// it.  Bound by VALU issue, 1430 (FP64) and 1250 (FP32) vector instructions per
+// interface, 0.6 ms at 256^3.  Measured there, ms per launch j / k: FP32 bulk
+// 0.79 / 0.91 (one interface per thread, no windows) -> 0.64 / 0.65; FP64 1.37 / 1.46
+// (two interfaces along i per thread) -> 1.24 / 1.26.
 template <int DN, int RM, int BORIS, int MHD, int BG, typename R, int CORR = 0>
-__device__ __forceinline__ void b_flux2(const unsigned vb, GVT<R> g, Tile t, MP m, BGV bg, const DClock *__restrict__ clk,
-                                        const R *__restrict__ Wn, const R *__restrict__ nB,
-                                        const R *__restrict__ Wh, const R *__restrict__ hB,
-                                        const R *__restrict__ hmag, const R *__restrict__ hGas,
-                                        R *__restrict__ Flx, const float *__restrict__ corr, double cs) {
-    static_assert(DN != 0, "pairs along i serve the j and k interfaces");
-    const int nx = g.Nip, ny = g.Njp + (DN == 1), nz = (m.do25D ? 1 : g.Nkp) + (DN == 2);
+__device__ __forceinline__ void b_flux_col(const unsigned vb, GVT<R> g, Tile t, MP m, BGV bg, const DClock *__restrict__ clk,
+                                           const R *__restrict__ Wn, const R *__restrict__ nB,
+                                           const R *__restrict__ Wh, const R *__restrict__ hB,
+                                           const R *__restrict__ hmag, const R *__restrict__ hGas,
+                                           R *__restrict__ Flx, const float *__restrict__ corr, double cs, int kc) {
+    static_assert(DN != 0, "columns along j or k");
+    constexpr int NV = MHD ? 8 : 5;
+    __shared__ R lim[4][NV][256];
+    const int ny = g.Njp, nz = m.do25D ? 1 : g.Nkp;
+    const int L = (DN == 1 ? ny : nz) + 1, nseg = cdiv(L, kc);
     int a, b, cz;
-    if (!tile_pos(vb, t, (nx + 1) / 2, ny, nz, a, b, cz) || clk->halt) return;
-    const int i = 2 * a + g.nG, j = b + g.nG, k = cz + g.nG;
+    if (!tile_pos(vb, t, g.Nip, DN == 1 ? nseg : ny, DN == 1 ? nz : nseg, a, b, cz) || clk->halt) return;
+    const int s0 = (DN == 1 ? b : cz) * kc, ns = L - s0 < kc ? L - s0 : kc;
+    const int i = a + g.nG, j = (DN == 1 ? s0 : b) + g.nG, k = (DN == 2 ? s0 : cz) + g.nG;
     const size_t nc = g.nc;
-    const int c = ci(g, i, j, k);
-    R oA[8], oB[8];
-    face_flux2<DN, RM, BORIS, MHD, BG>(g, m, bg, Wn, nB, Wh, hB, hmag, hGas, c, fi(g, i, j, k), oA, oB);
-    const bool two = 2 * a + 1 < nx;
-    if (CORR && !(DN == 2 && m.do25D)) {   // CORR instantiations run with a correction set only
-        const int f = fi(g, i, j, k);
-        const double A = (double)g.face[(size_t)g.nf * DN + f];
-        const float *oc = corr + pimg(g, i, j, k) * 8;
+    const int st = cstride(g, DN), fst = fstride(g, DN), tid = threadIdx.x;
+    const R pdmb = R(m.pdmb);
+    const R *limB = m.doLFMLim ? nB : hB;
+    int c = ci(g, i, j, k), f = fi(g, i, j, k);
+    __shared__ R vols[8][256];
+    R V[8], Q[NV][8], nl[NV];   // nl: the newest point of each limiter window
 #pragma unroll
-        for (int v = 0; v < 5; v++) oA[v] = corr_add(oA[v], cs, A, oc[v]);
-        if (two) {
-            const double AB = (double)g.face[(size_t)g.nf * DN + f + 1];
-            const float *ob = corr + pimg(g, i + 1, j, k) * 8;
+    for (int n = 0; n < 8; n++) vols[n][tid] = V[n] = at32(g.vol, c + (n - 4) * st);
 #pragma unroll
-            for (int v = 0; v < 5; v++) oB[v] = corr_add(oB[v], cs, AB, ob[v]);
-        }
+    for (int v = 0; v < NV; v++) {
+        const R *q = v < 5 ? Wh + nc * v : hB + nc * (v - 5), *l = v < 5 ? Wn + nc * v : limB + nc * (v - 5);
+#pragma unroll
+        for (int n = 0; n < 8; n++) Q[v][n] = V[n] * at32(q, c + (n - 4) * st);
+#pragma unroll
+        for (int n = 0; n < 3; n++) lim[n][v][tid] = at32(l, c + (n - 2) * st);
+        nl[v] = at32(l, c + st);
     }
+    constexpr bool EARLY = sizeof(R) == sizeof(float) || !(BORIS || BG || CORR);
+#pragma unroll 1
+    for (int s = 0; s < ns; s++) {
+        R pV, pq[NV];
+        auto fetch = [&]() {   // the next interface's new points (the last one's may lie past the box: not read)
+            const bool more = s + 1 < ns;
+            const int cq = more ? c + 4 * st : c, cl = more ? c + 2 * st : c;
+            pV = at32(g.vol, cq);
 #pragma unroll
-    for (int v = 0; v < (MHD ? 8 : 5); v++) {
-        Flx[nc * (8 * DN + v) + c] = oA[v];
-        if (two) Flx[nc * (8 * DN + v) + c + 1] = oB[v];
+            for (int v = 0; v < NV; v++) {
+                const R *q = v < 5 ? Wh + nc * v : hB + nc * (v - 5), *l = v < 5 ? Wn + nc * v : limB + nc * (v - 5);
+                pq[v] = at32(q, cq);
+                nl[v] = at32(l, cl);
+            }
+        };
+#pragma unroll
+        for (int n = 0; n < 8; n++) V[n] = vols[(s + n) & 7][tid];
+        const R rVi = R(1) / c8(V);
+        R PL[5], PR[5], MagL[3] = {0, 0, 0}, MagR[3] = {0, 0, 0};
+#pragma unroll
+        for (int v = 0; v < NV; v++) {
+            const R nQ[4] = {lim[s & 3][v][tid], lim[(s + 1) & 3][v][tid], lim[(s + 2) & 3][v][tid], nl[v]};
+            if (v < 5) get_lrs_w<RM>(pdmb, Q[v], nQ, rVi, PL[v], PR[v]);
+            else get_lrs_w<RM>(pdmb, Q[v], nQ, rVi, MagL[v - 5], MagR[v - 5]);
+            lim[(s + 3) & 3][v][tid] = nl[v];
+        }
+        if (EARLY) fetch();
+        R o[8];
+        lr_flux<DN, BORIS, MHD, BG>(g, m, bg, hmag, hGas, c, f, PL, PR, MagL, MagR, o);
+        if (CORR && !(DN == 2 && m.do25D)) {   // CORR instantiations run with a correction set only
+            const double A = (double)g.face[(size_t)g.nf * DN + f];
+            const float *oc = corr + pimg(g, i, DN == 1 ? j + s : j, DN == 2 ? k + s : k) * 8;
+#pragma unroll
+            for (int v = 0; v < 5; v++) o[v] = corr_add(o[v], cs, A, oc[v]);
+        }
+#pragma unroll
+        for (int v = 0; v < NV; v++) at32(Flx + nc * (8 * DN + v), c) = o[v];
+        if (!EARLY) fetch();
+        vols[s & 7][tid] = pV;
+#pragma unroll
+        for (int v = 0; v < NV; v++) {
+#pragma unroll
+            for (int n = 0; n < 7; n++) Q[v][n] = Q[v][n + 1];
+            Q[v][7] = pV * pq[v];
+        }
+        c += st;
+        f += fst;
     }
 }
 template <int DN, int RM, int BORIS, int MHD, int BG, typename R, int CORR = 0>
-__global__ void __launch_bounds__(256) k_flux2(GVT<R> g, Tile t, MP m, BGV bg, const DClock *__restrict__ clk,
-                                               const R *__restrict__ Wn, const R *__restrict__ nB,
-                                               const R *__restrict__ Wh, const R *__restrict__ hB,
-                                               const R *__restrict__ hmag, const R *__restrict__ hGas,
-                                               R *__restrict__ Flx, const float *__restrict__ corr, double cs) {
-    b_flux2<DN, RM, BORIS, MHD, BG, R, CORR>(blockIdx.x, g, t, m, bg, clk, Wn, nB, Wh, hB, hmag, hGas, Flx, corr, cs);
+__global__ void __launch_bounds__(256) FLUX_COL_WAVES k_flux_col(GVT<R> g, Tile t, MP m, BGV bg, const DClock *__restrict__ clk,
+                                                  const R *__restrict__ Wn, const R *__restrict__ nB,
+                                                  const R *__restrict__ Wh, const R *__restrict__ hB,
+                                                  const R *__restrict__ hmag, const R *__restrict__ hGas,
+                                                  R *__restrict__ Flx, const float *__restrict__ corr, double cs, int kc) {
+    b_flux_col<DN, RM, BORIS, MHD, BG, R, CORR>(blockIdx.x, g, t, m, bg, clk, Wn, nB, Wh, hB, hmag, hGas, Flx, corr, cs, kc);
 }
-// The correction of the gas fluxes in direction DN on their own (corr_add on the
-// stored fluxes of the flux box), for the one flux kernel whose correcting
-// instantiation the compiler cannot fit in its plain registers (the FP64 j pairs).
-template <int DN, typename R>
-__global__ void __launch_bounds__(256) k_corr_flux(GVT<R> g, MP m, const DClock *__restrict__ clk, R *__restrict__ Flx,
-                                                   const float *__restrict__ corr, double cs) {
-    const int nx = g.Nip + (DN == 0), ny = g.Njp + (DN == 1), nz = (m.do25D ? 1 : g.Nkp) + (DN == 2);
-    const long q = (long)blockIdx.x * 256 + threadIdx.x;
-    if (q >= (long)nx * ny * nz || clk->halt || (DN == 2 && m.do25D)) return;
-    const int i = (int)(q % nx) + g.nG, j = (int)((q / nx) % ny) + g.nG, k = (int)(q / ((long)nx * ny)) + g.nG;
-    const size_t nc = g.nc;
-    const int c = ci(g, i, j, k);
-    const double A = (double)g.face[(size_t)g.nf * DN + fi(g, i, j, k)];
-    const float *oc = corr + pimg(g, i, j, k) * 8;
-#pragma unroll
-    for (int v = 0; v < 5; v++) Flx[nc * (8 * DN + v) + c] = corr_add(Flx[nc * (8 * DN + v) + c], cs, A, oc[v]);
+
+// Interfaces per k_flux_col thread for columns of L interfaces over `cols`
+// lanes (speed only).  One round of resident blocks is 2 waves on each of 1024
+// SIMDs.  A column start loads 7 points that an interface inside a column does
+// not, so columns are long, at least 24 (lengths 33 to 129 differ by 3% at
+// 256^3), where that still gives four rounds of blocks, which even out the last
+// one; a smaller block takes whatever length fills one round, down to a single
+// interface.
+static inline int flux_col_kc(int L, long cols) {
+    const long round = 2L * 64 * 1024;
+    auto len = [&](long lanes) { return cdiv(L, (int)std::min<long>(L, std::max(1L, (lanes + cols - 1) / cols))); };
+    const int four = len(4 * round);
+    return four >= 24 ? four : std::min(24, len(round));
 }
 
 // ----------------------------------------------------------------- CT update
@@ -1711,7 +1728,7 @@ __global__ void __launch_bounds__(256) k_sum_ordered(const double *__restrict__ 
 // the update stays conservative and E2Flux keeps div.B exact.  A ghost cell
 // uses the o of its periodic image (the step's boundaries are periodic), so
 // the two copies of a boundary face or edge get one correction.  The step
-// adds it where k_emf/k_emf_jcol and k_flux/k_flux2 store (corr_add); the
+// adds it where k_emf/k_emf_jcol and k_flux/k_flux_col store (corr_add); the
 // training kernels below use the same faces (flux_box) and edges (edge_active).
 template <typename R> __device__ __forceinline__ bool flux_box(const GVT<R> &g, int do25D, int d, int i, int j, int k) {
     const int a0 = g.nG;
