@@ -564,9 +564,11 @@ extern "C" int gam_set_corners(gam_handle *h, const double *xyz) {
     GVw w = gvw(h);
     for (int d = 0; d < 3; d++) {
         long n = (long)(g.Ni + (d == 0)) * (g.Nj + (d == 1)) * (g.Nk + (d == 2));
-        hipLaunchKernelGGL(k_faces, grid1(n), 256, 0, h->stream, w, d);
+        if (h->prec) hipLaunchKernelGGL(k_faces<true>, grid1(n), 256, 0, h->stream, w, d);
+        else hipLaunchKernelGGL(k_faces<false>, grid1(n), 256, 0, h->stream, w, d);
     }
-    hipLaunchKernelGGL(k_volume, grid1(g.nc), 256, 0, h->stream, w);
+    if (h->prec) hipLaunchKernelGGL(k_volume<true>, grid1(g.nc), 256, 0, h->stream, w);
+    else hipLaunchKernelGGL(k_volume<false>, grid1(g.nc), 256, 0, h->stream, w);
     if (h->ring.on) {   // RingGridFix (init.F90:968), before the edge systems read the face normals
         hipLaunchKernelGGL(k_ring_dk, grid1((long)g.Ni * g.Nk * h->ring.nring * 2), 256, 0, h->stream, w, h->ring);
         hipLaunchKernelGGL(k_ring_ghost_geom, grid1((long)(g.Ni + 1) * (g.Nk + 1) * g.nG * 2), 256, 0, h->stream, w);

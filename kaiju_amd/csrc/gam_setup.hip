@@ -45,7 +45,14 @@ __global__ void k_fill(double *p, size_t n, double v) {
 }
 
 // Faces of direction d: area + centre (quadrature.F90:159-221 with A=1 and A=r)
-// and the face triad (init.F90:873-906, doQuadFT = F).
+// and the face triad (init.F90:873-906, doQuadFT = F).  POINTS: the sums point by
+// point, as the reference takes them; else through the moments of the area (the
+// same rule, other roundings).  FP32 bulk keeps the point sums here and in
+// k_volume: its step reads face and cell centres through differences rounded to
+// FP32 (k_b2f_coef), where the last bits of the FP64 centres flip single
+// roundings, and in a low-beta field those reach magFlux at 5e-9.  Bound by FP64
+// issue (the square root): 0.75 -> 0.45 ms per launch at 128^3.
+template <bool POINTS>
 __global__ void __launch_bounds__(256) k_faces(GVw g, int d) {
     const int nx = g.Ni + (d == 0), ny = g.Nj + (d == 1), nz = g.Nk + (d == 2);
     int idx = blockIdx.x * blockDim.x + threadIdx.x;
@@ -61,21 +68,52 @@ __global__ void __launch_bounds__(256) k_faces(GVw g, int d) {
     dy[0] = f1[1] - f0[1]; dy[1] = f2[1] - f0[1]; dy[2] = f3[1] + f0[1] - f2[1] - f1[1];
     dz[0] = f1[2] - f0[2]; dz[1] = f2[2] - f0[2]; dz[2] = f3[2] + f0[2] - f2[2] - f1[2];
     double A = 0.0, cx = 0.0, cy = 0.0, cz = 0.0;
-    for (int a = 0; a < 12; a++)
-        for (int b = 0; b < 12; b++) {
-            double eta = 0.5 * (1 + gA[a]), psi = 0.5 * (1 + gA[b]);
-            double w = gW[a] * gW[b];
-            double xp = f0[0] + dx[0] * eta + dx[1] * psi + dx[2] * eta * psi;
-            double yp = f0[1] + dy[0] * eta + dy[1] * psi + dy[2] * eta * psi;
-            double zp = f0[2] + dz[0] * eta + dz[1] * psi + dz[2] * eta * psi;
-            double eV[3] = {dx[0] + dx[2] * psi, dy[0] + dy[2] * psi, dz[0] + dz[2] * psi};
-            double pV[3] = {dx[1] + dx[2] * eta, dy[1] + dy[2] * eta, dz[1] + dz[2] * eta};
-            double cr[3];
-            cross3(eV, pV, cr);
-            double area = 0.25 * nrm3(cr) * w;
-            A = A + area * 1.0;
-            cx = cx + area * xp; cy = cy + area * yp; cz = cz + area * zp;
+    if constexpr (POINTS) {
+        for (int a = 0; a < 12; a++)
+            for (int b = 0; b < 12; b++) {
+                double eta = 0.5 * (1 + gA[a]), psi = 0.5 * (1 + gA[b]);
+                double w = gW[a] * gW[b];
+                double xp = f0[0] + dx[0] * eta + dx[1] * psi + dx[2] * eta * psi;
+                double yp = f0[1] + dy[0] * eta + dy[1] * psi + dy[2] * eta * psi;
+                double zp = f0[2] + dz[0] * eta + dz[1] * psi + dz[2] * eta * psi;
+                double eV[3] = {dx[0] + dx[2] * psi, dy[0] + dy[2] * psi, dz[0] + dz[2] * psi};
+                double pV[3] = {dx[1] + dx[2] * eta, dy[1] + dy[2] * eta, dz[1] + dz[2] * eta};
+                double cr[3];
+                cross3(eV, pV, cr);
+                double area = 0.25 * nrm3(cr) * w;
+                A = A + area * 1.0;
+                cx = cx + area * xp; cy = cy + area * yp; cz = cz + area * zp;
+            }
+    } else {
+        // On a bilinear face x = f0 + eta e1 + psi e2 + eta psi e3 the normal
+        // (e1 + psi e3) x (e2 + eta e3) is linear in eta and psi, and the centre
+        // needs only the area's moments in 1, eta, psi and eta psi: a Gauss point
+        // costs one norm and few products.
+        const double e1[3] = {dx[0], dy[0], dz[0]}, e2[3] = {dx[1], dy[1], dz[1]}, e3[3] = {dx[2], dy[2], dz[2]};
+        double n0v[3], nE[3], nP[3];
+        cross3(e1, e2, n0v);
+        cross3(e1, e3, nE);
+        cross3(e3, e2, nP);
+        double mE = 0.0, mP = 0.0, mEP = 0.0;
+        for (int a = 0; a < 12; a++) {
+            const double eta = 0.5 * (1 + gA[a]);
+            const double na[3] = {n0v[0] + eta * nE[0], n0v[1] + eta * nE[1], n0v[2] + eta * nE[2]};
+            double s0 = 0.0, s1 = 0.0;
+            for (int b = 0; b < 12; b++) {
+                const double psi = 0.5 * (1 + gA[b]);
+                const double cr[3] = {na[0] + psi * nP[0], na[1] + psi * nP[1], na[2] + psi * nP[2]};
+                const double area = nrm3(cr) * gW[b];
+                s0 = s0 + area;
+                s1 = s1 + area * psi;
+            }
+            const double w = 0.25 * gW[a];
+            A = A + w * s0; mE = mE + w * eta * s0;
+            mP = mP + w * s1; mEP = mEP + w * eta * s1;
         }
+        cx = f0[0] * A + e1[0] * mE + e2[0] * mP + e3[0] * mEP;
+        cy = f0[1] * A + e1[1] * mE + e2[1] * mP + e3[1] * mEP;
+        cz = f0[2] * A + e1[2] * mE + e2[2] * mP + e3[2] * mEP;
+    }
     const size_t nf = g.nf;
     int f = fiw(g, i, j, k);
     g.xfc[nf * (0 + 3 * d) + f] = cx / A;
@@ -115,8 +153,7 @@ __global__ void __launch_bounds__(256) k_faces(GVw g, int d) {
     }
 }
 
-// quadrature.F90:42-100 GaussianVolumeIntegral; W selects the integrand:
-// 0 = CellDV (metric.F90:298-307), 1 = blast-wave gas (prob.F90:280-297)
+// the blast wave's initial condition
 struct BWp { double x0, y0, z0, D0, P0, pRat, dRat, rC; };
 
 // quadrature.F90:42-100 GaussianVolumeIntegral of the integrand fn(x, y, z, W5)
@@ -156,19 +193,61 @@ __device__ void gauss_volume_fn(const double C[8][3], const Fn &fn, double *out5
             }
 }
 
-// W selects the integrand: 0 = CellDV (metric.F90:298-307), 1 = blast-wave gas
-// (prob.F90:280-297)
-template <int W>
-__device__ void gauss_volume(const double C[8][3], const BWp &bw, double *out5) {
-    gauss_volume_fn(C, [&](double x, double y, double z, double *Wp) {
-        if (W == 0) { Wp[0] = 1; Wp[1] = x; Wp[2] = y; Wp[3] = z; Wp[4] = 0; }
-        else {
-            double R = sqrt(sq(x - bw.x0) + sq(y - bw.y0) + sq(z - bw.z0));
-            double D = bw.D0, P = bw.P0;
-            if (R <= bw.rC) { D = bw.dRat * D; P = bw.pRat * P; }
-            Wp[0] = D; Wp[1] = 0.0; Wp[2] = 0.0; Wp[3] = 0.0; Wp[4] = P;
-        }
-    }, out5);
+// CellDV (metric.F90:298-307): the cell's volume and its first moments (out4 =
+// V, int x, int y, int z).  On a trilinear cell det J is a polynomial of degree 2 per axis
+// and x det J one of degree 3, so the 27-point Simpson rule gives the integrals
+// exactly; the 12-point Gauss rule would only repeat that with 1728
+// points.  |det J| equals det J up to a sign where det J keeps its sign: its 27
+// Bernstein coefficients (the nodes' values combined per axis) all of one sign
+// prove that.  False: they are not, the cell may be folded, out4 is not set.
+__device__ bool simpson_volume(const double C[8][3], double *out4) {
+    // corner n = (i + 2 j + 4 k) from cell_coords' order
+    const int ord[8] = {0, 1, 3, 2, 4, 5, 7, 6};
+    auto V = [&](int i, int j, int k, int x) { return C[ord[i + 2 * j + 4 * k]][x]; };
+    auto lerp = [](double a, double b, int t) { return t == 0 ? a : (t == 2 ? b : 0.5 * (a + b)); };
+    double d[27], V0 = 0.0, m[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int c = 0; c < 3; c++)
+#pragma unroll
+        for (int b = 0; b < 3; b++)
+#pragma unroll
+            for (int a = 0; a < 3; a++) {
+                double J[3][3], xp[3];
+#pragma unroll
+                for (int x = 0; x < 3; x++) {
+                    const double x00 = lerp(V(0, 0, 0, x), V(1, 0, 0, x), a), x10 = lerp(V(0, 1, 0, x), V(1, 1, 0, x), a);
+                    const double x01 = lerp(V(0, 0, 1, x), V(1, 0, 1, x), a), x11 = lerp(V(0, 1, 1, x), V(1, 1, 1, x), a);
+                    const double y0 = lerp(x00, x10, b), y1 = lerp(x01, x11, b);
+                    xp[x] = lerp(y0, y1, c);
+                    J[x][0] = 0.5 * lerp(lerp(V(1, 0, 0, x) - V(0, 0, 0, x), V(1, 1, 0, x) - V(0, 1, 0, x), b),
+                                         lerp(V(1, 0, 1, x) - V(0, 0, 1, x), V(1, 1, 1, x) - V(0, 1, 1, x), b), c);
+                    J[x][1] = 0.5 * lerp(x10 - x00, x11 - x01, c);
+                    J[x][2] = 0.5 * (y1 - y0);
+                }
+                const double det = J[0][0] * (J[1][1] * J[2][2] - J[1][2] * J[2][1])
+                                 - J[0][1] * (J[1][0] * J[2][2] - J[1][2] * J[2][0])
+                                 + J[0][2] * (J[1][0] * J[2][1] - J[1][1] * J[2][0]);
+                const double w = ((a == 1 ? 4.0 : 1.0) * (b == 1 ? 4.0 : 1.0) * (c == 1 ? 4.0 : 1.0)) / 27.0;
+                d[a + 3 * (b + 3 * c)] = det;
+                V0 = V0 + w * det;
+#pragma unroll
+                for (int x = 0; x < 3; x++) m[x] = m[x] + w * det * xp[x];
+            }
+    int st = 1;   // values at the nodes -> Bernstein coefficients, one axis at a time
+#pragma unroll
+    for (int ax = 0; ax < 3; ax++, st *= 3)
+#pragma unroll
+        for (int q = 0; q < 27; q++)
+            if ((q / st) % 3 == 1) d[q] = 2.0 * d[q] - 0.5 * (d[q - st] + d[q + st]);
+    double lo = d[0], hi = d[0];
+#pragma unroll
+    for (int q = 1; q < 27; q++) { lo = fmin(lo, d[q]); hi = fmax(hi, d[q]); }
+    if (!(lo > 0.0 || hi < 0.0)) return false;
+    const double sg = lo > 0.0 ? 1.0 : -1.0;
+    out4[0] = sg * V0;
+#pragma unroll
+    for (int x = 0; x < 3; x++) out4[1 + x] = sg * m[x];
+    return true;
 }
 
 __device__ __forceinline__ void cell_coords(const GVw &g, int i, int j, int k, double C[8][3]) {   // metric.F90:133-148
@@ -176,15 +255,18 @@ __device__ __forceinline__ void cell_coords(const GVw &g, int i, int j, int k, d
     xyzv(g, i, j, k + 1, C[4]); xyzv(g, i + 1, j, k + 1, C[5]); xyzv(g, i + 1, j + 1, k + 1, C[6]); xyzv(g, i, j + 1, k + 1, C[7]);
 }
 
-// init.F90:922-965 volume, barycentre, di/dj/dk (needs faces first)
+// init.F90:922-965 volume, barycentre, di/dj/dk (needs faces first).  POINTS: the
+// 1728-point quadrature on every cell (see k_faces), else only where simpson_volume
+// declines.  Per launch at 128^3: 26.3 -> 0.23 ms.
+template <bool POINTS>
 __global__ void __launch_bounds__(256) k_volume(GVw g) {
     int idx = blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= g.nc) return;
     int i = idx % g.Ni, r = idx / g.Ni, j = r % g.Nj, k = r / g.Nj;
     double C[8][3], W[5];
     cell_coords(g, i, j, k, C);
-    BWp dummy = {};
-    gauss_volume<0>(C, dummy, W);
+    if (POINTS || !simpson_volume(C, W))
+        gauss_volume_fn(C, [](double x, double y, double z, double *Wp) { Wp[0] = 1; Wp[1] = x; Wp[2] = y; Wp[3] = z; Wp[4] = 0; }, W);
     const size_t nc = g.nc, nf = g.nf;
     g.vol[idx] = W[0];
     g.xyzcc[idx] = W[1] / W[0];
@@ -299,24 +381,102 @@ __global__ void k_ic_ot(GV g, double gamma, double rho0, double p0, double b0, d
     mag[2 * nf + f] = 0.0;
 }
 
-// gridutils.F90:144-189 GasIC2State with the blast-wave integrand (active cells)
+// Whether every point of the cell is inside the sphere (1) or outside (-1): a
+// trilinear cell lies in the hull of its corners.  0: neither is certain (the
+// margin covers the rounding of the distances).
+__device__ __forceinline__ int cell_in_sphere(const double C[8][3], const BWp &bw) {
+    double ctr[3], far = 0.0, half = 0.0;
+    for (int x = 0; x < 3; x++) {
+        ctr[x] = 0.0;
+        for (int n = 0; n < 8; n++) ctr[x] += 0.125 * C[n][x];
+    }
+    for (int n = 0; n < 8; n++) {
+        far = fmax(far, sqrt(sq(C[n][0] - bw.x0) + sq(C[n][1] - bw.y0) + sq(C[n][2] - bw.z0)));
+        half = fmax(half, sqrt(sq(C[n][0] - ctr[0]) + sq(C[n][1] - ctr[1]) + sq(C[n][2] - ctr[2])));
+    }
+    const double mid = sqrt(sq(ctr[0] - bw.x0) + sq(ctr[1] - bw.y0) + sq(ctr[2] - bw.z0));
+    const double tol = 1.0e-12 * (fabs(bw.rC) + mid + half + fabs(bw.x0) + fabs(bw.y0) + fabs(bw.z0));
+    if (far < bw.rC - tol) return 1;
+    if (mid - half > bw.rC + tol) return -1;
+    return 0;
+}
+
+// 1728-point quadrature (quadrature.F90:42-100) of the blast wave's density and
+// pressure (prob.F90:280-297) over a cell: the points q0, q0 + dq, ... of the
+// 12^3, their sums into D, P
+__device__ void bw_points(const double C[8][3], const BWp &bw, int q0, int dq, double &D, double &P) {
+    D = P = 0.0;
+    for (int q = q0; q < 1728; q += dq) {
+        const double x = gA[q / 144], y = gA[(q / 12) % 12], z = gA[q % 12];
+        const double w = gW[q / 144] * gW[(q / 12) % 12] * gW[q % 12];
+        const double xs[2] = {0.5 * (1 - x), 0.5 * (1 + x)}, ys[2] = {0.5 * (1 - y), 0.5 * (1 + y)}, zs[2] = {0.5 * (1 - z), 0.5 * (1 + z)};
+        const int ord[8] = {0, 1, 3, 2, 4, 5, 7, 6};   // corner i + 2 j + 4 k in cell_coords' order
+        double p[3] = {0, 0, 0}, J[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
+#pragma unroll
+        for (int n = 0; n < 8; n++) {
+            const int i = n & 1, j = (n >> 1) & 1, k = n >> 2;
+#pragma unroll
+            for (int d = 0; d < 3; d++) {
+                const double c = C[ord[n]][d];
+                p[d] += c * (xs[i] * ys[j] * zs[k]);
+                J[d][0] += c * ((i ? 0.5 : -0.5) * ys[j] * zs[k]);
+                J[d][1] += c * (xs[i] * (j ? 0.5 : -0.5) * zs[k]);
+                J[d][2] += c * (xs[i] * ys[j] * (k ? 0.5 : -0.5));
+            }
+        }
+        const double dJ = w * fabs(J[0][0] * (J[1][1] * J[2][2] - J[1][2] * J[2][1])
+                                 - J[0][1] * (J[1][0] * J[2][2] - J[1][2] * J[2][0])
+                                 + J[0][2] * (J[1][0] * J[2][1] - J[1][1] * J[2][0]));
+        const bool in = sqrt(sq(p[0] - bw.x0) + sq(p[1] - bw.y0) + sq(p[2] - bw.z0)) <= bw.rC;
+        D += dJ * (in ? bw.dRat * bw.D0 : bw.D0);
+        P += dJ * (in ? bw.pRat * bw.P0 : bw.P0);
+    }
+}
+
+// gridutils.F90:144-189 GasIC2State with the blast-wave integrand on the active
+// cells (at rest).  A cell wholly inside or outside the sphere has a constant
+// integrand, whose integral is that constant times the volume; only the cells the
+// sphere's surface crosses need the quadrature.  They are few and lie a handful to
+// a wave, so the wave takes them one after the other, its 64 lanes sharing the points
+// (one lane walking the 1728 alone leaves the others idle: 6.1 ms per launch at
+// 128^3).  23.8 ms with the quadrature on every cell -> 0.57 ms.
 __global__ void __launch_bounds__(256) k_ic_bw_gas(GVw g, double gamma, BWp bw, double *Gas) {
     const int nx = g.Nip, ny = g.Njp, nz = g.Nkp;
-    int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= nx * ny * nz) return;
-    int i = g.nG + idx % nx, r = idx / nx, j = g.nG + r % ny, k = g.nG + r / ny;
-    double C[8][3], W[5];
+    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
+    const bool live = idx < nx * ny * nz;   // lanes past the end only share the points
+    const int id = live ? idx : 0;
+    const int i = g.nG + id % nx, r = id / nx, j = g.nG + r % ny, k = g.nG + r / ny;
+    double C[8][3], V[4], WD = 0.0, WP = 0.0;
     cell_coords(g, i, j, k, C);
-    int c = ciw(g, i, j, k);
-    double dV = g.vol[c];
-    gauss_volume<1>(C, bw, W);
-    for (int v = 0; v < 5; v++) W[v] = W[v] / dV;
-    double D = W[0], Mx = D * W[1], My = D * W[2], Mz = D * W[3], P = W[4];
-    double KinE = 0.5 * (sq(Mx) + sq(My) + sq(Mz)) / D;
-    double IntE = P / (gamma - 1.0);
+    const int side = cell_in_sphere(C, bw);
+    const bool whole = side != 0 && simpson_volume(C, V);
+    if (whole) {
+        WD = V[0] * (side > 0 ? bw.dRat * bw.D0 : bw.D0);
+        WP = V[0] * (side > 0 ? bw.pRat * bw.P0 : bw.P0);
+    }
+#ifdef GAM_EMU   // threads run one by one
+    else bw_points(C, bw, 0, 1, WD, WP);
+#else
+    const int lane = threadIdx.x & 63;
+    for (unsigned long long todo = __ballot(live && !whole); todo; todo &= todo - 1) {
+        const int src = __ffsll(todo) - 1;
+        double Cs[8][3], D, P;
+#pragma unroll
+        for (int n = 0; n < 8; n++)
+#pragma unroll
+            for (int d = 0; d < 3; d++) Cs[n][d] = __shfl(C[n][d], src, 64);
+        bw_points(Cs, bw, lane, 64, D, P);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) { D += __shfl_xor(D, o, 64); P += __shfl_xor(P, o, 64); }
+        if (lane == src) { WD = D; WP = P; }
+    }
+#endif
+    if (!live) return;
+    const int c = ciw(g, i, j, k);
+    const double dV = g.vol[c], D = WD / dV, P = WP / dV;
     const size_t nc = g.nc;
-    Gas[c] = D; Gas[nc + c] = Mx; Gas[2 * nc + c] = My; Gas[3 * nc + c] = Mz;
-    Gas[4 * nc + c] = IntE + KinE;
+    Gas[c] = D; Gas[nc + c] = 0.0; Gas[2 * nc + c] = 0.0; Gas[3 * nc + c] = 0.0;
+    Gas[4 * nc + c] = P / (gamma - 1.0);
 }
 
 // gridutils.F90:205-223 edge integrals of A (quadrature.F90:345-370), over isg..ieg-1
