@@ -66,6 +66,7 @@ struct gam_handle {
     double *ringTab = nullptr;         // cos, sin of the ring angles phi_n
     double *ringMean = nullptr;        // ring-average scratch (chunk means, Fourier coefficients)
     size_t ringMean_n = 0;             // its capacity in doubles
+    bool vf_partial = false;           // the last step filled only the face velocities its EMFs read
     int fused_np = 0;                  // block minima the fused step's CalcDT reduces
     WindP wind = {};                   // the solar wind of a GAM_BC_WIND outer i face (gam_set_wind*)
     double *windSer = nullptr;         // its time series (nt x WIND_COLS), wind.ser points here
@@ -359,6 +360,9 @@ static int scratch_lookup(gam_handle *h) {
     return 0;
 }
 
+template <typename R, typename TM> static void launch_b2f(gam_handle *h, int st, const TM *mag, void *B);
+static int complete_vf(gam_handle *h);
+
 // ----------------------------------------------------------------- lifetime
 extern "C" int gam_create(const gam_dims *dims, const gam_params *par, gam_handle **out) {
     if (!dims || !par || !out) return -1;
@@ -536,6 +540,7 @@ extern "C" int gam_set_grid(gam_handle *h, const double *xyz, const double *xyzc
                             const double *dk) {
     if (!h) return -1;
     const size_t G = gsz(h), F = fsz(h);
+    if (int rv = complete_vf(h)) return rv;
     const double *src[G_N] = {xyz, xyzcc, xfc, face, Tf, edge, Te, Teb, volume, di, dj, dk};
     const size_t n[G_N] = {3 * F, 3 * G, 9 * F, 3 * F, 27 * F, 3 * F, 27 * F, 12 * F, G, G, G, G};
     for (int q = 0; q < G_N; q++) { int rc = h2d(h, h->grid[q], src[q], n[q]); if (rc) return rc; }
@@ -559,8 +564,9 @@ extern "C" int gam_set_corners(gam_handle *h, const double *xyz) {
     if (!h || !xyz) return -1;
     const GV &g = h->gv;
     if (g.Nip < 8) return fail(h, -1, "gam_set_corners: Nip must be >= 8 for the 8-point stencils");
-    int rc = h2d(h, h->grid[G_XYZ], xyz, 3 * fsz(h));
+    int rc = complete_vf(h);
     if (rc) return rc;
+    if ((rc = h2d(h, h->grid[G_XYZ], xyz, 3 * fsz(h)))) return rc;
     GVw w = gvw(h);
     for (int d = 0; d < 3; d++) {
         long n = (long)(g.Ni + (d == 0)) * (g.Nj + (d == 1)) * (g.Nk + (d == 2));
@@ -598,7 +604,6 @@ static void state_ptrs(gam_handle *h, int which, void **Gas, void **mag, void **
     *Gas = h->Gas[q]; *mag = h->mag[q]; *B = h->B[q];
 }
 
-template <typename R, typename TM> static void launch_b2f(gam_handle *h, int st, const TM *mag, void *B);
 
 extern "C" int gam_put_state(gam_handle *h, int which, double time, const double *Gas, const double *magFlux,
                              const double *Bxyz) {
@@ -959,8 +964,10 @@ static int celldt(gam_handle *h, const void *Gas, const void *B) {
     return h->prec ? launch_celldt<float>(h, Gas, B) : launch_celldt<double>(h, Gas, B);
 }
 
-// k_update's launch box: (i, j, column of UpdateKC cells in k)
-static int update_kc(const gam_handle *h) { return h->prec ? 1 : UPDATE_KC; }
+// k_update's launch box: (i, j, column of update_kc cells in k); FP64: 2 waves per SIMD
+static int update_kc(const gam_handle *h) {
+    return h->prec ? 1 : col_len(h->gv.Nk, (long)h->gv.Ni * h->gv.Nj, UPDATE_KC, 2 * 65536);
+}
 static int update_blocks(const gam_handle *h) {
     return tile_blocks(h->tile[ST_UPDATE], h->gv.Ni, h->gv.Nj, cdiv(h->gv.Nk, update_kc(h)));
 }
@@ -1045,9 +1052,11 @@ static void launch_emf(gam_handle *h) {
     const int st = ST_EMF_I + ED;
     const WKT<R> w = wkt<R>(h);
     StageTimer t(h, st);
-    if (ED == 1)   // J edges: k columns with the k stencil in registers
-        PLAUNCH(h, (k_emf_jcol<RM, BO, R>), (b_emf_jcol<RM, BO, R>), tgrid(h, st, g.Nip + 1, g.Njp, cdiv(g.Nkp + 1, EMF_KC)),
-                256, g, h->tile[st], h->mp, h->bgv, h->clk, P<R>(h->Vf), P<R>(h->hGas), w.bn, w.bh, P<R>(h->E), h->corr, h->corr_scale);
+    if (ED == 1) {   // J edges: k columns with the k stencil in registers (FP64: 2 waves per SIMD, FP32: 4)
+        const int kc = col_len(g.Nkp + 1, (long)(g.Nip + 1) * g.Njp, EMF_KC, (sizeof(R) == sizeof(float) ? 4 : 2) * 65536L);
+        PLAUNCH(h, (k_emf_jcol<RM, BO, R>), (b_emf_jcol<RM, BO, R>), tgrid(h, st, g.Nip + 1, g.Njp, cdiv(g.Nkp + 1, kc)),
+                256, g, h->tile[st], h->mp, h->bgv, h->clk, P<R>(h->Vf), P<R>(h->hGas), w.bn, w.bh, P<R>(h->E), h->corr, h->corr_scale, kc);
+    }
     else
         PLAUNCH(h, (k_emf<ED, RM, BO, R>), (b_emf<ED, RM, BO, R>), tgrid(h, st, g.Nip + (ED != 0), g.Njp + (ED != 1), g.Nkp + (ED != 2)),
                 256, g, h->tile[st], h->mp, h->bgv, h->clk, P<R>(h->Vf), P<R>(h->hGas), w.bn, w.bh, P<R>(h->E), h->corr, h->corr_scale);
@@ -1076,6 +1085,25 @@ static void launch_b2f(gam_handle *h, int st, const TM *mag, void *B) {
     if (h->ring.on)   // RingFlux2FieldFix (gridutils.F90:298-300)
         hipLaunchKernelGGL(HIP_KERNEL_NAME(k_ring_bfix<R>), grid1((long)g.Ni * g.Nk * g.nG * 2), 256, 0, h->stream, g,
                            h->clk, P<R>(B));
+}
+
+// Mom2Face of the predictor state (FP64: 3 waves per SIMD, FP32: 5)
+template <typename R>
+static void launch_vf(gam_handle *h, int full) {
+    const GVT<R> &g = view<R>(h);
+    const int kc = col_len(g.Nk, (long)g.Ni * g.Nj, VF_KC, 4 * 65536);
+    PLAUNCH(h, (k_vf<R>), (b_vf<R>), tgrid(h, ST_MOM2FACE, g.Ni, g.Nj, cdiv(g.Nk, kc)), 256, g, h->tile[ST_MOM2FACE], h->clk,
+            P<R>(h->wk[W_VDV]), P<R>(h->Vf), kc, full);
+}
+
+// The rest of the last step's face velocities (gam_get_work), from its predictor
+// state and the geometry it ran on: also before that geometry changes
+static int complete_vf(gam_handle *h) {
+    if (!h->vf_partial) return 0;
+    if (h->prec) launch_vf<float>(h, 1); else launch_vf<double>(h, 1);
+    HIPCHK(h, hipGetLastError());
+    h->vf_partial = false;
+    return 0;
 }
 
 // RingAverage (ringav.F90:25-73) on State, after the update: smoothing EMF,
@@ -1122,8 +1150,8 @@ static int advance_t(gam_handle *h, int fuse_dt) {
     { StageTimer t(h, ST_BHALF); launch_b2f<R, R>(h, ST_BHALF, P<R>(h->hmag), h->hB); }
     if (m.doMHD) {
         { StageTimer t(h, ST_MOM2FACE);
-          PLAUNCH(h, (k_vf<R>), (b_vf<R>), tgrid(h, ST_MOM2FACE, g.Ni, g.Nj, cdiv(g.Nk, VF_KC)), 256, g,
-                  h->tile[ST_MOM2FACE], h->clk, P<R>(h->wk[W_VDV]), P<R>(h->Vf)); }
+          launch_vf<R>(h, 0);
+          h->vf_partial = true; }
         if (h->corr && h->corr_wait) HIPCHK(h, hipStreamWaitEvent(h->stream, h->corr_wait, 0));
         if (m.rmeth == 1) { if (m.doBoris) launch_emfs<1, 1, R>(h); else launch_emfs<1, 0, R>(h); }
         else { if (m.doBoris) launch_emfs<0, 1, R>(h); else launch_emfs<0, 0, R>(h); }
@@ -1154,14 +1182,14 @@ static int advance_t(gam_handle *h, int fuse_dt) {
         const Tile tu = h->tile[ST_UPDATE];
         const R *nGas = P<R>(h->Gas[S]), *nB = P<R>(h->B[S]), *Flx = P<R>(h->Flx);
         R *oGas = P<R>(h->Gas[O]), *oB = P<R>(h->B[O]);
-        const int skip = h->ring.on ? h->ring.nring + 3 : 0;
+        const int skip = h->ring.on ? h->ring.nring + 3 : 0, kcu = update_kc(h);
         // FP64: the k-column kernel; FP32 bulk: one cell per thread
         if constexpr (sizeof(R) == sizeof(double)) {
             if (m.doMHD) {
-                if (m.doBoris) PLAUNCH(h, (k_update_col<1, 1, R>), (b_update_col<1, 1, R>), gr, 256, g, tu, m, h->bgv, h->clk, nGas, nB, Flx, h->mag[O], oGas, oB, h->partial, skip);
-                else PLAUNCH(h, (k_update_col<0, 1, R>), (b_update_col<0, 1, R>), gr, 256, g, tu, m, h->bgv, h->clk, nGas, nB, Flx, h->mag[O], oGas, oB, h->partial, skip);
+                if (m.doBoris) PLAUNCH(h, (k_update_col<1, 1, R>), (b_update_col<1, 1, R>), gr, 256, g, tu, m, h->bgv, h->clk, nGas, nB, Flx, h->mag[O], oGas, oB, h->partial, skip, kcu);
+                else PLAUNCH(h, (k_update_col<0, 1, R>), (b_update_col<0, 1, R>), gr, 256, g, tu, m, h->bgv, h->clk, nGas, nB, Flx, h->mag[O], oGas, oB, h->partial, skip, kcu);
             } else {
-                PLAUNCH(h, (k_update_col<0, 0, R>), (b_update_col<0, 0, R>), gr, 256, g, tu, m, h->bgv, h->clk, nGas, nB, Flx, h->mag[O], oGas, oB, h->partial, skip);
+                PLAUNCH(h, (k_update_col<0, 0, R>), (b_update_col<0, 0, R>), gr, 256, g, tu, m, h->bgv, h->clk, nGas, nB, Flx, h->mag[O], oGas, oB, h->partial, skip, kcu);
             }
         } else {
           if (m.doMHD) {
@@ -1583,7 +1611,10 @@ extern "C" int gam_get_work(gam_handle *h, int which, double *out) {
     int rc;
     if (which == 0) rc = d2h_bulk(h, out, h->Flx, 24 * G);
     else if (which == 1) rc = d2h_bulk(h, out, h->E, 3 * G);
-    else if (which == 2) rc = d2h_bulk(h, out, h->Vf, 9 * G);
+    else if (which == 2) {
+        if ((rc = complete_vf(h))) return rc;
+        rc = d2h_bulk(h, out, h->Vf, 9 * G);
+    }
     else return fail(h, -1, "gam_get_work: which must be 0, 1 or 2");
     if (rc) return rc;
     return gam_sync(h);

@@ -162,7 +162,18 @@ __device__ __forceinline__ void cell_bxyz_kc(const GVT<R> &g, const TM *mag, int
     kc.fK = fKp;
 }
 
-// cells per k_update_col thread along k (a column walked bottom up)
+// Cells (edges) a column kernel's thread walks, of L along its column over
+// `cols` lanes (speed only): `most` where the launch still has `lanes` lanes,
+// fewer on a small block, down to one, so that its waves fill the chip instead
+// of walking a serial chain of dependent loads.  lanes: what keeps the kernel's
+// resident waves busy (its waves per SIMD x 65536).  A 32x32x4 step's k_vf, J-edge
+// EMF and update take 6, 7 and 8 us, 21, 17 and 19 with fixed columns of 8, 8 and 4.
+static inline int col_len(int L, long cols, int most, long lanes) {
+    const long n = (long)L * cols / lanes;
+    return n < 1 ? 1 : (n > most ? most : (int)n);
+}
+
+// k_update_col walks up to 4 cells up a k column
 #define UPDATE_KC 4
 
 // ----------------------------------------------------------------- clock
@@ -340,37 +351,41 @@ __device__ __forceinline__ void mom2face(const GVT<R> &g, const R *__restrict__ 
 }
 
 // Vf arrays: VfA[dT1][xyz] stored as slab (3*dT1 + xyz).  Each thread walks
-// VF_KC cells up a k column; the k-direction stencil (8 points along k) is a
-// window kept in registers, shifted by one point per cell.
+// kc <= VF_KC cells up a k column; the k-direction stencil (8 points along k) is a
+// window kept in registers, shifted by one point per cell.  full: every cell the
+// reference fills; else only those the edge EMFs read (K edges take the I faces'
+// velocities on the active k, I edges the J faces' on the active i, J edges the K
+// faces' on the active j): on a box 4 cells deep that is a third of the I faces.
 #define VF_KC 8
 template <typename R>
 __device__ __forceinline__ void b_vf(const unsigned vb, GVT<R> g, Tile t, const DClock *__restrict__ clk, const R *__restrict__ VdV,
-                                            R *__restrict__ Vf) {
+                                            R *__restrict__ Vf, int kc, int full) {
     int i, j, kb;
-    if (!tile_pos(vb, t, g.Ni, g.Nj, cdiv(g.Nk, VF_KC), i, j, kb) || clk->halt) return;
+    if (!tile_pos(vb, t, g.Ni, g.Nj, cdiv(g.Nk, kc), i, j, kb) || (clk->halt && !full)) return;
     const int a0 = g.nG;
     const size_t nc = g.nc;
     const int sk = cstride(g, 2);
+    const bool iact = full || (i >= a0 && i < a0 + g.Nip), jact = full || (j >= a0 && j < a0 + g.Njp);
     R wVol[8], wX[8], wY[8], wZ[8];   // k window of the K-face Mom2Face: points k-4 .. k+3
     bool haveW = false;
 #pragma unroll 1
-    for (int kk = 0; kk < VF_KC; kk++) {
-        const int k = kb * VF_KC + kk;
+    for (int kk = 0; kk < kc; kk++) {
+        const int k = kb * kc + kk;
         if (k >= g.Nk) break;
         const int idx = ci(g, i, j, k);
         R v[3];
         // dT1 = I (used by K edges): i in is..ie+1   (fields.F90:161-175)
-        if (i >= a0 && i <= a0 + g.Nip) {
+        if (i >= a0 && i <= a0 + g.Nip && (full || (k >= a0 && k < a0 + g.Nkp))) {
             mom2face(g, VdV, idx, 0, v);
             st_nt(&Vf[nc * 0 + idx], v[0]); st_nt(&Vf[nc * 1 + idx], v[1]); st_nt(&Vf[nc * 2 + idx], v[2]);
         }
         // dT1 = J (used by I edges): j in js..je+1   (fields.F90:119-133)
-        if (j >= a0 && j <= a0 + g.Njp) {
+        if (j >= a0 && j <= a0 + g.Njp && iact) {
             mom2face(g, VdV, idx, 1, v);
             st_nt(&Vf[nc * 3 + idx], v[0]); st_nt(&Vf[nc * 4 + idx], v[1]); st_nt(&Vf[nc * 5 + idx], v[2]);
         }
         // dT1 = K (used by J edges): k in ks..ke+1   (fields.F90:140-154)
-        if (k >= a0 && k <= a0 + g.Nkp) {
+        if (k >= a0 && k <= a0 + g.Nkp && jact) {
             if (!haveW) {
 #pragma unroll
                 for (int n = 0; n < 8; n++) {
@@ -391,8 +406,8 @@ __device__ __forceinline__ void b_vf(const unsigned vb, GVT<R> g, Tile t, const 
 }
 template <typename R>
 __global__ void __launch_bounds__(256) k_vf(GVT<R> g, Tile t, const DClock *__restrict__ clk, const R *__restrict__ VdV,
-                                            R *__restrict__ Vf) {
-    b_vf<R>(blockIdx.x, g, t, clk, VdV, Vf);
+                                            R *__restrict__ Vf, int kc, int full) {
+    b_vf<R>(blockIdx.x, g, t, clk, VdV, Vf, kc, full);
 }
 
 // fields.F90:288-362 EdgeLRs: dT1 faces reconstructed along dT2 at face point f;
@@ -532,7 +547,7 @@ __global__ void __launch_bounds__(256) k_emf(GVT<R> g, Tile t, MP m, BGV bg, con
     b_emf<ED, RM, BORIS, R>(blockIdx.x, g, t, m, bg, clk, Vf, hGas, bn, bh, E, corr, cs);
 }
 
-// J edges walking EMF_KC edges up a k column: the I faces' stencils along k
+// J edges walking kc <= EMF_KC edges up a k column: the I faces' stencils along k
 // (the one k-direction stencil of a J edge) are a register window shifted by
 // one point per edge.  Box [is,ie+1]x[js,je]x[ks,ke+1].
 #define EMF_KC 8
@@ -540,17 +555,17 @@ template <int RM, int BORIS, typename R>
 __device__ __forceinline__ void b_emf_jcol(const unsigned vb, GVT<R> g, Tile t, MP m, BGV bg, const DClock *__restrict__ clk,
                                                   const R *__restrict__ Vf, const R *__restrict__ hGas,
                                                   const R *__restrict__ bn, const R *__restrict__ bh, R *__restrict__ E,
-                                                  const float *__restrict__ corr, double cs) {
+                                                  const float *__restrict__ corr, double cs, int kc) {
     const int nz = g.Nkp + 1;
     int a, b, cb;
-    if (!tile_pos(vb, t, g.Nip + 1, g.Njp, cdiv(nz, EMF_KC), a, b, cb) || clk->halt) return;
+    if (!tile_pos(vb, t, g.Nip + 1, g.Njp, cdiv(nz, kc), a, b, cb) || clk->halt) return;
     const int i = a + g.nG, j = b + g.nG;
     const int st = fstride(g, 2);
     const R *fI = g.face, *bhI = bh, *bnI = bn;   // I-face slabs (direction 0)
     R wA[8], wB[8], wN[4];
 #pragma unroll 1
-    for (int kk = 0; kk < EMF_KC; kk++) {
-        const int cz = cb * EMF_KC + kk;
+    for (int kk = 0; kk < kc; kk++) {
+        const int cz = cb * kc + kk;
         if (cz >= nz) break;
         const int k = cz + g.nG;
         const int f = fi(g, i, j, k);
@@ -575,8 +590,8 @@ template <int RM, int BORIS, typename R>
 __global__ void __launch_bounds__(256) k_emf_jcol(GVT<R> g, Tile t, MP m, BGV bg, const DClock *__restrict__ clk,
                                                   const R *__restrict__ Vf, const R *__restrict__ hGas,
                                                   const R *__restrict__ bn, const R *__restrict__ bh, R *__restrict__ E,
-                                                  const float *__restrict__ corr, double cs) {
-    b_emf_jcol<RM, BORIS, R>(blockIdx.x, g, t, m, bg, clk, Vf, hGas, bn, bh, E, corr, cs);
+                                                  const float *__restrict__ corr, double cs, int kc) {
+    b_emf_jcol<RM, BORIS, R>(blockIdx.x, g, t, m, bg, clk, Vf, hGas, bn, bh, E, corr, cs, kc);
 }
 
 // ----------------------------------------------------------------- fluxes
@@ -1197,7 +1212,7 @@ __global__ void __launch_bounds__(256) k_update(GVT<R> g, Tile t, MP m, BGV bg, 
     b_update<BORIS, MHD, R>(blockIdx.x, g, t, m, bg, clk, nGas, nB, Flx, magNew, oGas, oB, partial, skip_nb);
 }
 
-// k_update walking UPDATE_KC cells up a k column per thread, reading each K
+// k_update walking kc <= UPDATE_KC cells up a k column per thread, reading each K
 // face's fluxes, magFlux and centre once (the FP64 step's update: less HBM
 // traffic there; in FP32 bulk it measured slower and k_update is used).
 template <int BORIS, int MHD, typename R>
@@ -1205,28 +1220,27 @@ __device__ __forceinline__ void b_update_col(const unsigned vb, GVT<R> g, Tile t
                                                 const R *__restrict__ nGas, const R *__restrict__ nB,
                                                 const R *__restrict__ Flx, const double *__restrict__ magNew,
                                                 R *__restrict__ oGas, R *__restrict__ oB,
-                                                double *__restrict__ partial, int skip_nb) {
+                                                double *__restrict__ partial, int skip_nb, int kc) {
     if (clk->halt) return;
     double dtl = GAM_HUGE;
-    constexpr int KC = UPDATE_KC;
     int i, j, kb;
-    if (tile_pos(vb, t, g.Ni, g.Nj, cdiv(g.Nk, KC), i, j, kb)) {
+    if (tile_pos(vb, t, g.Ni, g.Nj, cdiv(g.Nk, kc), i, j, kb)) {
         const size_t nc = g.nc;
         const int a0 = g.nG;
         const bool act_ij = i >= a0 && i < a0 + g.Nip && j >= a0 && j < a0 + g.Njp;
         auto F = [&](int slab, int c) { return (double)Flx[nc * slab + c]; };
-        KCarry kc;
+        KCarry kcar;
         double cF[8];          // K fluxes of the lower K face, carried from the cell below
         bool haveF = false;
 #pragma unroll 1
-        for (int kk = 0; kk < KC; kk++) {
-            const int k = kb * KC + kk;
+        for (int kk = 0; kk < kc; kk++) {
+            const int k = kb * kc + kk;
             if (k >= g.Nk) break;
             const int idx = ci(g, i, j, k);
             double U[5], Bn[3] = {0, 0, 0};
 #pragma unroll
             for (int v = 0; v < 5; v++) U[v] = (double)nGas[nc * v + idx];
-            cell_bxyz_kc(g, magNew, i, j, k, Bn, kc, kk > 0);
+            cell_bxyz_kc(g, magNew, i, j, k, Bn, kcar, kk > 0);
             const bool active = act_ij && k >= a0 && k < a0 + g.Nkp;
             if (active) {
                 const double dt = clk->dt;
@@ -1275,8 +1289,8 @@ __global__ void __launch_bounds__(256) k_update_col(GVT<R> g, Tile t, MP m, BGV 
                                                 const R *__restrict__ nGas, const R *__restrict__ nB,
                                                 const R *__restrict__ Flx, const double *__restrict__ magNew,
                                                 R *__restrict__ oGas, R *__restrict__ oB,
-                                                double *__restrict__ partial, int skip_nb) {
-    b_update_col<BORIS, MHD, R>(blockIdx.x, g, t, m, bg, clk, nGas, nB, Flx, magNew, oGas, oB, partial, skip_nb);
+                                                double *__restrict__ partial, int skip_nb, int kc) {
+    b_update_col<BORIS, MHD, R>(blockIdx.x, g, t, m, bg, clk, nGas, nB, Flx, magNew, oGas, oB, partial, skip_nb, kc);
 }
 
 // Stand-alone CellDT min over the DT box (CalcDT without the fused update)
