@@ -12,6 +12,7 @@
 #include <mutex>
 #include <string>
 #include <tuple>
+#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -66,6 +67,7 @@ struct gam_handle {
     double *ringTab = nullptr;         // cos, sin of the ring angles phi_n
     double *ringMean = nullptr;        // ring-average scratch (chunk means, Fourier coefficients)
     size_t ringMean_n = 0;             // its capacity in doubles
+    bool capturing = false;            // gam_graph_create is capturing its steps
     bool vf_partial = false;           // the last step filled only the face velocities its EMFs read
     int fused_np = 0;                  // block minima the fused step's CalcDT reduces
     WindP wind = {};                   // the solar wind of a GAM_BC_WIND outer i face (gam_set_wind*)
@@ -1062,15 +1064,74 @@ static void launch_emf(gam_handle *h) {
                 256, g, h->tile[st], h->mp, h->bgv, h->clk, P<R>(h->Vf), P<R>(h->hGas), w.bn, w.bh, P<R>(h->E), h->corr, h->corr_scale);
 }
 
-template <int RM, int BO, typename R>
-static void launch_emfs(gam_handle *h) {
-    launch_emf<0, RM, BO, R>(h);
-    launch_emf<1, RM, BO, R>(h);
-    launch_emf<2, RM, BO, R>(h);
+// RingFlux2FieldFix (gridutils.F90:298-300) after a bFlux2Fld into B
+template <typename R>
+static void launch_ring_bfix(gam_handle *h, void *B) {
+    const GVT<R> &g = view<R>(h);
+    if (h->ring.on)
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_ring_bfix<R>), grid1((long)g.Ni * g.Nk * g.nG * 2), 256, 0, h->stream, g, h->clk,
+                           P<R>(B));
 }
 
+// Blocks of the three EMF and three flux directions, one edge or interface per thread
+static MergeRanges emf_flux_ranges(const gam_handle *h) {
+    const GV &g = h->gv;
+    const int nz = h->mp.do25D ? 1 : g.Nkp;
+    MergeRanges mr = {};
+    unsigned n[6];
+    for (int d = 0; d < 3; d++) {
+        n[d] = h->mp.doMHD ? (unsigned)tile_blocks(MERGE_TILE, g.Nip + (d != 0), g.Njp + (d != 1), g.Nkp + (d != 2)) : 0u;
+        n[3 + d] = d == 2 && h->mp.do25D ? 0u : (unsigned)tile_blocks(MERGE_TILE, g.Nip + (d == 0), g.Njp + (d == 1), nz + (d == 2));
+    }
+    for (int q = 0; q < 6; q++) mr.first[q + 1] = mr.first[q] + n[q];
+    return mr;
+}
+
+// Whether a step takes the merged launches (speed only): up to this many blocks of
+// EMFs and fluxes, where running them side by side gains more than the j and k
+// fluxes' columns do.  Step time of an n^3 block, separate / merged: FP64 1.24 (n =
+// 48), 1.28 (64), 1.06 (96), 0.99 (112), 0.91 (160); FP32 bulk 1.29, 1.32, 1.09, 1.04,
+// 0.96; hydro FP64 1.10 (64), 1.00 (80), 0.95 (128).  96^3 has 21000 blocks, 112^3 33000.
+// Graphs (their blocks already run side by side), stage timers (one stage per
+// launch) and a correction keep the separate ones.
+static bool merged(const gam_handle *h) {
+    const unsigned most = !h->mp.doMHD ? 4096 : h->prec ? 40960 : 24576;
+    return !h->rec && !h->capturing && !h->timing && !h->corr && emf_flux_ranges(h).first[6] <= most;
+}
+
+template <typename R>
+static void launch_b2f_vf(gam_handle *h) {
+    const GVT<R> &g = view<R>(h);
+    const int kc = col_len(g.Nk, (long)g.Ni * g.Nj, VF_KC, 4 * 65536);
+    MergeRanges mr = {};
+    mr.first[1] = (unsigned)tile_blocks(MERGE_TILE, g.Ni, g.Nj, cdiv(g.Nk, kc));
+    mr.first[2] = mr.first[1] + (unsigned)tile_blocks(MERGE_TILE, g.Ni, g.Nj, g.Nk);
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_b2f_vf<R>), dim3(mr.first[2]), 256, 0, h->stream, g, h->clk, (const R *)P<R>(h->hmag),
+                       P<R>(h->hB), (const R *)P<R>(h->wk[W_VDV]), P<R>(h->Vf), kc, mr);
+    launch_ring_bfix<R>(h, h->hB);
+}
+
+// CalcElecField's edges and CalcStress's interfaces
 template <int RM, int BO, int MH, typename R>
-static void launch_fluxes(gam_handle *h) {
+static void launch_emf_flux(gam_handle *h, bool merge) {
+    if (merge) {
+        const GVT<R> &g = view<R>(h);
+        const MergeRanges mr = emf_flux_ranges(h);
+        const int S = h->s;
+        auto go = [&](auto bg) {
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_emf_flux<RM, BO, MH, decltype(bg)::value, R>), dim3(mr.first[6]), 256, 0, h->stream, g,
+                               h->mp, h->bgv, h->clk, wkt<R>(h), (const R *)P<R>(h->Vf), (const R *)P<R>(h->B[S]),
+                               (const R *)P<R>(h->hB), (const R *)P<R>(h->hmag), (const R *)P<R>(h->hGas), P<R>(h->E), P<R>(h->Flx), mr);
+        };
+        if (MH && h->bgv.on) go(std::integral_constant<int, MH>{});
+        else go(std::integral_constant<int, 0>{});
+        return;
+    }
+    if (MH) {
+        launch_emf<0, RM, BO, R>(h);
+        launch_emf<1, RM, BO, R>(h);
+        launch_emf<2, RM, BO, R>(h);
+    }
     launch_flux<RM, BO, MH, R>(h, 0);
     launch_flux<RM, BO, MH, R>(h, 1);
     if (!h->mp.do25D) launch_flux<RM, BO, MH, R>(h, 2);
@@ -1082,9 +1143,7 @@ static void launch_b2f(gam_handle *h, int st, const TM *mag, void *B) {
     const GVT<R> &g = view<R>(h);
     PLAUNCH(h, (k_b2f<R, TM>), (b_b2f<R, TM>), tgrid(h, st, g.Ni, g.Nj, g.Nk), 256, g, h->tile[st],
             h->clk, mag, P<R>(B));
-    if (h->ring.on)   // RingFlux2FieldFix (gridutils.F90:298-300)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_ring_bfix<R>), grid1((long)g.Ni * g.Nk * g.nG * 2), 256, 0, h->stream, g,
-                           h->clk, P<R>(B));
+    launch_ring_bfix<R>(h, B);
 }
 
 // Mom2Face of the predictor state (FP64: 3 waves per SIMD, FP32: 5)
@@ -1143,24 +1202,27 @@ static int advance_t(gam_handle *h, int fuse_dt) {
     const GVT<R> &g = view<R>(h);
     const MP &m = h->mp;
     const int S = h->s, O = 1 - h->s;
-    { StageTimer t(h, ST_CLOCK); PLAUNCH(h, (k_clock_begin), (b_clock_begin), dim3(1), 64, h->clk); }
     { StageTimer t(h, ST_PREDICT);
       PLAUNCH(h, (k_predict<R>), (b_predict<R>), grid1(g.nf), 256, g, m, h->clk, P<R>(h->Gas[S]), P<R>(h->Gas[O]),
               h->mag[S], h->mag[O], P<R>(h->hGas), P<R>(h->hmag), wkt<R>(h)); }
-    { StageTimer t(h, ST_BHALF); launch_b2f<R, R>(h, ST_BHALF, P<R>(h->hmag), h->hB); }
-    if (m.doMHD) {
-        { StageTimer t(h, ST_MOM2FACE);
-          launch_vf<R>(h, 0);
-          h->vf_partial = true; }
-        if (h->corr && h->corr_wait) HIPCHK(h, hipStreamWaitEvent(h->stream, h->corr_wait, 0));
-        if (m.rmeth == 1) { if (m.doBoris) launch_emfs<1, 1, R>(h); else launch_emfs<1, 0, R>(h); }
-        else { if (m.doBoris) launch_emfs<0, 1, R>(h); else launch_emfs<0, 0, R>(h); }
-    } else if (h->corr && h->corr_wait) HIPCHK(h, hipStreamWaitEvent(h->stream, h->corr_wait, 0));
-    if (m.doMHD) {
-        if (m.rmeth == 1) { if (m.doBoris) launch_fluxes<1, 1, 1, R>(h); else launch_fluxes<1, 0, 1, R>(h); }
-        else { if (m.doBoris) launch_fluxes<0, 1, 1, R>(h); else launch_fluxes<0, 0, 1, R>(h); }
+    const bool merge = merged(h);
+    if (merge && m.doMHD) {
+        launch_b2f_vf<R>(h);
+        h->vf_partial = true;
     } else {
-        if (m.rmeth == 1) launch_fluxes<1, 0, 0, R>(h); else launch_fluxes<0, 0, 0, R>(h);
+        { StageTimer t(h, ST_BHALF); launch_b2f<R, R>(h, ST_BHALF, P<R>(h->hmag), h->hB); }
+        if (m.doMHD) {
+            StageTimer t(h, ST_MOM2FACE);
+            launch_vf<R>(h, 0);
+            h->vf_partial = true;
+        }
+    }
+    if (h->corr && h->corr_wait) HIPCHK(h, hipStreamWaitEvent(h->stream, h->corr_wait, 0));
+    if (m.doMHD) {
+        if (m.rmeth == 1) { if (m.doBoris) launch_emf_flux<1, 1, 1, R>(h, merge); else launch_emf_flux<1, 0, 1, R>(h, merge); }
+        else { if (m.doBoris) launch_emf_flux<0, 1, 1, R>(h, merge); else launch_emf_flux<0, 0, 1, R>(h, merge); }
+    } else {
+        if (m.rmeth == 1) launch_emf_flux<1, 0, 0, R>(h, merge); else launch_emf_flux<0, 0, 0, R>(h, merge);
     }
     if (h->ring.on)   // RingFlux (stress.F90:137-139)
         hipLaunchKernelGGL(HIP_KERNEL_NAME(k_ring_flux<R>), grid1((long)g.Ni * g.Nk * 2 + (long)g.Nip * g.Njp), 256, 0,
@@ -1474,17 +1536,22 @@ extern "C" int gam_get_ring(gam_handle *h, int *nring, int *nch) {
 template <typename R>
 static int bcs_t(gam_handle *h, bool shell) {
     const int S = h->s;
+    const GVT<R> &g = view<R>(h);
+    if (shell && !h->mp.do25D && all_periodic(h)) {
+        StageTimer t(h, ST_BC);
+        PLAUNCH(h, (k_bc_b2f<R>), (b_bc_b2f<R>), grid1(bc_shell_count(bc_shell(g.Ni, g.Nj, g.Nk, g.Nip, g.Njp, g.Nkp, g.nG, 7, 0))),
+                256, g, h->clk, P<R>(h->Gas[S]), h->mag[S], P<R>(h->B[S]));
+        HIPCHK(h, hipGetLastError());
+        return 0;
+    }
     { StageTimer t(h, ST_BC); launch_bc<R>(h, false); }
     {
         StageTimer t(h, ST_BPOST);
-        const GVT<R> &g = view<R>(h);
         if (shell && !h->mp.do25D) {
             const long n = b2f_shell_count(g.Ni, g.Nj, g.Nk, g.Nip, g.Njp, g.Nkp);
             PLAUNCH(h, (k_b2f_shell<R>), (b_b2f_shell<R>), dim3((unsigned)((n + 255) / 256)), 256, g, h->clk,
                     (const double *)h->mag[S], P<R>(h->B[S]));
-            if (h->ring.on)
-                hipLaunchKernelGGL(HIP_KERNEL_NAME(k_ring_bfix<R>), grid1((long)g.Ni * g.Nk * g.nG * 2), 256, 0, h->stream, g,
-                                   h->clk, P<R>(h->B[S]));
+            launch_ring_bfix<R>(h, h->B[S]);
         } else {
             launch_b2f<R, double>(h, ST_BPOST, h->mag[S], h->B[S]);
         }
@@ -1691,12 +1758,14 @@ extern "C" int gam_graph_create(gam_handle *const *hs, int n, int nsteps, gam_gr
     for (int q = 0; q < n && !rc; q++) {
         gam_handle *h = hs[q];
         if ((e = hipStreamWaitEvent(h->stream, g->evs[0], 0)) != hipSuccess) { rc = -2; break; }
+        h->capturing = true;
         for (int k = 0; k < nsteps && !rc; k++) {
             rc = advance(h, 1);
             if (!rc) launch_dtfinal(h, 1, 1, h->fused_np);
             if (!rc) launch_cpr(h);
             if (!rc) rc = bcs(h, true);
         }
+        h->capturing = false;
         if (!rc && (e = hipEventRecord(g->evs[1 + q], h->stream)) != hipSuccess) rc = -2;
         if (!rc && (e = hipStreamWaitEvent(g->stream, g->evs[1 + q], 0)) != hipSuccess) rc = -2;
     }
@@ -1868,6 +1937,8 @@ extern "C" int gam_graph_launch(gam_graph *g, int replays) {
         g->s0[q] = h->s;
     }
     hipError_t e;
+    for (gam_handle *h : g->hs)
+        if (replays > 0 && h->mp.doMHD) h->vf_partial = true;
     for (int r = 0; r < replays; r++)
         if ((e = hipGraphLaunch(g->exec, g->stream)) != hipSuccess) return gfail(g, -2, "hipGraphLaunch", e);
     return 0;

@@ -2,8 +2,8 @@
 //
 // One step (reference gamapp.F90:73-116 stepGamera) is, with S = State,
 // O = oState, H = predictor (half-step) state:
-//   k_clock_begin     time trap + pdt/odt            mhdgroup.F90:25-31,459
-//   k_predict   (F)   AB2 magFlux, PredictCell       mhdgroup.F90:445-616
+//   k_predict   (F)   time trap, pdt/odt, AB2 magFlux, PredictCell
+//                                                    mhdgroup.F90:25-31,445-616
 //   k_b2f       (G)   H.Bxyz = bFlux2Fld(H.magFlux)  gridutils.F90:281-301,648-680
 //   k_vf        (G)   Mom2Face for the 3 sweeps      fields.F90:110-179,235-285
 //   k_emf<d>    (E)   edge EMFs, one direction each  fields.F90:186-226,288-517
@@ -13,8 +13,8 @@
 //                                                    stress.F90:152-194, mhdgroup.F90:79-442,
 //                                                    gridutils.F90:49-106
 //   k_dtfinal   (1)   time update + CalcDT checks    gamapp.F90:112-114, step.F90:58-168
-//   k_bc        (F)   periodic ghost fill            bcs.F90:279-450
-//   k_b2f       (G)   O.Bxyz = bFlux2Fld(O.magFlux)  gamapp.F90:89
+//   k_bc_b2f    (F)   periodic ghost fill and the ghosts' Bxyz = bFlux2Fld
+//                                                    bcs.F90:279-450, gamapp.F90:89
 // after which the host swaps the S and O buffer sets (CopyState becomes a
 // pointer swap, mhdgroup.F90:202-257).
 //
@@ -72,16 +72,15 @@ template <typename T> __device__ __forceinline__ T ab2(T dt, T Q, T oQ, T odt) {
 // FP32 bulk: the same sum over the six faces with the cell's lever arms from
 // the table g.b2fc (18 floats per cell instead of 13 FP64 positions and the
 // volume; the stored Bxyz is FP32 either way).
-template <typename R, typename TM>
-__device__ __forceinline__ void cell_bxyz(const GVT<R> &g, const TM *mag, int i, int j, int k, double *B) {
+// cell_bxyz_fl: from the fluxes fl of the cell's lower/upper I, J, K faces.
+template <typename R>
+__device__ __forceinline__ void cell_bxyz_fl(const GVT<R> &g, const double (&fl)[6], int i, int j, int k, double *B) {
     const int nf = g.nf;
     int c = ci(g, i, j, k), f0 = fi(g, i, j, k);
     int fi1 = f0 + 1, fj1 = f0 + (g.Ni + 1), fk1 = f0 + (g.Ni + 1) * (g.Nj + 1);
     if constexpr (sizeof(R) == sizeof(float)) {
         if (g.b2fc) {
             const size_t nc = g.nc;
-            const double fl[6] = {(double)mag[f0], (double)mag[fi1], (double)mag[nf + f0], (double)mag[nf + fj1],
-                                  (double)mag[2 * (size_t)nf + f0], (double)mag[2 * (size_t)nf + fk1]};
 #pragma unroll
             for (int x = 0; x < 3; x++) {
                 double b = fl[0] * (double)g.b2fc[(size_t)x * nc + c];
@@ -93,8 +92,8 @@ __device__ __forceinline__ void cell_bxyz(const GVT<R> &g, const TM *mag, int i,
         }
     }
     double dV = g.dvol[c];
-    double fI = mag[f0], fJ = mag[nf + f0], fK = mag[2 * nf + f0];
-    double fIp = mag[fi1], fJp = mag[nf + fj1], fKp = mag[2 * (size_t)nf + fk1];
+    double fI = fl[0], fJ = fl[2], fK = fl[4];
+    double fIp = fl[1], fJp = fl[3], fKp = fl[5];
     double Div = fIp - fI + fJp - fJ + fKp - fK;
 #pragma unroll
     for (int x = 0; x < 3; x++) {
@@ -105,6 +104,14 @@ __device__ __forceinline__ void cell_bxyz(const GVT<R> &g, const TM *mag, int i,
         double b = (fIp * xfIp + fJp * xfJp + fKp * xfKp - fI * xfI - fJ * xfJ - fK * xfK) / dV;
         B[x] = b - Div * g.xyzcc[(size_t)g.nc * x + c] / dV;
     }
+}
+template <typename R, typename TM>
+__device__ __forceinline__ void cell_bxyz(const GVT<R> &g, const TM *mag, int i, int j, int k, double *B) {
+    const size_t nf = g.nf;
+    const int f0 = fi(g, i, j, k);
+    const double fl[6] = {(double)mag[f0], (double)mag[f0 + 1], (double)mag[nf + f0], (double)mag[nf + f0 + (g.Ni + 1)],
+                          (double)mag[2 * nf + f0], (double)mag[2 * nf + f0 + (g.Ni + 1) * (g.Nj + 1)]};
+    cell_bxyz_fl(g, fl, i, j, k, B);
 }
 
 // FP32 bulk: the lever arms of every cell for cell_bxyz, +-(face centre - cell
@@ -176,30 +183,24 @@ static inline int col_len(int L, long cols, int most, long lanes) {
 // k_update_col walks up to 4 cells up a k column
 #define UPDATE_KC 4
 
-// ----------------------------------------------------------------- clock
-__device__ __forceinline__ void b_clock_begin(const unsigned vb, DClock *clk) {
-    // mhdgroup.F90:25-28 trap and :31,459 pdt/odt
-    if (threadIdx.x == 0 && vb == 0 && !clk->halt) {
-        if (fabs(clk->otime - clk->stime) < GAM_TINY) clk->otime = clk->stime - clk->dt;
-        clk->odt = clk->stime - clk->otime;
-        clk->pdt = 0.5 * clk->dt;
-    }
-}
-__global__ void k_clock_begin(DClock *clk) {
-    b_clock_begin(blockIdx.x, clk);
-}
-
 // ----------------------------------------------------------------- predictor
 // magFlux AB2 (FP64 in, bulk out) on every face point; PredictCell on every
-// cell plus the per-point stencil inputs (WKT).
+// cell plus the per-point stencil inputs (WKT).  The step's first kernel also
+// sets the clock's trap and pdt/odt (mhdgroup.F90:25-31,459): every thread forms
+// them from the clock, one stores them (a thread that reads the stored otime
+// forms the same odt).
 template <typename R>
-__device__ __forceinline__ void b_predict(const unsigned vb, GVT<R> g, MP m, const DClock *__restrict__ clk,
+__device__ __forceinline__ void b_predict(const unsigned vb, GVT<R> g, MP m, DClock *clk,
                                                  const R *__restrict__ Gas, const R *__restrict__ oGas,
                                                  const double *__restrict__ mag, const double *__restrict__ omag,
                                                  R *__restrict__ hGas, R *__restrict__ hmag, WKT<R> w) {
     int idx = vb * blockDim.x + threadIdx.x;
     if (idx >= g.nf || clk->halt) return;
-    const double pdt = clk->pdt, odt = clk->odt;
+    double otime = clk->otime;
+    const double stime = clk->stime, dt = clk->dt;
+    if (fabs(otime - stime) < GAM_TINY) otime = stime - dt;
+    const double odt = stime - otime, pdt = 0.5 * dt;
+    if (idx == 0) { clk->otime = otime; clk->odt = odt; clk->pdt = pdt; }
     const int nf = g.nf, nc = g.nc;
     if (m.doMHD) {
 #pragma unroll
@@ -244,7 +245,7 @@ __device__ __forceinline__ void b_predict(const unsigned vb, GVT<R> g, MP m, con
     for (int x = 0; x < 3; x++) w.VdV[(size_t)nc * x + c] = vol * pQ[1 + x] / D;
 }
 template <typename R>
-__global__ void __launch_bounds__(256) k_predict(GVT<R> g, MP m, const DClock *__restrict__ clk,
+__global__ void __launch_bounds__(256) k_predict(GVT<R> g, MP m, DClock *clk,
                                                  const R *__restrict__ Gas, const R *__restrict__ oGas,
                                                  const double *__restrict__ mag, const double *__restrict__ omag,
                                                  R *__restrict__ hGas, R *__restrict__ hmag, WKT<R> w) {
@@ -758,9 +759,10 @@ __device__ __forceinline__ void face_flux(const GVT<R> &g, const MP &m, const BG
     lr_flux<DN, BORIS, MHD, BG>(g, m, bg, hmag, hGas, c, f, PL, PR, MagL, MagR, out);
 }
 
-// Fluxes of the i interfaces, box [is,ie+1]x[js,je]x[ks,ke] (k a single slice
-// in 2.5D), one interface per thread: the 8 points of a stencil lie in the
-// cache lines its neighbouring lanes load.
+// Fluxes of the interfaces in direction DN, one per thread.  The i interfaces of
+// every block (box [is,ie+1]x[js,je]x[ks,ke], k a single slice in 2.5D): the 8
+// points of a stencil lie in the cache lines its neighbouring lanes load.  The j
+// and k interfaces only in a small block's merged launch (k_emf_flux).
 // Output slabs Flx[(8*DN + v)*nc + c], v = 0..4 gas, 5..7 magnetic.  CORR = 1:
 // with the learned correction (corr, cs) added to the gas fluxes (corr_add); a
 // separate instantiation, so the plain kernels keep their registers.
@@ -770,9 +772,8 @@ __device__ __forceinline__ void b_flux(const unsigned vb, GVT<R> g, Tile t, MP m
                                               const R *__restrict__ Wh, const R *__restrict__ hB,
                                               const R *__restrict__ hmag, const R *__restrict__ hGas,
                                               R *__restrict__ Flx, const float *__restrict__ corr, double cs) {
-    static_assert(DN == 0, "the j and k interfaces go through b_flux_col");
     int a, b, cz;
-    if (!tile_pos(vb, t, g.Nip + 1, g.Njp, m.do25D ? 1 : g.Nkp, a, b, cz) || clk->halt) return;
+    if (!tile_pos(vb, t, g.Nip + (DN == 0), g.Njp + (DN == 1), (m.do25D ? 1 : g.Nkp) + (DN == 2), a, b, cz) || clk->halt) return;
     const int i = a + g.nG, j = b + g.nG, k = cz + g.nG;
     const size_t nc = g.nc;
     const int c = ci(g, i, j, k);
@@ -898,6 +899,42 @@ __global__ void __launch_bounds__(256) FLUX_COL_WAVES k_flux_col(GVT<R> g, Tile 
                                                   const R *__restrict__ hmag, const R *__restrict__ hGas,
                                                   R *__restrict__ Flx, const float *__restrict__ corr, double cs, int kc) {
     b_flux_col<DN, RM, BORIS, MHD, BG, R, CORR>(blockIdx.x, g, t, m, bg, clk, Wn, nB, Wh, hB, hmag, hGas, Flx, corr, cs, kc);
+}
+
+// A small block's half-step field and face velocities in one launch, and its
+// three EMF and three flux directions in another: within each none reads what
+// another writes.  Launched one by one each leaves most of the chip idle and waits for
+// the last block of the one before; together their blocks run side by side.
+// Block ranges first[q] .. first[q + 1] - 1 run body q over 256-point rows.
+// Bound by latency: six launches of 6-17 us on a 45x38x51 FP64 block (8CENT, Boris)
+// become one of 46 us, a step of it 176 -> 138 us; of a 32x32x4 box 133 -> 91 us.
+struct MergeRanges { unsigned first[7]; };
+#define MERGE_TILE Tile{256, 1, 1, TILE_LINEAR | TILE_NOXCD}
+template <typename R>
+__global__ void __launch_bounds__(256) k_b2f_vf(GVT<R> g, const DClock *__restrict__ clk, const R *__restrict__ hmag, R *__restrict__ hB,
+                                                const R *__restrict__ VdV, R *__restrict__ Vf, int kc, MergeRanges mr) {
+    const unsigned b = blockIdx.x;
+    if (b < mr.first[1]) b_vf<R>(b, g, MERGE_TILE, clk, VdV, Vf, kc, 0);
+    else b_b2f<R, R>(b - mr.first[1], g, MERGE_TILE, clk, hmag, hB);
+}
+template <int RM, int BORIS, int MHD, int BG, typename R>
+__global__ void __launch_bounds__(256) k_emf_flux(GVT<R> g, MP m, BGV bg, const DClock *__restrict__ clk, WKT<R> w,
+                                                  const R *__restrict__ Vf, const R *__restrict__ nB, const R *__restrict__ hB,
+                                                  const R *__restrict__ hmag, const R *__restrict__ hGas, R *__restrict__ E,
+                                                  R *__restrict__ Flx, MergeRanges mr) {
+    const unsigned b = blockIdx.x;
+    const Tile t = MERGE_TILE;
+    if constexpr (MHD) {
+        if (b < mr.first[1]) return b_emf<0, RM, BORIS, R>(b, g, t, m, bg, clk, Vf, hGas, w.bn, w.bh, E, nullptr, 0.0);
+        if (b < mr.first[2]) return b_emf<1, RM, BORIS, R>(b - mr.first[1], g, t, m, bg, clk, Vf, hGas, w.bn, w.bh, E, nullptr, 0.0);
+        if (b < mr.first[3]) return b_emf<2, RM, BORIS, R>(b - mr.first[2], g, t, m, bg, clk, Vf, hGas, w.bn, w.bh, E, nullptr, 0.0);
+    }
+    if (b < mr.first[4])
+        b_flux<0, RM, BORIS, MHD, BG, R>(b - mr.first[3], g, t, m, bg, clk, w.Wn, nB, w.Wh, hB, hmag, hGas, Flx, nullptr, 0.0);
+    else if (b < mr.first[5])
+        b_flux<1, RM, BORIS, MHD, BG, R>(b - mr.first[4], g, t, m, bg, clk, w.Wn, nB, w.Wh, hB, hmag, hGas, Flx, nullptr, 0.0);
+    else
+        b_flux<2, RM, BORIS, MHD, BG, R>(b - mr.first[5], g, t, m, bg, clk, w.Wn, nB, w.Wh, hB, hmag, hGas, Flx, nullptr, 0.0);
 }
 
 // Interfaces per k_flux_col thread for columns of L interfaces over `cols`
@@ -1476,17 +1513,11 @@ __host__ __device__ __forceinline__ long bc_shell_count(const BcShell &s) {
     return (long)s.np[0] * s.np[1] * s.np[2] - (long)s.in[0] * s.in[1] * s.in[2];
 }
 
-// mask: the periodic axes (bit 0 i, 1 j, 2 k) mapped by this pass; the
-// others are left for their own BCs.
-template <typename R>
-__device__ __forceinline__ void b_bc(const unsigned vb, GVT<R> g, const DClock *__restrict__ clk, int do25D, int mask, R *__restrict__ Gas,
-                                            double *__restrict__ mag, R *__restrict__ B) {
-    const BcShell sh = bc_shell(g.Ni, g.Nj, g.Nk, g.Nip, g.Njp, g.Nkp, g.nG, mask, do25D);
-    const long t = (long)vb * blockDim.x + threadIdx.x;
+// (i, j, k) of shell point t; false past the shell
+__device__ __forceinline__ bool bc_shell_pos(const BcShell &sh, long t, int &i, int &j, int &k) {
     const long nplane = (long)(sh.np[2] - sh.in[2]) * sh.np[0] * sh.np[1];
     const long nrow = (long)sh.in[2] * (sh.np[1] - sh.in[1]) * sh.np[0];
-    if (t >= bc_shell_count(sh) || clk->halt) return;
-    int i, j, k;
+    if (t >= bc_shell_count(sh)) return false;
     if (t < nplane) {
         const long pl = (long)sh.np[0] * sh.np[1];
         const int p = (int)(t / pl), r = (int)(t % pl);
@@ -1508,6 +1539,17 @@ __device__ __forceinline__ void b_bc(const unsigned vb, GVT<R> g, const DClock *
         j = sh.lo[1] + rr % sh.in[1];
         k = sh.lo[2] + rr / sh.in[1];
     }
+    return true;
+}
+
+// mask: the periodic axes (bit 0 i, 1 j, 2 k) mapped by this pass; the
+// others are left for their own BCs.
+template <typename R>
+__device__ __forceinline__ void b_bc(const unsigned vb, GVT<R> g, const DClock *__restrict__ clk, int do25D, int mask, R *__restrict__ Gas,
+                                            double *__restrict__ mag, R *__restrict__ B) {
+    const BcShell sh = bc_shell(g.Ni, g.Nj, g.Nk, g.Nip, g.Njp, g.Nkp, g.nG, mask, do25D);
+    int i, j, k;
+    if (clk->halt || !bc_shell_pos(sh, (long)vb * blockDim.x + threadIdx.x, i, j, k)) return;
     const int idx = i + sh.np[0] * (j + sh.np[1] * k);
     const int a0 = g.nG;
     const size_t nc = g.nc, nf = g.nf;
@@ -1547,6 +1589,41 @@ template <typename R>
 __global__ void __launch_bounds__(256) k_bc(GVT<R> g, const DClock *__restrict__ clk, int do25D, int mask, R *__restrict__ Gas,
                                             double *__restrict__ mag, R *__restrict__ B) {
     b_bc<R>(blockIdx.x, g, clk, do25D, mask, Gas, mag, B);
+}
+
+// The all-periodic 3D BCs and bFlux2Fld of the ghost cells in one pass.  A ghost
+// cell's six faces after the BCs are the owned (or untouched) faces the maps name, and
+// no thread writes those, so the pass needs none of its own results.  (Bxyz of the active
+// cells: see k_b2f_shell.)  Two launches before: 0.063 + 0.100 ms at 256^3 FP64,
+// 6.8 + 3.8 us on a 32x32x4 box -> 0.145 ms and 8-10 us, and one launch less.
+template <typename R>
+__device__ __forceinline__ void b_bc_b2f(const unsigned vb, GVT<R> g, const DClock *__restrict__ clk, R *__restrict__ Gas,
+                                         double *__restrict__ mag, R *__restrict__ B) {
+    b_bc<R>(vb, g, clk, 0, 7, Gas, mag, (R *)nullptr);
+    const BcShell sh = bc_shell(g.Ni, g.Nj, g.Nk, g.Nip, g.Njp, g.Nkp, g.nG, 7, 0);
+    int i, j, k;
+    if (clk->halt || !bc_shell_pos(sh, (long)vb * blockDim.x + threadIdx.x, i, j, k)) return;
+    if (i >= g.Ni || j >= g.Nj || k >= g.Nk) return;
+    const int a0 = g.nG;
+    const size_t nc = g.nc, nf = g.nf;
+    const int ic = pmap_c(i, a0, g.Nip), jc = pmap_c(j, a0, g.Njp), kc = pmap_c(k, a0, g.Nkp);
+    // the lower and upper face of the pair along its normal
+    const int il = pmap_f(i, a0, g.Nip), iu = pmap_f(i + 1, a0, g.Nip);
+    const int jl = pmap_f(j, a0, g.Njp), ju = pmap_f(j + 1, a0, g.Njp);
+    const int kl = pmap_f(k, a0, g.Nkp), ku = pmap_f(k + 1, a0, g.Nkp);
+    const double fl[6] = {mag[fi(g, il, jc, kc)], mag[fi(g, iu, jc, kc)],
+                          mag[nf + fi(g, ic, jl, kc)], mag[nf + fi(g, ic, ju, kc)],
+                          mag[2 * nf + fi(g, ic, jc, kl)], mag[2 * nf + fi(g, ic, jc, ku)]};
+    double b[3];
+    cell_bxyz_fl(g, fl, i, j, k, b);
+    const int c = ci(g, i, j, k);
+#pragma unroll
+    for (int x = 0; x < 3; x++) B[nc * x + c] = R(b[x]);
+}
+template <typename R>
+__global__ void __launch_bounds__(256) k_bc_b2f(GVT<R> g, const DClock *__restrict__ clk, R *__restrict__ Gas,
+                                                double *__restrict__ mag, R *__restrict__ B) {
+    b_bc_b2f<R>(blockIdx.x, g, clk, Gas, mag, B);
 }
 
 // One face's non-periodic BC, restating bcs.F90: zeroGrad_{i,o}bc{I,J,K}

@@ -27,7 +27,7 @@ from collections import defaultdict
 
 # kernel-name prefix -> stage name used by the library's stage timers
 STAGE_OF = [
-    ("k_clock_begin", "clock"), ("k_predict", "predictor"), ("k_b2f_shell", "bflux_post"), ("k_b2f_rows", "ring"),
+    ("k_predict", "predictor"), ("k_bc_b2f", "bcs"), ("k_b2f_vf", "mom2face"), ("k_emf_flux", "flux_i"), ("k_b2f_shell", "bflux_post"), ("k_b2f_rows", "ring"),
     ("k_b2f", "bflux_half"), ("k_ring_", "ring"), ("k_pole_e", "ring"), ("k_fix_e", "ring"),
     ("k_celldt_rows", "celldt"), ("k_bc_wind", "bcs"), ("k_wind_", "bcs"),
     ("k_vf", "mom2face"), ("k_emf_jcol", "emf_j"), ("k_emf<0", "emf_i"), ("k_emf<1", "emf_j"), ("k_emf<2", "emf_k"),
