@@ -80,7 +80,7 @@ struct gam_handle {
     int npart = 0;             // blocks of the 1-D CellDT launch
     int pcap = 0;              // capacity of partial (block minima / sums)
     DClock *clk = nullptr;      // device
-    DClock *clk_host = nullptr; // pinned
+    DClock *clk_host = nullptr; // pinned; equals *clk once the stream's work is done (k_dtfinal writes both)
     std::string err;
     bool timing = false;
     std::vector<PendingEv> pending;
@@ -624,7 +624,6 @@ extern "C" int gam_put_state(gam_handle *h, int which, double time, const double
     }
     HIPCHK(h, hipGetLastError());
     HIPCHK(h, hipStreamSynchronize(h->stream));
-    HIPCHK(h, hipMemcpy(h->clk_host, h->clk, sizeof(DClock), hipMemcpyDeviceToHost));
     if (which == 0) h->clk_host->stime = time; else h->clk_host->otime = time;
     HIPCHK(h, hipMemcpy(h->clk, h->clk_host, sizeof(DClock), hipMemcpyHostToDevice));
     return 0;
@@ -646,7 +645,6 @@ extern "C" int gam_put_state_device(gam_handle *h, int which, double time, const
     else launch_b2f<double, double>(h, ST_BPOST, (const double *)m, b);
     HIPCHK(h, hipGetLastError());
     HIPCHK(h, hipStreamSynchronize(h->stream));
-    HIPCHK(h, hipMemcpy(h->clk_host, h->clk, sizeof(DClock), hipMemcpyDeviceToHost));
     if (which == 0) h->clk_host->stime = time; else h->clk_host->otime = time;
     HIPCHK(h, hipMemcpy(h->clk, h->clk_host, sizeof(DClock), hipMemcpyHostToDevice));
     return 0;
@@ -660,7 +658,6 @@ extern "C" int gam_get_state(gam_handle *h, int which, double *time, double *Gas
     if ((rc = d2h_bulk(h, Gas, g, 5 * gsz(h)))) return rc;
     if ((rc = d2h_bulk(h, magFlux, m, 3 * fsz(h), which == 2))) return rc;
     if ((rc = d2h_bulk(h, Bxyz, b, 3 * gsz(h)))) return rc;
-    HIPCHK(h, hipMemcpyAsync(h->clk_host, h->clk, sizeof(DClock), hipMemcpyDeviceToHost, h->stream));
     if ((rc = gam_sync(h))) return rc;
     if (time) *time = which == 0 ? h->clk_host->stime : (which == 1 ? h->clk_host->otime : h->clk_host->stime + h->clk_host->pdt);
     return 0;
@@ -669,7 +666,6 @@ extern "C" int gam_get_state(gam_handle *h, int which, double *time, double *Gas
 extern "C" int gam_set_clock(gam_handle *h, const gam_clock *c) {
     if (!h || !c) return -1;
     HIPCHK(h, hipStreamSynchronize(h->stream));
-    HIPCHK(h, hipMemcpy(h->clk_host, h->clk, sizeof(DClock), hipMemcpyDeviceToHost));
     DClock &d = *h->clk_host;
     d.t = c->t; d.dt = c->dt; d.dt0 = c->dt0; d.stime = c->stateTime; d.otime = c->oStateTime;
     d.ts = c->ts; d.status = c->status; d.dt0_after = c->dt0_after; d.ncpr = c->ncpr; d.cpr_pending = 0;
@@ -680,8 +676,7 @@ extern "C" int gam_set_clock(gam_handle *h, const gam_clock *c) {
 
 extern "C" int gam_get_clock(gam_handle *h, gam_clock *c) {
     if (!h || !c) return -1;
-    HIPCHK(h, hipMemcpyAsync(h->clk_host, h->clk, sizeof(DClock), hipMemcpyDeviceToHost, h->stream));
-    int rc = gam_sync(h);
+    int rc = gam_sync(h);   // the kernels that change the clock keep clk_host up to date (k_dtfinal)
     if (rc) return rc;
     const DClock &d = *h->clk_host;
     c->t = d.t; c->dt = d.dt; c->dt0 = d.dt0; c->stateTime = d.stime; c->oStateTime = d.otime;
@@ -995,7 +990,7 @@ static int ensure_partial(gam_handle *h, int n) {
 // np = number of block minima in h->partial (calc != 0)
 static void launch_dtfinal(gam_handle *h, int advance, int calc, int np) {
     StageTimer t(h, ST_DTFINAL);
-    PLAUNCH(h, (k_dtfinal), (b_dtfinal), dim3(1), 1024, h->clk, h->partial, np, advance, calc);
+    PLAUNCH(h, (k_dtfinal), (b_dtfinal), dim3(1), 1024, h->clk, h->clk_host, h->partial, np, advance, calc);
 }
 
 // StateCPR on State when the CalcDT just done asked for it (doCPR only; the
@@ -1591,7 +1586,6 @@ extern "C" int gam_enforce_bcs(gam_handle *h) {
 
 extern "C" int gam_step(gam_handle *h, int nsteps) {
     if (!h || nsteps < 0) return -1;
-    HIPCHK(h, hipMemcpyAsync(h->clk_host, h->clk, sizeof(DClock), hipMemcpyDeviceToHost, h->stream));
     HIPCHK(h, hipStreamSynchronize(h->stream));
     const int ts0 = h->clk_host->ts;
     const int s0 = h->s;

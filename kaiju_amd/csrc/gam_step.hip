@@ -1358,8 +1358,20 @@ __global__ void __launch_bounds__(256) k_celldt(GVT<R> g, MP m, BGV bg, const DC
 }
 
 // UpdateStateData time update (gamapp.F90:112-114, mhdgroup.F90:104-105,255)
-// when advance != 0, then CalcDT's checks and clamps (step.F90:103-166).
-__device__ __forceinline__ void b_dtfinal(const unsigned vb, DClock *clk, const double *__restrict__ partial, int np, int advance, int calc) {
+// when advance != 0, then CalcDT's checks and clamps (step.F90:103-166).  host: the
+// handle's pinned copy of the clock, written with every change of it, so that the
+// host reads the clock after waiting for the stream, without a copy of its own.
+__device__ __forceinline__ void clock_to_host(const DClock *clk, DClock *host) {
+    static_assert(sizeof(DClock) % sizeof(double) == 0, "whole words");
+    const double *s = (const double *)clk;
+    volatile double *d = (volatile double *)host;
+    for (size_t q = 0; q < sizeof(DClock) / sizeof(double); q++) d[q] = s[q];
+#ifndef GAM_EMU
+    __threadfence_system();
+#endif
+}
+__device__ __forceinline__ void b_dtfinal(const unsigned vb, DClock *clk, DClock *host, const double *__restrict__ partial, int np,
+                                          int advance, int calc) {
     if (clk->halt) return;
     if (threadIdx.x == 0) clk->cpr_pending = 0;
 #ifdef GAM_EMU
@@ -1383,8 +1395,8 @@ __device__ __forceinline__ void b_dtfinal(const unsigned vb, DClock *clk, const 
         clk->ts = clk->ts + 1;
         clk->t = clk->t + clk->dt;
     }
-    if (!calc) return;
-    if (clk->fixedTimestep) { clk->status = 0; return; }
+    if (!calc) { clock_to_host(clk, host); return; }
+    if (clk->fixedTimestep) { clk->status = 0; clock_to_host(clk, host); return; }
     double dtOld = clk->dt;
     int disaster = (dtMin == GAM_HUGE), bad = 0;
     double dt = dtMin;
@@ -1408,9 +1420,10 @@ __device__ __forceinline__ void b_dtfinal(const unsigned vb, DClock *clk, const 
     if (status) clk->halt = 1;   // the reference stops here (step.F90:138-154); the host decides
     // console-output dt0 capture (output.F90:57-59) at the configured cadence
     if (clk->dt0_after > 0 && clk->ts >= clk->dt0_after && clk->dt0 < GAM_TINY) clk->dt0 = clk->dt;
+    clock_to_host(clk, host);
 }
-__global__ void k_dtfinal(DClock *clk, const double *__restrict__ partial, int np, int advance, int calc) {
-    b_dtfinal(blockIdx.x, clk, partial, np, advance, calc);
+__global__ void k_dtfinal(DClock *clk, DClock *host, const double *__restrict__ partial, int np, int advance, int calc) {
+    b_dtfinal(blockIdx.x, clk, host, partial, np, advance, calc);
 }
 
 // step.F90:279-302 StateCPR after a bad (not disastrous) CalcDT with doCPR:
