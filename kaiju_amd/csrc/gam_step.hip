@@ -1358,45 +1358,17 @@ __global__ void __launch_bounds__(256) k_celldt(GVT<R> g, MP m, BGV bg, const DC
 }
 
 // UpdateStateData time update (gamapp.F90:112-114, mhdgroup.F90:104-105,255)
-// when advance != 0, then CalcDT's checks and clamps (step.F90:103-166).  host: the
-// handle's pinned copy of the clock, written with every change of it, so that the
-// host reads the clock after waiting for the stream, without a copy of its own.
-__device__ __forceinline__ void clock_to_host(const DClock *clk, DClock *host) {
-    static_assert(sizeof(DClock) % sizeof(double) == 0, "whole words");
-    const double *s = (const double *)clk;
-    volatile double *d = (volatile double *)host;
-    for (size_t q = 0; q < sizeof(DClock) / sizeof(double); q++) d[q] = s[q];
-#ifndef GAM_EMU
-    __threadfence_system();
-#endif
-}
-__device__ __forceinline__ void b_dtfinal(const unsigned vb, DClock *clk, DClock *host, const double *__restrict__ partial, int np,
-                                          int advance, int calc) {
-    if (clk->halt) return;
-    if (threadIdx.x == 0) clk->cpr_pending = 0;
-#ifdef GAM_EMU
-    if (threadIdx.x != 0) return;
-    double dtMin = GAM_HUGE;
-    for (int q = 0; q < np; q++) dtMin = fmin(dtMin, partial[q]);
-#else
-    __shared__ double red[16];
-    double v = GAM_HUGE;
-    for (int q = threadIdx.x; q < np; q += blockDim.x) v = fmin(v, partial[q]);
-    v = wave_min(v);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    double dtMin = red[0];
-    for (int q = 1; q < (int)(blockDim.x >> 6); q++) dtMin = fmin(dtMin, red[q]);
-#endif
+// when advance != 0, then CalcDT's checks and clamps (step.F90:103-166).
+__device__ __forceinline__ void clock_advance(DClock *clk, double dtMin, int advance, int calc) {
+    clk->cpr_pending = 0;
     if (advance) {
         clk->otime = clk->stime;
         clk->stime = clk->stime + clk->dt;
         clk->ts = clk->ts + 1;
         clk->t = clk->t + clk->dt;
     }
-    if (!calc) { clock_to_host(clk, host); return; }
-    if (clk->fixedTimestep) { clk->status = 0; clock_to_host(clk, host); return; }
+    if (!calc) return;
+    if (clk->fixedTimestep) { clk->status = 0; return; }
     double dtOld = clk->dt;
     int disaster = (dtMin == GAM_HUGE), bad = 0;
     double dt = dtMin;
@@ -1420,7 +1392,38 @@ __device__ __forceinline__ void b_dtfinal(const unsigned vb, DClock *clk, DClock
     if (status) clk->halt = 1;   // the reference stops here (step.F90:138-154); the host decides
     // console-output dt0 capture (output.F90:57-59) at the configured cadence
     if (clk->dt0_after > 0 && clk->ts >= clk->dt0_after && clk->dt0 < GAM_TINY) clk->dt0 = clk->dt;
-    clock_to_host(clk, host);
+}
+
+// The minimum of the np block minima, then clock_advance.  host: the handle's
+// pinned copy of the clock, written with every change, so that the host reads it
+// after waiting for the stream, without a copy of its own; one store of the first
+// lanes (a serial copy by one thread with a system fence took 8 us more).
+__device__ __forceinline__ void b_dtfinal(const unsigned vb, DClock *clk, DClock *host, const double *__restrict__ partial, int np,
+                                          int advance, int calc) {
+    static_assert(sizeof(DClock) % sizeof(double) == 0 && sizeof(DClock) / sizeof(double) <= 64, "one word per lane");
+    constexpr unsigned NW = sizeof(DClock) / sizeof(double);
+    if (clk->halt) return;
+#ifdef GAM_EMU
+    if (threadIdx.x != 0) return;
+    double dtMin = GAM_HUGE;
+    for (int q = 0; q < np; q++) dtMin = fmin(dtMin, partial[q]);
+    clock_advance(clk, dtMin, advance, calc);
+    *host = *clk;
+#else
+    __shared__ double red[16];
+    double v = GAM_HUGE;
+    for (int q = threadIdx.x; q < np; q += blockDim.x) v = fmin(v, partial[q]);
+    v = wave_min(v);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();   // every thread has read clk->halt before thread 0 may set it
+    if (threadIdx.x == 0) {
+        double dtMin = red[0];
+        for (int q = 1; q < (int)(blockDim.x >> 6); q++) dtMin = fmin(dtMin, red[q]);
+        clock_advance(clk, dtMin, advance, calc);
+    }
+    __syncthreads();
+    if (threadIdx.x < NW) ((volatile double *)host)[threadIdx.x] = ((volatile double *)clk)[threadIdx.x];
+#endif
 }
 __global__ void k_dtfinal(DClock *clk, DClock *host, const double *__restrict__ partial, int np, int advance, int calc) {
     b_dtfinal(blockIdx.x, clk, host, partial, np, advance, calc);
