@@ -22,7 +22,9 @@
 // box plus one layer only, 4 ghost layers deep).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <algorithm>
 #include <string>
+#include <type_traits>
 #include <vector>
 #include <cstring>
 #include <cmath>
@@ -133,112 +135,139 @@ __global__ void __launch_bounds__(256) k_conv(NetDims d, const u16 *__restrict__
     }
 }
 
-// 8 BF16 at element offset S (0..7) of the 16 aligned ones in w[0..7] (dwords)
-template <int S> __device__ __forceinline__ bf16x8 take8(const uint32_t *w) {
-    uint32_t r[4];
-#pragma unroll
-    for (int j = 0; j < 4; j++)
-        r[j] = (S % 2 == 0) ? w[j + S / 2] : __builtin_amdgcn_alignbyte(w[j + S / 2 + 1], w[j + S / 2], 2);
+// Weight and bias gradients of one layer, dW[tap][co][ci] += sum_p g[p][co] *
+// a[p + off][ci] and db[co] += sum_p g[p][co]: per tap a GEMM with M = output
+// channels, N = input channels and K = cells.  A wave keeps the sums of the 9 taps
+// of one dz (up to 144 accumulator registers) while it walks its cells, 32 per K
+// step: the gradient rows (A, channel-major, 16 aligned bytes per lane) are loaded
+// once for all 9 taps, the activation rows (B) once per dy, 24 bytes per lane from
+// which the three dx are taken (whole dwords or v_alignbyte by one element).  So a K
+// step is up to 38 MFMAs on 14 16-byte and 6 8-byte loads; one tap per wave would
+// load 6 16-byte vectors for every 4 MFMAs and was bound by them.  The bias is one
+// more MFMA against ones, on the waves of the first dz.  The 4 waves of a block add up in
+// LDS and the block writes its sums to a workspace that k_wreduce adds in block
+// order, so the gradients do not depend on the order blocks finish in.  Cells outside the
+// computed range carry a zero gradient (never written, zero from allocation); the
+// arrays' zero padding covers the reads past either end.
+// Per launch on a 104^3 grid, layers 2 / 1 / 0: 463 / 813 / 435 us (one tap per wave,
+// FP32 atomics, and 38 us each for the bias) -> 187 / 231 / 119, and 18 for the sums.
+struct alignas(4) u32x4u { uint32_t v[4]; };   // loads at dword alignment
+struct alignas(4) u32x2u { uint32_t v[2]; };
+__device__ __forceinline__ bf16x8 bf8(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+    const uint32_t r[4] = {a, b, c, d};
     bf16x8 v;
     memcpy(&v, r, 16);
     return v;
 }
-__device__ __forceinline__ void ld16x2(const u16 *p, uint32_t *w) {   // 32 bytes from a 16-byte aligned address
-    const uint4 a = *reinterpret_cast<const uint4 *>(p), b = *reinterpret_cast<const uint4 *>(p + 8);
-    w[0] = a.x; w[1] = a.y; w[2] = a.z; w[3] = a.w; w[4] = b.x; w[5] = b.y; w[6] = b.z; w[7] = b.w;
-}
+#define WG_BLOCKS 170   // blocks per dz: 2 waves on each of the chip's 1024 SIMDs in all
 
-// Weight gradient of one layer, dW[tap][co][ci] += sum_p g[p][co] * a[p + off][ci]:
-// per tap a GEMM with M = output channels, N = input channels and K = cells.
-// Block = 4 waves on 4 consecutive chunks of cells of one tap (blocks ordered
-// tap fastest, so the 27 taps of a chunk run together and share its gradient
-// rows in L2).  Per 32 cells a wave loads its A tiles (gradient, channel-major,
-// 16 aligned bytes per lane: chunks start at multiples of 8 cells) and its B
-// tiles (activation at the tap-shifted cells: 32 aligned bytes per lane, then
-// the 8 wanted values taken at the wave-uniform misalignment S of the tap
-// offset).  Cells outside the computed range carry a zero gradient (never
-// written, zero from allocation), the arrays' zero padding covers the reads
-// past either end.  The 4 waves' sums meet in LDS; one FP32 atomic per weight
-// per block goes to the unpadded parameter layout [tap][nco][nci].
-template <int NCO, int NT, int S>
-__device__ __forceinline__ void wgrad_chunk(const NetDims &d, const u16 *__restrict__ gT, const u16 *__restrict__ aT,
-                                            int c0, int cend, int off, f32x4 (&acc)[NCO / 16][NT]) {
-    const int lane = threadIdx.x & 63, row = lane & 15, kg = lane >> 4;
-    for (int c = c0; c < cend; c += 32) {
-        const int pk = c + 8 * kg;                             // 8 cells of this lane group
-        bf16x8 bv[NT];
-#pragma unroll
-        for (int n = 0; n < NT; n++) {                         // B[k = cell][n = ci] at cell pk + off
-            uint32_t w[8];
-            ld16x2(aT + (size_t)(16 * n + row) * d.ncs + pk + off - S, w);
-            bv[n] = take8<S>(w);
-        }
-#pragma unroll
-        for (int m = 0; m < NCO / 16; m++) {                   // A[m = co][k = cell]
-            const bf16x8 av = ld8(gT + (size_t)(16 * m + row) * d.ncs + pk);
-#pragma unroll
-            for (int n = 0; n < NT; n++) acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv[n], acc[m][n], 0, 0, 0);
-        }
-    }
-}
-
-template <int NCO, int NT>
-__global__ void __launch_bounds__(256) k_wgrad(NetDims d, const u16 *__restrict__ gT, const u16 *__restrict__ aT,
-                                               int chunk, int nchunk, int nco, int nci, float *__restrict__ dW) {
-    __shared__ float red[4][NCO][16 * NT];
-    const int tap = blockIdx.x % NET_TAPS;
+template <int MT, int NT>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+k_wgrad(NetDims d, const u16 *__restrict__ gT, const u16 *__restrict__ aT, int steps,
+                                               float *__restrict__ ws) {
+    __shared__ float red[9 * MT * NT * 256 + MT * 16];
+    const int zi = blockIdx.x % 3, blk = blockIdx.x / 3;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, row = lane & 15, kg = lane >> 4;
-    const int q = (blockIdx.x / NET_TAPS) * 4 + wave;          // this wave's chunk
     const int A0 = d.lo & ~7, A1 = d.lo + 16 * d.ntile;
-    const int off = d.off[tap];
-    f32x4 acc[NCO / 16][NT];
+    const int c0 = A0 + 64 * steps * (blk * 4 + wave), c1 = min(c0 + 64 * steps, A1);
+    const uint32_t o1 = 0x3F803F80u;   // two BF16 ones
+    const bf16x8 ones = bf8(o1, o1, o1, o1);
+    f32x4 acc[3][3][MT][NT], accb[MT];
 #pragma unroll
-    for (int m = 0; m < NCO / 16; m++)
+    for (int m = 0; m < MT; m++) {
+        accb[m] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int n = 0; n < NT; n++) acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (q < nchunk) {
-        const int c0 = A0 + q * chunk, cend = min(c0 + chunk, A1);
-        switch (off & 7) {   // the misalignment S of cell pk + off, pk a multiple of 8
-        case 0: wgrad_chunk<NCO, NT, 0>(d, gT, aT, c0, cend, off, acc); break;
-        case 1: wgrad_chunk<NCO, NT, 1>(d, gT, aT, c0, cend, off, acc); break;
-        case 2: wgrad_chunk<NCO, NT, 2>(d, gT, aT, c0, cend, off, acc); break;
-        case 3: wgrad_chunk<NCO, NT, 3>(d, gT, aT, c0, cend, off, acc); break;
-        case 4: wgrad_chunk<NCO, NT, 4>(d, gT, aT, c0, cend, off, acc); break;
-        case 5: wgrad_chunk<NCO, NT, 5>(d, gT, aT, c0, cend, off, acc); break;
-        case 6: wgrad_chunk<NCO, NT, 6>(d, gT, aT, c0, cend, off, acc); break;
-        default: wgrad_chunk<NCO, NT, 7>(d, gT, aT, c0, cend, off, acc); break;
+        for (int q = 0; q < 9 * NT; q++) acc[q / (3 * NT)][(q / NT) % 3][m][q % NT] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    for (int c = c0; c < c1; c += 64) {
+        const int pk = c + 16 * kg;                            // 16 cells of this lane group, 8 in each of two K steps
+        bf16x8 av[2][MT];                                      // A[m = co][k = cell]
+#pragma unroll
+        for (int m = 0; m < MT; m++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) av[h][m] = ld8(gT + (size_t)(16 * m + row) * d.ncs + pk + 8 * h);
+        if (zi == 0) {
+#pragma unroll
+            for (int m = 0; m < MT; m++)
+#pragma unroll
+                for (int h = 0; h < 2; h++) accb[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[h][m], ones, accb[m], 0, 0, 0);
+        }
+#pragma unroll
+        for (int dy = 0; dy < 3; dy++) {
+            const int off = d.off[9 * zi + 3 * dy + 1];        // the tap dx = 0
+            const bool odd = (off + 1) & 1;                    // uniform: the wanted cells start at an odd element of u
+#pragma unroll
+            for (int n = 0; n < NT; n++) {
+                uint32_t u[10], sh[9];                         // cells pk + off - 1 (- 1 if odd) ..; moved by one element
+                const u16 *p = aT + (ptrdiff_t)(16 * n + row) * d.ncs + (pk + off - 1 - (odd ? 1 : 0));
+                const u32x4u x0 = *reinterpret_cast<const u32x4u *>(p), x1 = *reinterpret_cast<const u32x4u *>(p + 8);
+                const u32x2u y = *reinterpret_cast<const u32x2u *>(p + 16);
+#pragma unroll
+                for (int q = 0; q < 4; q++) { u[q] = x0.v[q]; u[4 + q] = x1.v[q]; }
+                u[8] = y.v[0]; u[9] = y.v[1];
+#pragma unroll
+                for (int q = 0; q < 9; q++) sh[q] = __builtin_amdgcn_alignbyte(u[q + 1], u[q], 2);
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const uint32_t *a = u + 4 * h, *b = sh + 4 * h;
+                    bf16x8 bv[3];
+                    if (odd) { bv[0] = bf8(b[0], b[1], b[2], b[3]); bv[1] = bf8(a[1], a[2], a[3], a[4]); bv[2] = bf8(b[1], b[2], b[3], b[4]); }
+                    else { bv[0] = bf8(a[0], a[1], a[2], a[3]); bv[1] = bf8(b[0], b[1], b[2], b[3]); bv[2] = bf8(a[1], a[2], a[3], a[4]); }
+#pragma unroll
+                    for (int dx = 0; dx < 3; dx++)
+#pragma unroll
+                        for (int m = 0; m < MT; m++)
+                            acc[dy][dx][m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[h][m], bv[dx], acc[dy][dx][m][n], 0, 0, 0);
+                }
+            }
         }
     }
     // D[i = co][j = ci]: lane holds co = 16m + 4kg + r, ci = 16n + row
+    for (int w = 0; w < 4; w++) {
+        if (wave == w) {
 #pragma unroll
-    for (int m = 0; m < NCO / 16; m++)
+            for (int t = 0; t < 9; t++)
 #pragma unroll
-        for (int n = 0; n < NT; n++)
+                for (int m = 0; m < MT; m++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) red[wave][16 * m + 4 * kg + r][16 * n + row] = acc[m][n][r];
-    __syncthreads();
-    for (int e = threadIdx.x; e < NCO * 16 * NT; e += 256) {
-        const int co = e / (16 * NT), ci = e % (16 * NT);
-        if (co < nco && ci < nci)
-            atomicAdd(&dW[((size_t)tap * nco + co) * nci + ci], red[0][co][ci] + red[1][co][ci] + red[2][co][ci] + red[3][co][ci]);
-    }
-}
-
-// bias gradient: db[co] += sum over the tile range of g[p][co]
-template <int NCO>
-__global__ void __launch_bounds__(256) k_bgrad(NetDims d, const u16 *__restrict__ gT, float *__restrict__ db) {
-    __shared__ float red[256];
-    const int co = blockIdx.y;
-    const int n = 16 * d.ntile;
-    float s = 0.f;
-    for (int q = blockIdx.x * 256 + threadIdx.x; q < n; q += gridDim.x * 256) s += bf2f(gT[(size_t)co * d.ncs + d.lo + q]);
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+                    for (int n = 0; n < NT; n++)
+#pragma unroll
+                        for (int r = 0; r < 4; r++) {
+                            float &x = red[((t * MT + m) * 16 + 4 * kg + r) * (16 * NT) + 16 * n + row];
+                            x = w == 0 ? acc[t / 3][t % 3][m][n][r] : x + acc[t / 3][t % 3][m][n][r];
+                        }
+            if (row == 0) {
+#pragma unroll
+                for (int m = 0; m < MT; m++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        float &x = red[9 * MT * NT * 256 + 16 * m + 4 * kg + r];
+                        x = w == 0 ? accb[m][r] : x + accb[m][r];
+                    }
+            }
+        }
         __syncthreads();
     }
-    if (threadIdx.x == 0) atomicAdd(&db[co], red[0]);
+    // workspace of a block index: 27 taps of [co][ci], then the biases
+    float *out = ws + (size_t)blk * (27 * MT * NT * 256 + MT * 16);
+    for (int e = threadIdx.x; e < 9 * MT * NT * 256; e += 256) out[(size_t)zi * (9 * MT * NT * 256) + e] = red[e];
+    if (zi == 0 && threadIdx.x < MT * 16) out[27 * MT * NT * 256 + threadIdx.x] = red[9 * MT * NT * 256 + threadIdx.x];
+}
+
+// the blocks' sums, in block order, onto the unpadded parameter layout [tap][nco][nci], [nco]
+template <int MT, int NT>
+__global__ void __launch_bounds__(256) k_wreduce(const float *__restrict__ ws, int nblk, int nco, int nci, float *__restrict__ dW,
+                                                 float *__restrict__ db) {
+    constexpr int NW = 27 * MT * NT * 256, N = NW + MT * 16;
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    if (e >= N) return;
+    const int ci = e % (16 * NT), co = e < NW ? (e / (16 * NT)) % (16 * MT) : e - NW, tap = e / (MT * NT * 256);
+    if (co >= nco || (e < NW && ci >= nci)) return;
+    float s = 0.f;
+#pragma unroll 10
+    for (int b = 0; b < nblk; b++) s += ws[(size_t)b * N + e];
+    if (e < NW) dW[((size_t)tap * nco + co) * nci + ci] += s;
+    else db[co] += s;
 }
 
 // dL/dout (FP32 [nc][8]) -> BF16 gradient of the last layer, both layouts (16
@@ -514,6 +543,7 @@ struct gam_net {
     u16 *actT0[4] = {}, *grT0[2] = {};   // allocations of the channel-major arrays (NET_PAD before row 0)
     float *out = nullptr;
     float *dbuf = nullptr;               // upstream gradient uploaded from the host
+    float *ws = nullptr;                 // the weight-gradient blocks' sums (k_wgrad)
     float4 scales = {1.f, 1.f, 1.f, 1.f};
     float gamma = 5.f / 3.f;
     float2 offs = {0.f, 0.f};
@@ -536,7 +566,7 @@ static int nfail(gam_net *n, int code, const char *msg, hipError_t e) {
 extern "C" int gam_net_destroy(gam_net *n) {
     if (!n) return 0;
     if (n->own) (void)hipStreamSynchronize(n->own);   // work on a caller's stream: hipFree below waits for the device
-    void *bufs[] = {n->w, n->g, n->m, n->v, n->out, n->dbuf};
+    void *bufs[] = {n->w, n->g, n->m, n->v, n->out, n->dbuf, n->ws};
     for (void *b : bufs) if (b) (void)hipFree(b);
     for (int l = 0; l < 3; l++) { (void)hipFree(n->Wf[l]); (void)hipFree(n->Wb[l]); }
     for (int q = 0; q < 4; q++) { (void)hipFree(n->act[q]); (void)hipFree(n->actT0[q]); }
@@ -590,6 +620,7 @@ extern "C" int gam_net_create(int Ni, int Nj, int Nk, gam_net **out) {
     }
     if (hipMalloc(&n->out, (size_t)nc * 8 * sizeof(float)) != hipSuccess) return cleanup(-3);
     if (hipMalloc(&n->dbuf, (size_t)nc * 8 * sizeof(float)) != hipSuccess) return cleanup(-3);
+    if (hipMalloc(&n->ws, (size_t)WG_BLOCKS * (27 * 1024 + 32) * sizeof(float)) != hipSuccess) return cleanup(-3);
     if (hipMemset(n->out, 0, (size_t)nc * 8 * sizeof(float)) != hipSuccess) return cleanup(-2);
     *out = n;
     return 0;
@@ -734,26 +765,28 @@ extern "C" void *gam_net_infer_event(gam_net *n) { return n ? (void *)n->done : 
 extern "C" int gam_net_backward(gam_net *n, const float *dout) {
     if (!n || !dout) return -1;
     const NetDims &d = n->d;
-    const int chunk = 8192;   // cells per wave, a multiple of 32
-    const int nchunk = (d.lo + 16 * d.ntile - (d.lo & ~7) + chunk - 1) / chunk;
-    const dim3 wg((unsigned)(NET_TAPS * ((nchunk + 3) / 4)));
+    const int cells = d.lo + 16 * d.ntile - (d.lo & ~7);
+    const int steps = std::max(1, (cells + 64 * 4 * WG_BLOCKS - 1) / (64 * 4 * WG_BLOCKS));   // 64-cell steps per wave
+    const int nblk = (cells + 256 * steps - 1) / (256 * steps);
+    auto wgrad = [&](auto mt, auto nt, const u16 *gT, const u16 *aT, int l) {
+        constexpr int MT = decltype(mt)::value, NT = decltype(nt)::value;
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wgrad<MT, NT>), dim3(3 * nblk), 256, 0, n->stream, d, gT, aT, steps, n->ws);
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wreduce<MT, NT>), dim3((27 * MT * NT * 256 + MT * 16 + 255) / 256), 256, 0, n->stream,
+                           (const float *)n->ws, nblk, kCo[l], kCi[l], n->g + woff(l), n->g + boff(l));
+    };
+    const std::integral_constant<int, 1> one;
+    const std::integral_constant<int, 2> two;
     hipLaunchKernelGGL(k_dout, dim3((d.nc + 255) / 256), 256, 0, n->stream, d, dout, n->gr[0], n->grT[0]);
     // layer 2 (linear, 8 outputs padded to 16)
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wgrad<16, 2>), wg, 256, 0, n->stream, d, (const u16 *)n->grT[0], (const u16 *)n->actT[2], chunk,
-                       nchunk, kCo[2], kCi[2], n->g + woff(2));
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_bgrad<16>), dim3(64, 8), 256, 0, n->stream, d, (const u16 *)n->grT[0], n->g + boff(2));
+    wgrad(one, two, n->grT[0], n->actT[2], 2);
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_conv<32, 2, 1>), conv_grid(n), 256, 0, n->stream, d, (const u16 *)n->gr[0], (const u16 *)n->Wb[2],
                        (const float *)nullptr, (const u16 *)n->act[2], n->gr[1], n->grT[1], (float *)nullptr);
     // layer 1
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wgrad<32, 2>), wg, 256, 0, n->stream, d, (const u16 *)n->grT[1], (const u16 *)n->actT[1], chunk,
-                       nchunk, kCo[1], kCi[1], n->g + woff(1));
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_bgrad<32>), dim3(64, 32), 256, 0, n->stream, d, (const u16 *)n->grT[1], n->g + boff(1));
+    wgrad(two, two, n->grT[1], n->actT[1], 1);
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_conv<32, 2, 1>), conv_grid(n), 256, 0, n->stream, d, (const u16 *)n->gr[1], (const u16 *)n->Wb[1],
                        (const float *)nullptr, (const u16 *)n->act[1], n->gr[0], n->grT[0], (float *)nullptr);
     // layer 0 (input gradient not needed)
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wgrad<32, 1>), wg, 256, 0, n->stream, d, (const u16 *)n->grT[0], (const u16 *)n->actT[0], chunk,
-                       nchunk, kCo[0], kCi[0], n->g + woff(0));
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_bgrad<32>), dim3(64, 32), 256, 0, n->stream, d, (const u16 *)n->grT[0], n->g + boff(0));
+    wgrad(two, one, n->grT[0], n->actT[0], 0);
     NCHK(n, hipGetLastError());
     return 0;
 }
