@@ -39,7 +39,7 @@ typedef unsigned short u16;
 #define NET_TAPS 27
 #define NET_G0 7      // K steps of the first layer: ceil(27 taps / 4)
 #define NET_PAD 64    // zero elements before and after a channel-major array
-#define NET_MT 4      // 16-cell tiles per wave in the convolutions
+#define NET_LEAK 0.125f
 
 // round-to-nearest-even FP32 -> BF16 (finite inputs)
 __host__ __device__ inline u16 f2bf(float f) {
@@ -61,77 +61,172 @@ __device__ __forceinline__ bf16x8 ld8(const u16 *p) {   // 16-byte aligned
     return *reinterpret_cast<const bf16x8 *>(p);
 }
 
-#define NET_LEAK 0.125f
-
 // ----------------------------------------------------------------- convolution
+// The training convolutions and the inference (k_infer below) work on bricks of
+// NB_I x NB_J x NB_K cells, wave w of a block on the brick's k row w: NB_J tiles of 16
+// cells (one per j row).
+#define NB_I 16
+#ifndef NB_J
+#define NB_J 4
+#endif
+#define NB_K 4
+#define NB_LI (NB_I + 2)
+#define NB_LJ (NB_J + 2)
+#define NB_LK (NB_K + 2)
+#define NB_LC (NB_LI * NB_LJ * NB_LK)   // staged cells
+#define NB_OC (NB_I * NB_J * NB_K)      // output cells
+
 // Hidden activation: leaky ReLU, x > 0 ? x : x/8 (a slope that keeps every
 // unit trainable; 1/8 is exact in BF16 and FP32).
 // MODE 0: activation, write act_out (channels last) and actT_out (channel-major), NCO = 32
 // MODE 1: linear output, write out[p][0..7] FP32 (NCO = 16, channels 8..15 padding)
 // MODE 2: backward data: multiply by the activation's slope at the forward
 //         output (mask act > 0: 1, else 1/8), write both BF16 layouts, NCO = 32
-// TPK taps per K step: 1 (K = 32 channels of one tap) or 4 (the first layer:
-// K = 8 channels of 4 taps, lane group kg reading tap 4s + kg).
-// One wave = NET_MT tiles of 16 cells x NCO channels (each K step's weights
-// loaded once for all its tiles); blockDim 256 = 4 waves.
-template <int NCO, int MODE, int TPK>
+// CIN = 32, or 8 for the first layer, which packs 4 taps per K step (lane group kg
+// reading tap 4s + kg).
+// A brick's input, the brick and one cell around it, is staged once in LDS (80 bytes per
+// cell of 32 channels: the lanes of a 16-byte read fall on distinct banks), so an input
+// cell comes from L2 2.5 times instead of once per tap.  Neighbours are
+// those of the flattened cell index (p + off), as at the box faces, whose cells
+// are never used; cells outside [lo, lo + 16 ntile) are not stored.  The results
+// leave through LDS, as whole cells and as rows of 16 cells per channel.  Per
+// launch on a 104^3 grid, A operands from L2 before: hidden layer 230 -> 151 us, first
+// 111 -> 84, last 182 -> 70, backward data 272 -> 192.
+template <int CIN, int NCO, int MODE>
 __global__ void __launch_bounds__(256) k_conv(NetDims d, const u16 *__restrict__ in, const u16 *__restrict__ W,
                                               const float *__restrict__ bias, const u16 *__restrict__ mask,
                                               u16 *__restrict__ act_out, u16 *__restrict__ actT_out,
                                               float *__restrict__ out) {
-    const int lane = threadIdx.x & 63;
-    const int tile0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * NET_MT;   // this wave's NET_MT consecutive tiles
-    if (tile0 >= d.ntile) return;                      // whole waves exit together
-    const int row = lane & 15, kg = lane >> 4;         // A row (cell), K group of 8 channels
-    f32x4 acc[NET_MT][NCO / 16];
-#pragma unroll
-    for (int m = 0; m < NET_MT; m++)
-#pragma unroll
-        for (int t = 0; t < NCO / 16; t++) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    static_assert(CIN == 8 || CIN == 32, "8 or 32 input channels");
+    static_assert(NB_I == 16 && NB_K == 4, "one 16-cell tile per row, one k row per wave");
+    constexpr int TPK = CIN == 8 ? 4 : 1;
     constexpr int NSTEP = (NET_TAPS + TPK - 1) / TPK;
-    for (int st = 0; st < NSTEP; st++) {
-        const int tap = TPK == 1 ? st : TPK * st + kg;
-        bf16x8 b[NCO / 16];                            // this K step's weights, used by every tile of the wave
+    constexpr int CS = CIN == 32 ? 40 : 8;                // BF16 elements per staged cell
+    constexpr int OS = 40;                                // and per output cell: 80 bytes
+    constexpr int FS = 36;                                // FP32 elements per output cell (MODE 2)
+    constexpr int OUTB = MODE == 1 ? NB_OC * 32 : NB_OC * OS * 2 + (MODE == 2 ? NB_OC * FS * 4 : 0);
+    constexpr int SB = NB_LC * CS * 2 > OUTB ? NB_LC * CS * 2 : OUTB;
+    __shared__ uint4 smem[SB / 16];
+    u16 *sA = reinterpret_cast<u16 *>(smem);
+    const int nbi = (d.Ni + NB_I - 1) / NB_I, nbj = (d.Nj + NB_J - 1) / NB_J;
+    const int b = blockIdx.x;
+    const int oi = NB_I * (b % nbi), oj = NB_J * ((b / nbi) % nbj), ok = NB_K * (b / (nbi * nbj));   // brick origin
+    {
+        constexpr int PER = CIN / 8;                      // 16-byte pieces per cell
+        constexpr int NIT = (NB_LC * PER + 255) / 256;
+        uint4 v[NIT];
 #pragma unroll
-        for (int t = 0; t < NCO / 16; t++) b[t] = ld8(W + ((size_t)st * NCO + 16 * t + row) * NET_C + 8 * kg);
-        const bool live = TPK == 1 || tap < NET_TAPS;  // K slots past the last tap: weights are zero there too
-        const int q0 = d.lo + 16 * tile0 + row + (live ? d.off[tap] : 0);
+        for (int it = 0; it < NIT; it++) {
+            const int e = threadIdx.x + 256 * it, c = e / PER;
+            const int li = c % NB_LI, lj = (c / NB_LI) % NB_LJ, lk = c / (NB_LI * NB_LJ);
+            const int p = (oi - 1 + li) + d.Ni * ((oj - 1 + lj) + d.Nj * (ok - 1 + lk));
+            v[it] = uint4{0u, 0u, 0u, 0u};
+            if (c < NB_LC && p >= 0 && p < d.nc) v[it] = *reinterpret_cast<const uint4 *>(in + (size_t)p * NET_C + 8 * (e % PER));
+        }
 #pragma unroll
-        for (int m = 0; m < NET_MT; m++) {
-            if (tile0 + m >= d.ntile) break;           // uniform in the wave
-            const bf16x8 a = live ? ld8(in + (size_t)(q0 + 16 * m) * NET_C + (TPK == 1 ? 8 * kg : 0)) : bf16x8{};
-#pragma unroll
-            for (int t = 0; t < NCO / 16; t++) acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[t], acc[m][t], 0, 0, 0);
+        for (int it = 0; it < NIT; it++) {
+            const int e = threadIdx.x + 256 * it, c = e / PER;
+            if (c < NB_LC) smem[c * (CS / 8) + e % PER] = v[it];
         }
     }
-    // D layout: lane holds rows 4*kg + r (cells), column row (channel)
+    __syncthreads();
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, row = lane & 15, kg = lane >> 4;
+    f32x4 acc[NB_J][NCO / 16];
 #pragma unroll
-    for (int m = 0; m < NET_MT; m++) {
-        if (tile0 + m >= d.ntile) break;
-        const int p0 = d.lo + 16 * (tile0 + m);
+    for (int m = 0; m < NB_J; m++)
+#pragma unroll
+        for (int t = 0; t < NCO / 16; t++) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // the K steps' weights (the same for every block, from L2) two steps ahead of their MFMAs
+    const u16 *wl = W + ((size_t)row) * NET_C + 8 * kg;
+    bf16x8 wn[2][NCO / 16];
+#pragma unroll
+    for (int q = 0; q < 2; q++)
+#pragma unroll
+        for (int t = 0; t < NCO / 16; t++) wn[q][t] = ld8(wl + ((size_t)q * NCO + 16 * t) * NET_C);
+    for (int st = 0; st < NSTEP; st++) {
+        const int tap = TPK == 1 ? st : TPK * st + kg;
+        const bool live = TPK == 1 || tap < NET_TAPS;   // K slots past the last tap: weights are zero there too
+        const int tp = live ? tap : 13;
+        bf16x8 bw[NCO / 16];
+        const int sn = st + 2 < NSTEP ? st + 2 : NSTEP - 1;
+#pragma unroll
+        for (int t = 0; t < NCO / 16; t++) {
+            bw[t] = wn[0][t];
+            wn[0][t] = wn[1][t];
+            wn[1][t] = ld8(wl + ((size_t)sn * NCO + 16 * t) * NET_C);
+        }
+        const int dx = tp % 3 - 1, dy = (tp / 3) % 3 - 1, dz = tp / 9 - 1;
+        const int c0 = (wave + 1 + dz) * (NB_LJ * NB_LI) + (1 + dy) * NB_LI + 1 + dx + row;
+#pragma unroll
+        for (int m = 0; m < NB_J; m++) {
+            bf16x8 a = *reinterpret_cast<const bf16x8 *>(sA + (size_t)(c0 + m * NB_LI) * CS + (TPK == 1 ? 8 * kg : 0));
+            if (!live) a = bf16x8{};
+#pragma unroll
+            for (int t = 0; t < NCO / 16; t++) acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bw[t], acc[m][t], 0, 0, 0);
+        }
+    }
+    __syncthreads();   // every wave is done with the staged input: the LDS takes the outputs
+    float *sF = reinterpret_cast<float *>(reinterpret_cast<char *>(smem) + (MODE == 2 ? NB_OC * OS * 2 : 0));
+    // D layout: lane holds cells 4*kg + r of the tile, channel 16*t + row
+#pragma unroll
+    for (int m = 0; m < NB_J; m++)
 #pragma unroll
         for (int t = 0; t < NCO / 16; t++) {
             const int co = 16 * t + row;
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const int p = p0 + 4 * kg + r;
-                float v = acc[m][t][r];
+                const int oc = (wave * NB_J + m) * NB_I + 4 * kg + r;
+                const float v = acc[m][t][r];
                 if (MODE == 0) {
-                    v = v + bias[co];
-                    v = v > 0.f ? v : NET_LEAK * v;
-                    const u16 bb = f2bf(v);
-                    act_out[(size_t)p * NET_C + co] = bb;
-                    actT_out[(size_t)co * d.ncs + p] = bb;
+                    const float x = v + bias[co];
+                    sA[oc * OS + co] = f2bf(x > 0.f ? x : NET_LEAK * x);
                 } else if (MODE == 1) {
-                    if (co < 8) out[(size_t)p * 8 + co] = v + bias[co];
+                    if (co < 8) sF[oc * 8 + co] = v + bias[co];
                 } else {
-                    if (bf2f(mask[(size_t)p * NET_C + co]) <= 0.f) v = NET_LEAK * v;   // slope at the forward output
-                    const u16 bb = f2bf(v);
-                    act_out[(size_t)p * NET_C + co] = bb;
-                    actT_out[(size_t)co * d.ncs + p] = bb;
+                    sF[oc * FS + co] = v;
                 }
             }
         }
+    __syncthreads();
+    const int hi = d.lo + 16 * d.ntile;
+    auto cell = [&](int oc, int &p) {   // flattened index of output cell oc; false: not stored
+        const int i = oi + oc % NB_I, j = oj + (oc / NB_I) % NB_J, k = ok + oc / (NB_I * NB_J);
+        p = i + d.Ni * (j + d.Nj * k);
+        return i < d.Ni && j < d.Nj && k < d.Nk && p >= d.lo && p < hi;
+    };
+    if (MODE == 1) {
+        for (int e = threadIdx.x; e < NB_OC * 2; e += 256) {
+            int p;
+            if (cell(e >> 1, p)) *reinterpret_cast<uint4 *>(out + (size_t)p * 8 + 4 * (e & 1)) = smem[e];
+        }
+        return;
+    }
+    for (int e = threadIdx.x; e < NB_OC * 4; e += 256) {   // whole cells, 8 channels a thread
+        const int oc = e >> 2, q = e & 3;
+        int p;
+        const bool st = cell(oc, p);
+        uint4 *cellp = smem + oc * (OS / 8) + q;
+        if (MODE == 2) {
+            uint4 mk = {0u, 0u, 0u, 0u};
+            if (st) mk = *reinterpret_cast<const uint4 *>(mask + (size_t)p * NET_C + 8 * q);
+            const uint32_t mw[4] = {mk.x, mk.y, mk.z, mk.w};
+            uint32_t o[4];
+#pragma unroll
+            for (int h = 0; h < 4; h++) {
+                float x = sF[oc * FS + 8 * q + 2 * h], y = sF[oc * FS + 8 * q + 2 * h + 1];
+                if (bf2f((u16)(mw[h] & 0xFFFFu)) <= 0.f) x = NET_LEAK * x;   // slope at the forward output
+                if (bf2f((u16)(mw[h] >> 16)) <= 0.f) y = NET_LEAK * y;
+                o[h] = (uint32_t)f2bf(x) | ((uint32_t)f2bf(y) << 16);
+            }
+            *cellp = uint4{o[0], o[1], o[2], o[3]};
+        }
+        if (st) *reinterpret_cast<uint4 *>(act_out + (size_t)p * NET_C + 8 * q) = *cellp;
+    }
+    if (MODE == 2) __syncthreads();
+    for (int e = threadIdx.x; e < NB_OC * NET_C; e += 256) {   // rows of 16 cells per channel
+        const int oc = (e / (NB_I * NET_C)) * NB_I + e % NB_I, co = (e / NB_I) % NET_C;
+        int p;
+        if (cell(oc, p)) actT_out[(size_t)co * d.ncs + p] = sA[oc * OS + co];
     }
 }
 
@@ -270,18 +365,39 @@ __global__ void __launch_bounds__(256) k_wreduce(const float *__restrict__ ws, i
     else db[co] += s;
 }
 
-// dL/dout (FP32 [nc][8]) -> BF16 gradient of the last layer, both layouts (16
-// padded channels); zero outside the computed cells, where the output is not defined
+__device__ __forceinline__ uint4 pack8(const float (&f)[8]) {
+    uint32_t o[4];
+#pragma unroll
+    for (int h = 0; h < 4; h++) o[h] = (uint32_t)f2bf(f[2 * h]) | ((uint32_t)f2bf(f[2 * h + 1]) << 16);
+    return uint4{o[0], o[1], o[2], o[3]};
+}
+// 8 BF16 channels of cell p to the rows of a channel-major array
+__device__ __forceinline__ void put_rows(const uint4 &v, u16 *T, int ncs, int p) {
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int c = 0; c < 8; c++) T[(size_t)c * ncs + p] = (u16)(w[c / 2] >> (16 * (c & 1)));
+}
+
+// dL/dout (FP32 [nc][8]) -> BF16 gradient of the last layer, both layouts; zero
+// outside the computed cells, where the output is not defined.  The cell's
+// channels 8..31 are zeros (the buffer held another layer's gradient); the rows 8..15
+// that the weight gradient also reads only reach outputs it drops.  Whole 16-byte
+// stores: 76 -> 31 us on a 104^3 grid with one 2-byte store per channel before.
 __global__ void __launch_bounds__(256) k_dout(NetDims d, const float *__restrict__ dout, u16 *__restrict__ g, u16 *__restrict__ gT) {
-    const int nc = d.nc;
-    int p = blockIdx.x * 256 + threadIdx.x;
-    if (p >= nc) return;
-    const bool in = p >= d.lo && p < d.lo + 16 * d.ntile;
-    for (int c = 0; c < NET_C; c++) {
-        const u16 b = (c < 8 && in) ? f2bf(dout[(size_t)p * 8 + c]) : (u16)0;
-        g[(size_t)p * NET_C + c] = b;
-        if (c < 16) gT[(size_t)c * d.ncs + p] = b;
+    const int p = blockIdx.x * 256 + threadIdx.x;
+    if (p >= d.nc) return;
+    uint4 v = {0u, 0u, 0u, 0u};
+    if (p >= d.lo && p < d.lo + 16 * d.ntile) {
+        float f[8];
+#pragma unroll
+        for (int c = 0; c < 8; c++) f[c] = dout[(size_t)p * 8 + c];
+        v = pack8(f);
     }
+    uint4 *gp = reinterpret_cast<uint4 *>(g + (size_t)p * NET_C);
+    gp[0] = v;
+#pragma unroll
+    for (int q = 1; q < 4; q++) gp[q] = uint4{0u, 0u, 0u, 0u};
+    put_rows(v, gT, d.ncs, p);
 }
 
 // state -> input features ((rho - rho0)/s_rho, v/s_v, (p - p0)/s_p, B/s_B) of cell p
@@ -310,7 +426,7 @@ __device__ __forceinline__ void features_of(size_t p, size_t n, const R *__restr
     features_calc(q, gamma, sc, off, f);
 }
 
-// the features, BF16, both layouts
+// the features, BF16, both layouts (channels 8..31 stay the zeros of the allocation)
 template <typename R>
 __global__ void __launch_bounds__(256) k_features(int nc, int ncs, const R *__restrict__ Gas, const R *__restrict__ B, float gamma,
                                                   float4 sc, float2 off, u16 *__restrict__ act, u16 *__restrict__ actT) {
@@ -318,11 +434,9 @@ __global__ void __launch_bounds__(256) k_features(int nc, int ncs, const R *__re
     if (p >= nc) return;
     float f[8];
     features_of<R>(p, nc, Gas, B, gamma, sc, off, f);
-    for (int c = 0; c < NET_C; c++) {
-        const u16 b = c < 8 ? f2bf(f[c]) : (u16)0;
-        act[(size_t)p * NET_C + c] = b;
-        actT[(size_t)c * ncs + p] = b;
-    }
+    const uint4 v = pack8(f);
+    *reinterpret_cast<uint4 *>(act + (size_t)p * NET_C) = v;
+    put_rows(v, actT, ncs, p);
 }
 
 // ----------------------------------------------------------------- inference
@@ -340,17 +454,6 @@ __global__ void __launch_bounds__(256) k_features(int nc, int ncs, const R *__re
 // Wave w of the block computes the brick's k row w: NB_J tiles of 16 cells (one
 // per j row).  The results go through LDS to leave as whole cells (64 bytes of
 // BF16 activations, or 32 bytes of FP32 output).
-#define NB_I 16
-#ifndef NB_J
-#define NB_J 4
-#endif
-#define NB_K 4
-#define NB_LI (NB_I + 2)
-#define NB_LJ (NB_J + 2)
-#define NB_LK (NB_K + 2)
-#define NB_LC (NB_LI * NB_LJ * NB_LK)   // staged cells
-#define NB_OC (NB_I * NB_J * NB_K)      // output cells
-
 struct InferBox { int lo[3], n[3], nb[3]; };
 
 template <int CIN, int NCO, int MODE, typename R>
@@ -401,10 +504,7 @@ __global__ void __launch_bounds__(256) k_infer(NetDims d, InferBox bx, const u16
             if (ok_[it]) {
                 float f[8];
                 features_calc(q[it], gamma, sc, offs, f);
-                v.x = (uint32_t)f2bf(f[0]) | ((uint32_t)f2bf(f[1]) << 16);
-                v.y = (uint32_t)f2bf(f[2]) | ((uint32_t)f2bf(f[3]) << 16);
-                v.z = (uint32_t)f2bf(f[4]) | ((uint32_t)f2bf(f[5]) << 16);
-                v.w = (uint32_t)f2bf(f[6]) | ((uint32_t)f2bf(f[7]) << 16);
+                v = pack8(f);
             }
             smem[c] = v;
         }
@@ -706,16 +806,19 @@ extern "C" int gam_net_set_features(gam_net *n, const float *feat) {
     return 0;
 }
 
-static dim3 conv_grid(const gam_net *n) { return dim3((unsigned)((n->d.ntile + 4 * NET_MT - 1) / (4 * NET_MT))); }
+static dim3 conv_grid(const gam_net *n) {
+    const NetDims &d = n->d;
+    return dim3((unsigned)(((d.Ni + NB_I - 1) / NB_I) * ((d.Nj + NB_J - 1) / NB_J) * ((d.Nk + NB_K - 1) / NB_K)));
+}
 
 extern "C" int gam_net_forward(gam_net *n) {
     if (!n) return -1;
     const NetDims &d = n->d;
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_conv<32, 0, 4>), conv_grid(n), 256, 0, n->stream, d, (const u16 *)n->act[0], (const u16 *)n->Wf[0],
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_conv<8, 32, 0>), conv_grid(n), 256, 0, n->stream, d, (const u16 *)n->act[0], (const u16 *)n->Wf[0],
                        (const float *)(n->w + boff(0)), (const u16 *)nullptr, n->act[1], n->actT[1], (float *)nullptr);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_conv<32, 0, 1>), conv_grid(n), 256, 0, n->stream, d, (const u16 *)n->act[1], (const u16 *)n->Wf[1],
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_conv<32, 32, 0>), conv_grid(n), 256, 0, n->stream, d, (const u16 *)n->act[1], (const u16 *)n->Wf[1],
                        (const float *)(n->w + boff(1)), (const u16 *)nullptr, n->act[2], n->actT[2], (float *)nullptr);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_conv<16, 1, 1>), conv_grid(n), 256, 0, n->stream, d, (const u16 *)n->act[2], (const u16 *)n->Wf[2],
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_conv<32, 16, 1>), conv_grid(n), 256, 0, n->stream, d, (const u16 *)n->act[2], (const u16 *)n->Wf[2],
                        (const float *)(n->w + boff(2)), (const u16 *)nullptr, (u16 *)nullptr, (u16 *)nullptr, n->out);
     NCHK(n, hipGetLastError());
     return 0;
@@ -779,11 +882,11 @@ extern "C" int gam_net_backward(gam_net *n, const float *dout) {
     hipLaunchKernelGGL(k_dout, dim3((d.nc + 255) / 256), 256, 0, n->stream, d, dout, n->gr[0], n->grT[0]);
     // layer 2 (linear, 8 outputs padded to 16)
     wgrad(one, two, n->grT[0], n->actT[2], 2);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_conv<32, 2, 1>), conv_grid(n), 256, 0, n->stream, d, (const u16 *)n->gr[0], (const u16 *)n->Wb[2],
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_conv<32, 32, 2>), conv_grid(n), 256, 0, n->stream, d, (const u16 *)n->gr[0], (const u16 *)n->Wb[2],
                        (const float *)nullptr, (const u16 *)n->act[2], n->gr[1], n->grT[1], (float *)nullptr);
     // layer 1
     wgrad(two, two, n->grT[1], n->actT[1], 1);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_conv<32, 2, 1>), conv_grid(n), 256, 0, n->stream, d, (const u16 *)n->gr[1], (const u16 *)n->Wb[1],
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_conv<32, 32, 2>), conv_grid(n), 256, 0, n->stream, d, (const u16 *)n->gr[1], (const u16 *)n->Wb[1],
                        (const float *)nullptr, (const u16 *)n->act[1], n->gr[0], n->grT[0], (float *)nullptr);
     // layer 0 (input gradient not needed)
     wgrad(two, one, n->grT[0], n->actT[0], 0);

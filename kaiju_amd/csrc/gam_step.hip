@@ -1867,19 +1867,23 @@ __global__ void __launch_bounds__(256) k_corr_cells(GVT<R> g, int do25D, const f
         const int a0 = g.nG;
         const bool active = i >= a0 && i < a0 + g.Nip && j >= a0 && j < a0 + g.Njp && k >= a0 && k < a0 + g.Nkp;
         const double wv[5] = {w0, w1, w1, w1, w4};
+        double sum[5] = {0, 0, 0, 0, 0}, V = 1.0;
+        if (active) {   // the faces and the upper cells' images once for the five variables
+            V = g.dvol[idx];
+            const int f = fi(g, i, j, k);
+            for (int d = 0; d < 3; d++) {
+                if (do25D && d == 2) continue;
+                const double lo = s * (double)g.face[nf * d + f], hi = s * (double)g.face[nf * d + f + fstride(g, d)];
+                const size_t up = pimg(g, i + (d == 0), j + (d == 1), k + (d == 2));
+#pragma unroll
+                for (int v = 0; v < 5; v++) sum[v] += lo * (double)o[(size_t)idx * 8 + v] - hi * (double)o[up * 8 + v];
+            }
+        }
+#pragma unroll
         for (int v = 0; v < 5; v++) {
             double r = 0.0;
             if (active) {
-                const double V = g.dvol[idx];
-                double sum = 0.0;
-                for (int d = 0; d < 3; d++) {
-                    if (do25D && d == 2) continue;
-                    const int f = fi(g, i, j, k), fs = fstride(g, d);
-                    const size_t up = pimg(g, i + (d == 0), j + (d == 1), k + (d == 2));
-                    sum += s * (double)g.face[nf * d + f] * (double)o[(size_t)idx * 8 + v]
-                         - s * (double)g.face[nf * d + f + fs] * (double)o[up * 8 + v];
-                }
-                const double dU = dt * sum / V;
+                const double dU = dt * sum[v] / V;
                 const double e = dU - tG[nc * v + idx];
                 l += wv[v] * e * e;
                 r = 2.0 * wv[v] * e / V;
