@@ -67,6 +67,7 @@ struct gam_handle {
     double *ringTab = nullptr;         // cos, sin of the ring angles phi_n
     double *ringMean = nullptr;        // ring-average scratch (chunk means, Fourier coefficients)
     size_t ringMean_n = 0;             // its capacity in doubles
+    double pack_share = 1.0;           // recording for a packed graph: all its blocks' zones over this block's
     bool capturing = false;            // gam_graph_create is capturing its steps
     bool vf_partial = false;           // the last step filled only the face velocities its EMFs read
     int fused_np = 0;                  // block minima the fused step's CalcDT reduces
@@ -963,7 +964,7 @@ static int celldt(gam_handle *h, const void *Gas, const void *B) {
 
 // k_update's launch box: (i, j, column of update_kc cells in k); FP64: 2 waves per SIMD
 static int update_kc(const gam_handle *h) {
-    return h->prec ? 1 : col_len(h->gv.Nk, (long)h->gv.Ni * h->gv.Nj, UPDATE_KC, 2 * 65536);
+    return h->prec ? 1 : col_len(h->gv.Nk, (long)(h->pack_share * h->gv.Ni * h->gv.Nj), UPDATE_KC, 2 * 65536);
 }
 static int update_blocks(const gam_handle *h) {
     return tile_blocks(h->tile[ST_UPDATE], h->gv.Ni, h->gv.Nj, cdiv(h->gv.Nk, update_kc(h)));
@@ -1022,7 +1023,7 @@ static void launch_flux_bg(gam_handle *h, int d) {
     R *Flx = P<R>(h->Flx);
     StageTimer t(h, ST_FLUX_I + d);
     const int L = (d == 1 ? ny : nz) + 1;   // interfaces along a j or k column
-    const int kc = d == 0 ? 0 : flux_col_kc(L, (long)nx * (d == 1 ? nz : ny));
+    const int kc = d == 0 ? 0 : flux_col_kc(L, (long)(h->pack_share * nx * (d == 1 ? nz : ny)));
     const dim3 gr = d == 0 ? tgrid(h, ST_FLUX_I, nx, ny, nz)
                            : tgrid(h, ST_FLUX_I + d, nx, d == 1 ? cdiv(L, kc) : ny, d == 1 ? nz : cdiv(L, kc));
 #define FLUX_ARGS g, tl, h->mp, h->bgv, h->clk, w.Wn, nB, w.Wh, hB, hmag, hGas, Flx, h->corr, h->corr_scale
@@ -1043,14 +1044,40 @@ static void launch_flux(gam_handle *h, int d) {
     else launch_flux_bg<RM, BO, MH, 0, R>(h, d);
 }
 
+// Whether the I and K edges form their face velocities themselves (k_emf_col; speed
+// only).  Each of its columns starts with 7 more face velocities, so a launch must have
+// the lanes for long ones.  k_vf and the two EMFs, separate / folded in: 256^3 2.85 /
+// 2.30 ms (FP64), 1.44 / 1.19 (FP32); 9.4 M zones of FP32 0.92 / 0.79; 128^3 0.405 /
+// 0.406 (FP64), so the line lies between the last two.  The launch's own tile choice
+// (gam_set_tile) applies to the separate kernel only.
+#ifndef EMF_COL_MIN
+#define EMF_COL_MIN 4e6
+#endif
+static bool emf_cols(const gam_handle *h) {
+    return h->pack_share * h->gv.Nip * (double)h->gv.Njp * h->gv.Nkp >= EMF_COL_MIN;
+}
+
 template <int ED, int RM, int BO, typename R>
 static void launch_emf(gam_handle *h) {
     const GVT<R> &g = view<R>(h);
     const int st = ST_EMF_I + ED;
     const WKT<R> w = wkt<R>(h);
     StageTimer t(h, st);
+    if constexpr (ED != 1) {
+        if (emf_cols(h)) {
+            const int n[3] = {g.Nip + (ED != 0), g.Njp + (ED != 1), g.Nkp + (ED != 2)};
+            const int T2 = (ED + 2) % 3, kc = flux_col_kc(n[T2], (long)(h->pack_share * n[0] * n[3 - T2]));
+            const int ns = cdiv(n[T2], kc);
+            // I edges: 64 x 4 bricks, whose rows share the j stencils of the face velocities
+            const Tile tl = ED == 0 ? Tile{64, 4, 1, sizeof(R) == sizeof(float) ? 0 : TILE_NOXCD} : Tile{256, 1, 1, TILE_LINEAR};
+            const dim3 gr((unsigned)tile_blocks(tl, n[0], T2 == 1 ? ns : n[1], T2 == 2 ? ns : n[2]));
+            PLAUNCH(h, (k_emf_col<ED, RM, BO, R>), (b_emf_col<ED, RM, BO, R>), gr, 256, g, tl, h->mp, h->bgv, h->clk,
+                    P<R>(h->wk[W_VDV]), P<R>(h->hGas), w.bn, w.bh, P<R>(h->E), h->corr, h->corr_scale, kc);
+            return;
+        }
+    }
     if (ED == 1) {   // J edges: k columns with the k stencil in registers (FP64: 2 waves per SIMD, FP32: 4)
-        const int kc = col_len(g.Nkp + 1, (long)(g.Nip + 1) * g.Njp, EMF_KC, (sizeof(R) == sizeof(float) ? 4 : 2) * 65536L);
+        const int kc = col_len(g.Nkp + 1, (long)(h->pack_share * (g.Nip + 1) * g.Njp), EMF_KC, (sizeof(R) == sizeof(float) ? 4 : 2) * 65536L);
         PLAUNCH(h, (k_emf_jcol<RM, BO, R>), (b_emf_jcol<RM, BO, R>), tgrid(h, st, g.Nip + 1, g.Njp, cdiv(g.Nkp + 1, kc)),
                 256, g, h->tile[st], h->mp, h->bgv, h->clk, P<R>(h->Vf), P<R>(h->hGas), w.bn, w.bh, P<R>(h->E), h->corr, h->corr_scale, kc);
     }
@@ -1097,7 +1124,7 @@ static bool merged(const gam_handle *h) {
 template <typename R>
 static void launch_b2f_vf(gam_handle *h) {
     const GVT<R> &g = view<R>(h);
-    const int kc = col_len(g.Nk, (long)g.Ni * g.Nj, VF_KC, 4 * 65536);
+    const int kc = col_len(g.Nk, (long)(h->pack_share * g.Ni * g.Nj), VF_KC, 4 * 65536);
     MergeRanges mr = {};
     mr.first[1] = (unsigned)tile_blocks(MERGE_TILE, g.Ni, g.Nj, cdiv(g.Nk, kc));
     mr.first[2] = mr.first[1] + (unsigned)tile_blocks(MERGE_TILE, g.Ni, g.Nj, g.Nk);
@@ -1143,18 +1170,18 @@ static void launch_b2f(gam_handle *h, int st, const TM *mag, void *B) {
 
 // Mom2Face of the predictor state (FP64: 3 waves per SIMD, FP32: 5)
 template <typename R>
-static void launch_vf(gam_handle *h, int full) {
+static void launch_vf(gam_handle *h, int what) {
     const GVT<R> &g = view<R>(h);
-    const int kc = col_len(g.Nk, (long)g.Ni * g.Nj, VF_KC, 4 * 65536);
+    const int kc = col_len(g.Nk, (long)(h->pack_share * g.Ni * g.Nj), VF_KC, 4 * 65536);
     PLAUNCH(h, (k_vf<R>), (b_vf<R>), tgrid(h, ST_MOM2FACE, g.Ni, g.Nj, cdiv(g.Nk, kc)), 256, g, h->tile[ST_MOM2FACE], h->clk,
-            P<R>(h->wk[W_VDV]), P<R>(h->Vf), kc, full);
+            P<R>(h->wk[W_VDV]), P<R>(h->Vf), kc, what);
 }
 
 // The rest of the last step's face velocities (gam_get_work), from its predictor
 // state and the geometry it ran on: also before that geometry changes
 static int complete_vf(gam_handle *h) {
     if (!h->vf_partial) return 0;
-    if (h->prec) launch_vf<float>(h, 1); else launch_vf<double>(h, 1);
+    if (h->prec) launch_vf<float>(h, VF_FULL); else launch_vf<double>(h, VF_FULL);
     HIPCHK(h, hipGetLastError());
     h->vf_partial = false;
     return 0;
@@ -1208,7 +1235,7 @@ static int advance_t(gam_handle *h, int fuse_dt) {
         { StageTimer t(h, ST_BHALF); launch_b2f<R, R>(h, ST_BHALF, P<R>(h->hmag), h->hB); }
         if (m.doMHD) {
             StageTimer t(h, ST_MOM2FACE);
-            launch_vf<R>(h, 0);
+            launch_vf<R>(h, emf_cols(h) ? VF_K : VF_NEEDED);
             h->vf_partial = true;
         }
     }
@@ -1806,9 +1833,13 @@ extern "C" int gam_graph_create_packed(gam_handle *const *hs, int n, int nsteps,
             return fail(h, -1, "gam_graph_create_packed: periodic MHD blocks only (no ring average, no correction)");
     }
     std::vector<std::vector<std::unique_ptr<PackRec>>> recs(n);
+    auto zones = [](const gam_handle *h) { return (double)h->gv.Nip * h->gv.Njp * h->gv.Nkp; };
+    double all = 0.0;
+    for (int q = 0; q < n; q++) all += zones(hs[q]);
     for (int q = 0; q < n; q++) {
         gam_handle *h = hs[q];
         h->rec = &recs[q];
+        h->pack_share = all / zones(h);   // column lengths for the packed launch, not for this block alone
         int rc = 0;
         for (int k = 0; k < nsteps && !rc; k++) {   // gam_step's sequence; the State swaps return with nsteps even
             rc = advance(h, 1);
@@ -1817,6 +1848,7 @@ extern "C" int gam_graph_create_packed(gam_handle *const *hs, int n, int nsteps,
             if (!rc) rc = bcs(h, true);
         }
         h->rec = nullptr;
+        h->pack_share = 1.0;
         if (rc) return rc;
     }
     // Merge the handles' launch sequences: each packed launch takes, of the

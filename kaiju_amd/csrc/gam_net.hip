@@ -233,11 +233,12 @@ __global__ void __launch_bounds__(256) k_conv(NetDims d, const u16 *__restrict__
 // Weight and bias gradients of one layer, dW[tap][co][ci] += sum_p g[p][co] *
 // a[p + off][ci] and db[co] += sum_p g[p][co]: per tap a GEMM with M = output
 // channels, N = input channels and K = cells.  A wave keeps the sums of the 9 taps
-// of one dz (up to 144 accumulator registers) while it walks its cells, 32 per K
-// step: the gradient rows (A, channel-major, 16 aligned bytes per lane) are loaded
-// once for all 9 taps, the activation rows (B) once per dy, 24 bytes per lane from
-// which the three dx are taken (whole dwords or v_alignbyte by one element).  So a K
-// step is up to 38 MFMAs on 14 16-byte and 6 8-byte loads; one tap per wave would
+// of one dz (up to 144 accumulator registers) while it walks its cells, 64 (two K
+// steps, a whole 128-byte line of each row) at a time: the gradient rows (A,
+// channel-major, 32 aligned bytes per lane) are loaded once for all 9 taps, the
+// activation rows (B) once per dy, 40 bytes per lane from which the three dx are taken
+// (whole dwords or v_alignbyte by one element).  So 64 cells are up to 76 MFMAs on 16
+// 16-byte and 6 8-byte loads; one tap per wave would
 // load 6 16-byte vectors for every 4 MFMAs and was bound by them.  The bias is one
 // more MFMA against ones, on the waves of the first dz.  The 4 waves of a block add up in
 // LDS and the block writes its sums to a workspace that k_wreduce adds in block

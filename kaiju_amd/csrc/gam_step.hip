@@ -353,15 +353,18 @@ __device__ __forceinline__ void mom2face(const GVT<R> &g, const R *__restrict__ 
 
 // Vf arrays: VfA[dT1][xyz] stored as slab (3*dT1 + xyz).  Each thread walks
 // kc <= VF_KC cells up a k column; the k-direction stencil (8 points along k) is a
-// window kept in registers, shifted by one point per cell.  full: every cell the
-// reference fills; else only those the edge EMFs read (K edges take the I faces'
+// window kept in registers, shifted by one point per cell.  VF_FULL: every cell the
+// reference fills; VF_NEEDED: only those the edge EMFs read (K edges take the I faces'
 // velocities on the active k, I edges the J faces' on the active i, J edges the K
 // faces' on the active j): on a box 4 cells deep that is a third of the I faces.
+// VF_K: of those only the K faces' (k_emf_col forms the others itself).
+enum { VF_NEEDED = 0, VF_FULL = 1, VF_K = 2 };
 #define VF_KC 8
 template <typename R>
 __device__ __forceinline__ void b_vf(const unsigned vb, GVT<R> g, Tile t, const DClock *__restrict__ clk, const R *__restrict__ VdV,
-                                            R *__restrict__ Vf, int kc, int full) {
+                                            R *__restrict__ Vf, int kc, int what) {
     int i, j, kb;
+    const bool full = what == VF_FULL;
     if (!tile_pos(vb, t, g.Ni, g.Nj, cdiv(g.Nk, kc), i, j, kb) || (clk->halt && !full)) return;
     const int a0 = g.nG;
     const size_t nc = g.nc;
@@ -376,12 +379,12 @@ __device__ __forceinline__ void b_vf(const unsigned vb, GVT<R> g, Tile t, const 
         const int idx = ci(g, i, j, k);
         R v[3];
         // dT1 = I (used by K edges): i in is..ie+1   (fields.F90:161-175)
-        if (i >= a0 && i <= a0 + g.Nip && (full || (k >= a0 && k < a0 + g.Nkp))) {
+        if (what != VF_K && i >= a0 && i <= a0 + g.Nip && (full || (k >= a0 && k < a0 + g.Nkp))) {
             mom2face(g, VdV, idx, 0, v);
             st_nt(&Vf[nc * 0 + idx], v[0]); st_nt(&Vf[nc * 1 + idx], v[1]); st_nt(&Vf[nc * 2 + idx], v[2]);
         }
         // dT1 = J (used by I edges): j in js..je+1   (fields.F90:119-133)
-        if (j >= a0 && j <= a0 + g.Njp && iact) {
+        if (what != VF_K && j >= a0 && j <= a0 + g.Njp && iact) {
             mom2face(g, VdV, idx, 1, v);
             st_nt(&Vf[nc * 3 + idx], v[0]); st_nt(&Vf[nc * 4 + idx], v[1]); st_nt(&Vf[nc * 5 + idx], v[2]);
         }
@@ -407,8 +410,8 @@ __device__ __forceinline__ void b_vf(const unsigned vb, GVT<R> g, Tile t, const 
 }
 template <typename R>
 __global__ void __launch_bounds__(256) k_vf(GVT<R> g, Tile t, const DClock *__restrict__ clk, const R *__restrict__ VdV,
-                                            R *__restrict__ Vf, int kc, int full) {
-    b_vf<R>(blockIdx.x, g, t, clk, VdV, Vf, kc, full);
+                                            R *__restrict__ Vf, int kc, int what) {
+    b_vf<R>(blockIdx.x, g, t, clk, VdV, Vf, kc, what);
 }
 
 // fields.F90:288-362 EdgeLRs: dT1 faces reconstructed along dT2 at face point f;
@@ -593,6 +596,124 @@ __global__ void __launch_bounds__(256) k_emf_jcol(GVT<R> g, Tile t, MP m, BGV bg
                                                   const R *__restrict__ bn, const R *__restrict__ bh, R *__restrict__ E,
                                                   const float *__restrict__ corr, double cs, int kc) {
     b_emf_jcol<RM, BORIS, R>(blockIdx.x, g, t, m, bg, clk, Vf, hGas, bn, bh, E, corr, cs, kc);
+}
+
+// I and K edges with Mom2Face folded in: a thread walks up to kc edges along dT2 (I
+// edges k, K edges j), lanes along i.  The corner velocity is an 8-point
+// interpolation along dT2 of face velocities that are themselves 8-point
+// interpolations along dT1: walking along dT2 forms each face velocity once and
+// keeps the last eight in registers, where k_vf wrote 6 slabs for k_emf to read
+// back 8 times.  The same operations in the same order, so the same bits.
+// Bound by memory at 256^3 (23 slabs of a value per edge, 0.62 ms in FP64 at the rate of a
+// large copy) and the latency of its loads at 2 waves per SIMD.  Measured there, ms for
+// k_vf, the I and the K edges: FP64 0.86 + 1.01 + 0.98 -> 0.26 + 1.03 + 1.01; FP32 bulk
+// 0.40 + 0.53 + 0.51 -> 0.13 + 0.56 + 0.51.
+template <int ED, int RM, int BORIS, typename R>
+__device__ __forceinline__ void b_emf_col(const unsigned vb, GVT<R> g, Tile t, MP m, BGV bg, const DClock *__restrict__ clk,
+                                          const R *__restrict__ VdV, const R *__restrict__ D0, const R *__restrict__ bn,
+                                          const R *__restrict__ bh, R *__restrict__ E, const float *__restrict__ corr, double cs,
+                                          int kc) {
+    constexpr int T1 = (ED + 1) % 3, T2 = (ED + 2) % 3;   // velocities on T1 faces, built along T1, interpolated along T2
+    static_assert(ED != 1, "J edges: b_emf_jcol");
+    const int n3[3] = {g.Nip + (ED != 0), g.Njp + (ED != 1), g.Nkp + (ED != 2)};
+    const int L = n3[T2], nseg = cdiv(L, kc);
+    int p[3];
+    if (!tile_pos(vb, t, n3[0], T2 == 1 ? nseg : n3[1], T2 == 2 ? nseg : n3[2], p[0], p[1], p[2]) || clk->halt) return;
+    const int s0 = p[T2] * kc, ns = L - s0 < kc ? L - s0 : kc;
+    p[T2] = s0;
+    const int i = p[0] + g.nG, j = p[1] + g.nG, k = p[2] + g.nG;
+    const size_t nf = g.nf, nc = g.nc;
+    const int c1 = cstride(g, T1), c2 = cstride(g, T2), f1 = fstride(g, T1), f2 = fstride(g, T2);
+    int c = ci(g, i, j, k), f = fi(g, i, j, k);
+    const R dt = R(clk->dt), pdmb = R(m.pdmb), Ca = R(m.Ca);
+    const R *fA = g.face + nf * T1, *bhA = bh + nf * T1, *bnA = bn + nf * T1;
+    const R *fB = g.face + nf * T2, *bhB = bh + nf * T2, *bnB = bn + nf * T2;
+    const R *Te = g.Te + nf * 9 * ED, *Teb = g.Teb + nf * 4 * ED;
+    // windows along the column, points -4 .. 3 of the edge: T1 face area, area x bh,
+    // area x face velocity; bn at -2 .. 1
+    R A[8], M[8], AX[8], AY[8], AZ[8], nM[4];
+    auto vf = [&](int cc, R a, R &x, R &y, R &z) {   // a * Mom2Face at cell cc (T1 face at its lower side)
+        R sv = R(0.0), sx = R(0.0), sy = R(0.0), sz = R(0.0);
+#pragma unroll
+        for (int n = 0; n < 8; n++) {
+            const int q = cc + (n - 4) * c1;
+            sv += w8<R>(n) * at32(g.vol, q);
+            sx += w8<R>(n) * at32(VdV, q);
+            sy += w8<R>(n) * at32(VdV + nc, q);
+            sz += w8<R>(n) * at32(VdV + 2 * nc, q);
+        }
+        const R dV = rmax(sv, R(GAM_TINY));
+        x = a * (sx / dV); y = a * (sy / dV); z = a * (sz / dV);
+    };
+#pragma unroll
+    for (int n = 0; n < 8; n++) { A[n] = at32(fA, f + (n - 4) * f2); M[n] = A[n] * at32(bhA, f + (n - 4) * f2); }
+#pragma unroll
+    for (int n = 0; n < 4; n++) nM[n] = at32(bnA, f + (n - 2) * f2);
+    // the velocity's newest point is added at the top of each edge
+#pragma unroll
+    for (int n = 0; n < 7; n++) vf(c + (n - 4) * c2, A[n], AX[n], AY[n], AZ[n]);
+    R Dl = at32(D0, c - c2), Dlm = at32(D0, c - c2 - c1);   // the corner's densities of the row before
+#pragma unroll 1
+    for (int s = 0; s < ns; s++) {
+        vf(c + 3 * c2, A[7], AX[7], AY[7], AZ[7]);
+        const R Ai = c8(A);
+        const R dA = rmax(Ai, R(GAM_TINY));
+        const R Vx = c8(AX) / dA, Vy = c8(AY) / dA, Vz = c8(AZ) / dA;
+        const R v1 = Vx * at32(Te + nf * TAN1X, f) + Vy * at32(Te + nf * TAN1Y, f) + Vz * at32(Te + nf * TAN1Z, f);
+        const R v2 = Vx * at32(Te + nf * TAN2X, f) + Vy * at32(Te + nf * TAN2Y, f) + Vz * at32(Te + nf * TAN2Z, f);
+        R vDiff = rroot(sq(v1) + sq(v2));
+        const R Dc0 = at32(D0, c), Dc1 = at32(D0, c - c1);
+        const R Dc = R(0.25) * (Dc0 + Dc1 + Dl + Dlm);
+        Dl = Dc0; Dlm = Dc1;
+        R l, r, bT1L, bT1R, bT2L, bT2R, fA2;
+        get_lrs_w<RM>(pdmb, M, nM, R(1) / Ai, l, r);
+        bT1L = l * Ai; bT1R = r * Ai;
+        {
+            R AB[8], MB[8], nB4[4];
+#pragma unroll
+            for (int n = 0; n < 8; n++) { AB[n] = at32(fB, f + (n - 4) * f1); MB[n] = at32(bhB, f + (n - 4) * f1); }
+#pragma unroll
+            for (int n = 0; n < 4; n++) nB4[n] = at32(bnB, f + (n - 2) * f1);
+            edge_lrs_w<RM>(m, AB, MB, nB4, bT2L, bT2R, fA2);
+        }
+        const R xni = at32(Teb + nf * XNQI, f), yni = at32(Teb + nf * YNQI, f), xnj = at32(Teb + nf * XNQJ, f), ynj = at32(Teb + nf * YNQJ, f);
+        const R detT = R(1.0) / (xni * ynj - xnj * yni);
+        const R bT1 = R(0.5) * (bT1L + bT1R) / Ai, bT2 = R(0.5) * (bT2L + bT2R) / fA2;
+        const R db1 = (bT1R - bT1L) / Ai, db2 = (bT2R - bT2L) / fA2;
+        const R Jd = db2 - db1;
+        R b1 = detT * (ynj * bT1 - yni * bT2), b2 = detT * (-xnj * bT1 + xni * bT2);
+        if (bg.on) {
+            b1 = b1 + R(bg.edgB0[nc * (0 + 2 * ED) + c]);
+            b2 = b2 + R(bg.edgB0[nc * (1 + 2 * ED) + c]);
+        }
+        R vA = rroot(sq(b1) + sq(b2)) / rroot(Dc);
+        if (BORIS) vA = Ca * vA / rroot(sq(Ca) + sq(vA));
+        vDiff = vDiff + vA;
+        const R ed = at32(g.edge + nf * ED, f);
+        vDiff = rmin(vDiff, R(m.CFL) * ed / dt);
+        R e = -(v1 * b2 - v2 * b1) + R(m.Vd0) * vDiff * Jd;
+        e = e * ed;
+        if (corr) e = corr_add(e, cs, (double)ed, corr[pimg(g, i, j + (T2 == 1 ? s : 0), k + (T2 == 2 ? s : 0)) * 8 + 5 + ED]);
+        at32(E + nc * ED, c) = e;
+        const bool more = s + 1 < ns;
+        const int fq = more ? f + 4 * f2 : f, fl = more ? f + 2 * f2 : f;
+#pragma unroll
+        for (int n = 0; n < 7; n++) { A[n] = A[n + 1]; M[n] = M[n + 1]; }
+#pragma unroll
+        for (int n = 0; n < 6; n++) { AX[n] = AX[n + 1]; AY[n] = AY[n + 1]; AZ[n] = AZ[n + 1]; }
+        AX[6] = AX[7]; AY[6] = AY[7]; AZ[6] = AZ[7];
+#pragma unroll
+        for (int n = 0; n < 3; n++) nM[n] = nM[n + 1];
+        A[7] = at32(fA, fq); M[7] = A[7] * at32(bhA, fq); nM[3] = at32(bnA, fl);
+        c += c2; f += f2;
+    }
+}
+template <int ED, int RM, int BORIS, typename R>
+__global__ void __launch_bounds__(256) k_emf_col(GVT<R> g, Tile t, MP m, BGV bg, const DClock *__restrict__ clk,
+                                                 const R *__restrict__ VdV, const R *__restrict__ D0, const R *__restrict__ bn,
+                                                 const R *__restrict__ bh, R *__restrict__ E, const float *__restrict__ corr,
+                                                 double cs, int kc) {
+    b_emf_col<ED, RM, BORIS, R>(blockIdx.x, g, t, m, bg, clk, VdV, D0, bn, bh, E, corr, cs, kc);
 }
 
 // ----------------------------------------------------------------- fluxes
@@ -914,7 +1035,7 @@ template <typename R>
 __global__ void __launch_bounds__(256) k_b2f_vf(GVT<R> g, const DClock *__restrict__ clk, const R *__restrict__ hmag, R *__restrict__ hB,
                                                 const R *__restrict__ VdV, R *__restrict__ Vf, int kc, MergeRanges mr) {
     const unsigned b = blockIdx.x;
-    if (b < mr.first[1]) b_vf<R>(b, g, MERGE_TILE, clk, VdV, Vf, kc, 0);
+    if (b < mr.first[1]) b_vf<R>(b, g, MERGE_TILE, clk, VdV, Vf, kc, VF_NEEDED);
     else b_b2f<R, R>(b - mr.first[1], g, MERGE_TILE, clk, hmag, hB);
 }
 template <int RM, int BORIS, int MHD, int BG, typename R>
@@ -937,7 +1058,7 @@ __global__ void __launch_bounds__(256) k_emf_flux(GVT<R> g, MP m, BGV bg, const 
         b_flux<2, RM, BORIS, MHD, BG, R>(b - mr.first[5], g, t, m, bg, clk, w.Wn, nB, w.Wh, hB, hmag, hGas, Flx, nullptr, 0.0);
 }
 
-// Interfaces per k_flux_col thread for columns of L interfaces over `cols`
+// Interfaces (edges) per k_flux_col (k_emf_col) thread for columns of L over `cols`
 // lanes (speed only).  One round of resident blocks is 2 waves on each of 1024
 // SIMDs.  A column start loads 7 points that an interface inside a column does
 // not, so columns are long, at least 24 (lengths 33 to 129 differ by 3% at

@@ -43,16 +43,21 @@ CASES = _cases()
 @pytest.mark.gpu
 @pytest.mark.parametrize("name", list(CASES))
 def test_one_step(name):
+    """The merged launches of small blocks, and the separate ones (the flux columns,
+    and the EMF columns of large blocks where EMF_COL_MIN is 0)."""
     say(f"[shapes] {name}")
     oc = oracle.OracleCase(CASES[name])
     oc.step(1)
-    with app_from_oracle(oc) as app:
+    with app_from_oracle(oc) as app, app_from_oracle(oc) as sep:
         assert app.steps(2) == 0
+        sep.set_timing(True)
+        assert sep.steps(2) == 0
         oc.step(2)
-        e = compare_state(app, oc, 0)
-        say(f"   {e}")
-        assert max(e["Gas"], e["magFlux"], e["Bxyz"]) <= TOL_STEP, e
-        assert abs(app.Model.dt - oc.m.dt) <= TOL_STEP * oc.m.dt
+        for a in (app, sep):
+            e = compare_state(a, oc, 0)
+            say(f"   {e}")
+            assert max(e["Gas"], e["magFlux"], e["Bxyz"]) <= TOL_STEP, e
+            assert abs(a.Model.dt - oc.m.dt) <= TOL_STEP * oc.m.dt
 
 
 @pytest.mark.gpu
@@ -82,14 +87,74 @@ def test_volumes_of_skewed_and_folded_cells(amp, mirror):
     assert np.max(np.abs(vol - ref) / ref) <= TOL_METRIC
 
 
-def test_shapes_on_cpu_emulation():
-    """The same checks on the CPU emulation of the kernels, in bounds under AddressSanitizer."""
+@pytest.mark.gpu
+@pytest.mark.parametrize("mkw", [{}, dict(precision=1, rmeth="8CENT", doBoris=True, Ca=6.0)], ids=["fp64", "fp32_8cent_boris"])
+def test_large_block_of_periods(mkw):
+    """A block large enough for the EMF columns (more than EMF_COL_MIN zones, no extent a
+    multiple of 8) that repeats a small periodic block, with the same metrics (positions
+    in multiples of 2^-44, so that whole periods add exactly), does what the small
+    one does in its merged launches.  The same operations but for the absolute positions
+    in the cell-centred field's sums: 6 terms of up to 205 cell sizes, 6 x 205 x 2^-53 =
+    1.4e-13, twice a step for two steps: 1e-12 normwise.  FP32 bulk: 2^-24 and
+    a few tens of operations in a chain, 1e-5."""
+    from kaiju_amd.gamera import GamApp
+    n, rep = (41, 33, 35), (4, 5, 5)
+    say(f"[periods] {mkw}")
+    tol = 1e-5 if mkw.get("precision") else 1e-12
+
+    def tile(a, position=False, rep=rep):   # arrays with ghosts, faces one longer
+        for ax in range(3):
+            ng = (a.shape[ax] - n[ax]) // 2
+            q = np.arange(n[ax] * rep[ax] + a.shape[ax] - n[ax]) - ng
+            a = np.take(a, ng + q % n[ax], axis=ax)
+            if position:   # components (x, y, z) along the 4th axis, unit period
+                a[:, :, :, ax] += (q // n[ax]).reshape([-1 if d == ax else 1 for d in range(3)] + [1] * (a.ndim - 4))
+        return np.asfortranarray(a)
+
+    with GamApp(configs.blast_wave(n, **mkw)) as small:
+        small.InitModel()
+        pos = ("xyz", "xyzcc", "xfc")
+        grid = {k: np.round(v * 2.0**44) / 2.0**44 if k in pos else v for k, v in small.get_grid().items()}
+        small.set_grid({k: tile(v, k in pos, (1, 1, 1)) for k, v in grid.items()})   # ghost cells as the cells they repeat
+        assert small.steps(1) == 0
+        big_spec = configs.blast_wave(tuple(q * r for q, r in zip(n, rep)), **mkw)
+        with GamApp(big_spec) as big:
+            big.set_grid({k: tile(v, k in pos) for k, v in grid.items()})
+            for w in (0, 1):
+                st = small.get_state(w)
+                big.put_state(w, st["time"], *[tile(st[q]) for q in ("Gas", "magFlux", "Bxyz")])
+            big.set_clock(small.get_clock())
+            big._sync_model()
+            assert small.steps(2) == 0
+            assert big.steps(2) == 0
+            assert abs(big.Model.dt - small.Model.dt) <= tol * small.Model.dt
+            g = big_spec.nG
+            xs, ys = small.get_state(0), big.get_state(0)
+            for q in ("Gas", "magFlux", "Bxyz"):
+                x, y = tile(xs[q]), ys[q]
+                act = tuple(slice(g, d - g) for d in x.shape[:3])
+                assert relerr(y[act], x[act]) <= tol
+
+
+EMU_EXPR = {"all": "one_step and (thin or 25d) or volumes", "asan": "one_step and 25d or volumes", "cols": "one_step and not ragged"}
+
+
+@pytest.mark.parametrize("kind", list(EMU_EXPR))
+def test_shapes_on_cpu_emulation(kind, tmp_path):
+    """The same checks on the CPU emulation of the kernels, in bounds under
+    AddressSanitizer; cols: the EMF columns at every size."""
     from tests.emu import build_emu
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-    for asan, expr in ((False, "thin or 25d or volumes"), (True, "thin_k or 25d or volumes")):
-        env = dict(os.environ, KAIJU_EMU_LIB=build_emu.build(asan=asan))
-        if asan:
-            env.update(LD_PRELOAD=build_emu.asan_runtime(), ASAN_OPTIONS="detect_leaks=0:abort_on_error=1")
-        r = subprocess.run([sys.executable, "-m", "pytest", "-q", "-p", "no:cacheprovider", "-m", "gpu", os.path.abspath(__file__),
-                            "-k", expr], cwd=root, env=env, capture_output=True, text=True, timeout=900)
-        assert r.returncode == 0, r.stdout[-3000:] + r.stderr[-2000:]
+    lib = build_emu.build(asan=kind == "asan") if kind != "cols" else str(tmp_path / "libgamera_emu.so")
+    env = dict(os.environ, KAIJU_EMU_LIB=lib)
+    if kind == "asan":
+        env.update(LD_PRELOAD=build_emu.asan_runtime(), ASAN_OPTIONS="detect_leaks=0:abort_on_error=1")
+    if kind == "cols":
+        subprocess.run([build_emu._cxx(), "-std=c++17", "-O1", "-fPIC", "-shared", "-DGAM_EMU", "-DEMF_COL_MIN=0", "-ffp-contract=off",
+                        "-fno-fast-math", "-fsanitize=address", "-fno-omit-frame-pointer", "-x", "c++", "-I",
+                        os.path.join(root, "include"), "-I", build_emu.CSRC, "-I", build_emu.HERE,
+                        os.path.join(build_emu.CSRC, "gam_api.hip"), "-o", lib], check=True)
+        env.update(LD_PRELOAD=build_emu.asan_runtime(), ASAN_OPTIONS="detect_leaks=0:abort_on_error=1")
+    r = subprocess.run([sys.executable, "-m", "pytest", "-q", "-p", "no:cacheprovider", "-m", "gpu", os.path.abspath(__file__),
+                        "-k", EMU_EXPR[kind]], cwd=root, env=env, capture_output=True, text=True, timeout=900)
+    assert r.returncode == 0, r.stdout[-3000:] + r.stderr[-2000:]
