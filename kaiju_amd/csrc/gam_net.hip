@@ -62,59 +62,152 @@ __device__ __forceinline__ bf16x8 ld8(const u16 *p) {   // 16-byte aligned
 }
 
 // ----------------------------------------------------------------- convolution
-// The training convolutions and the inference (k_infer below) work on bricks of
-// NB_I x NB_J x NB_K cells, wave w of a block on the brick's k row w: NB_J tiles of 16
-// cells (one per j row).
+// The training convolutions (k_conv) and the inference (k_infer below) work on bricks of
+// NB_I x NB_J x NB_K cells, tiles of 16 cells along i.  A brick's input, the brick and
+// one cell around it, is staged once in LDS (80 bytes per cell of 32 channels: the
+// lanes of a 16-byte read fall on distinct banks), so an input cell comes from L2 2.5
+// times instead of once per tap.
+// CIN = 8: a wave has the tiles of one k row and all output channels, and packs 4 taps
+// per K step (lane group kg reading tap 4s + kg).
+// CIN = 32, one tap per K step: a wave has one 16-channel output tile on NCO / 16 k rows, so
+// its weights of all 27 taps fit its registers (108), and blocks stay
+// for several bricks, the next one's input on its way to registers meanwhile.  Fetched per
+// brick, the 55 KB of weights passed the 32 KB L1 for every 64 cells, and the MFMAs
+// waited for them.  The tile rows of a staged plane are each read once for
+// the up to 3 x NCO / 16 output rows that they feed.
+// The taps add in the order dx, dy, dz in either form.
 #define NB_I 16
-#ifndef NB_J
 #define NB_J 4
-#endif
 #define NB_K 4
 #define NB_LI (NB_I + 2)
 #define NB_LJ (NB_J + 2)
 #define NB_LK (NB_K + 2)
 #define NB_LC (NB_LI * NB_LJ * NB_LK)   // staged cells
 #define NB_OC (NB_I * NB_J * NB_K)      // output cells
+#define NB_STAY 512   // blocks of the 32-channel kernels: 2 on each of 256 CUs
+
+template <int CIN, int NCO>
+struct ConvT {
+    static constexpr int CS = CIN == 32 ? 40 : 8;           // BF16 elements per staged cell
+    static constexpr int OS = 40;                           // and per output cell of 32 channels: 80 bytes
+    static constexpr int TW = CIN == 32 ? 1 : NCO / 16;     // output tiles per wave
+    static constexpr int KT = CIN == 32 ? NCO / 16 : 1;     // k rows per wave
+    static constexpr int NS = CIN == 32 ? NET_TAPS : (NET_TAPS + 3) / 4;   // K steps
+    bf16x8 w[CIN == 32 ? NS : 2][TW];   // CIN = 8: two K steps ahead
+    f32x4 acc[KT][NB_J][TW];
+    const u16 *W;
+    int row, kg, t0, kr;   // lane's row and K group; the wave's first output tile and k row
+    __device__ __forceinline__ bf16x8 weight(int q, int t) const {
+        return ld8(W + (size_t)(q * NCO + 16 * (t0 + t) + row) * NET_C + 8 * kg);
+    }
+    __device__ __forceinline__ void init(const u16 *W_) {
+        const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+        W = W_;
+        row = lane & 15; kg = lane >> 4;
+        t0 = CIN == 32 ? wave % (NCO / 16) : 0;
+        kr = CIN == 32 ? wave / (NCO / 16) * KT : wave;
+#pragma unroll
+        for (int q = 0; q < (CIN == 32 ? NS : 2); q++)
+#pragma unroll
+            for (int t = 0; t < TW; t++) w[q][t] = weight(q, t);
+    }
+    __device__ __forceinline__ void run(const u16 *sA) {
+#pragma unroll
+        for (int q = 0; q < KT * NB_J * TW; q++) acc[q / (NB_J * TW)][(q / TW) % NB_J][q % TW] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if constexpr (CIN == 8) {
+#pragma unroll 1
+            for (int st = 0; st < NS; st++) {
+                const int tap = 4 * st + kg;
+                const bool live = tap < NET_TAPS;   // K slots past the last tap: zero A (their weights are zero too)
+                const int tp = live ? tap : 13;     // a staged cell for the dead slots
+                const int c0 = (kr + tp / 9) * (NB_LJ * NB_LI) + ((tp / 3) % 3) * NB_LI + tp % 3 + row;
+                bf16x8 bw[TW];
+                const int sn = st + 2 < NS ? st + 2 : NS - 1;
+#pragma unroll
+                for (int t = 0; t < TW; t++) { bw[t] = w[0][t]; w[0][t] = w[1][t]; w[1][t] = weight(sn, t); }
+#pragma unroll
+                for (int m = 0; m < NB_J; m++) {
+                    bf16x8 a = *reinterpret_cast<const bf16x8 *>(sA + (size_t)(c0 + m * NB_LI) * CS);
+                    if (!live) a = bf16x8{};
+#pragma unroll
+                    for (int t = 0; t < TW; t++) acc[0][m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bw[t], acc[0][m][t], 0, 0, 0);
+                }
+            }
+        } else {
+            // the staged tile rows (plane pl, row r) in turn, each read one row ahead; row r of
+            // plane pl is the tap (dy, dz) = (r - m, pl - kt) - 1 of output row m, k row kt
+            const u16 *s0 = sA + (size_t)(kr * (NB_LJ * NB_LI) + row) * CS + 8 * kg;
+            bf16x8 a[2][3];
+            auto rd = [&](int n) {
+#pragma unroll
+                for (int dx = 0; dx < 3; dx++) a[n & 1][dx] = *reinterpret_cast<const bf16x8 *>(s0 + (n * NB_LI + dx) * CS);
+            };
+            rd(0);
+#pragma unroll
+            for (int n = 0; n < (KT + 2) * NB_LJ; n++) {
+                if (n + 1 < (KT + 2) * NB_LJ) rd(n + 1);
+                const int pl = n / NB_LJ, r = n % NB_LJ;
+#pragma unroll
+                for (int kt = 0; kt < KT; kt++)
+#pragma unroll
+                    for (int m = 0; m < NB_J; m++) {
+                        if (pl - kt < 0 || pl - kt > 2 || r - m < 0 || r - m > 2) continue;
+#pragma unroll
+                        for (int dx = 0; dx < 3; dx++)
+                            acc[kt][m][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[n & 1][dx], w[9 * (pl - kt) + 3 * (r - m) + dx][0],
+                                                                                    acc[kt][m][0], 0, 0, 0);
+                    }
+                __builtin_amdgcn_sched_barrier(0);   // no reads hoisted further: registers
+            }
+        }
+    }
+};
+
+// Bricks of a block: the launch's bricks in 8 runs, one per XCD, whose L2 then holds
+// the neighbours' shared cells.
+__device__ __forceinline__ int brick_run(int nbrick) { return (nbrick + 7) / 8; }
+static unsigned brick_blocks(int cin, long nbrick) {
+    const long all = (nbrick + 7) / 8 * 8;
+    return (unsigned)(cin == 32 ? std::min<long>(NB_STAY, all) : all);
+}
+
+struct alignas(2) u16x4u { u16 v[4]; };   // 4 cells of a channel, at element alignment
 
 // Hidden activation: leaky ReLU, x > 0 ? x : x/8 (a slope that keeps every
 // unit trainable; 1/8 is exact in BF16 and FP32).
 // MODE 0: activation, write act_out (channels last) and actT_out (channel-major), NCO = 32
 // MODE 1: linear output, write out[p][0..7] FP32 (NCO = 16, channels 8..15 padding)
 // MODE 2: backward data: multiply by the activation's slope at the forward
-//         output (mask act > 0: 1, else 1/8), write both BF16 layouts, NCO = 32
-// CIN = 32, or 8 for the first layer, which packs 4 taps per K step (lane group kg
-// reading tap 4s + kg).
-// A brick's input, the brick and one cell around it, is staged once in LDS (80 bytes per
-// cell of 32 channels: the lanes of a 16-byte read fall on distinct banks), so an input
-// cell comes from L2 2.5 times instead of once per tap.  Neighbours are
-// those of the flattened cell index (p + off), as at the box faces, whose cells
-// are never used; cells outside [lo, lo + 16 ntile) are not stored.  The results
-// leave through LDS, as whole cells and as rows of 16 cells per channel.  Per
-// launch on a 104^3 grid, A operands from L2 before: hidden layer 230 -> 151 us, first
-// 111 -> 84, last 182 -> 70, backward data 272 -> 192.
+//         output (maskT, channel-major, > 0: 1, else 1/8), write both BF16 layouts, NCO = 32
+// Neighbours are those of the flattened cell index (p + off), as at the box faces, whose
+// cells are never used; cells outside [lo, lo + 16 ntile) are not stored.  A lane holds
+// 4 cells of a channel, which go to the channel-major array as they are; whole cells
+// leave through LDS.
+// Per launch on a 104^3 grid, A operands from L2 / staged, weights per brick / as now:
+// hidden layer 230 / 151 / 94 us, first 111 / 84 / 62, last 182 / 70 / 43, backward
+// data 272 / 192 / 131.
 template <int CIN, int NCO, int MODE>
-__global__ void __launch_bounds__(256) k_conv(NetDims d, const u16 *__restrict__ in, const u16 *__restrict__ W,
-                                              const float *__restrict__ bias, const u16 *__restrict__ mask,
-                                              u16 *__restrict__ act_out, u16 *__restrict__ actT_out,
-                                              float *__restrict__ out) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CIN == 32 ? 2 : 4)))
+k_conv(NetDims d, const u16 *__restrict__ in, const u16 *__restrict__ W, const float *__restrict__ bias,
+       const u16 *__restrict__ maskT, u16 *__restrict__ act_out, u16 *__restrict__ actT_out, float *__restrict__ out) {
     static_assert(CIN == 8 || CIN == 32, "8 or 32 input channels");
-    static_assert(NB_I == 16 && NB_K == 4, "one 16-cell tile per row, one k row per wave");
-    constexpr int TPK = CIN == 8 ? 4 : 1;
-    constexpr int NSTEP = (NET_TAPS + TPK - 1) / TPK;
-    constexpr int CS = CIN == 32 ? 40 : 8;                // BF16 elements per staged cell
-    constexpr int OS = 40;                                // and per output cell: 80 bytes
-    constexpr int FS = 36;                                // FP32 elements per output cell (MODE 2)
-    constexpr int OUTB = MODE == 1 ? NB_OC * 32 : NB_OC * OS * 2 + (MODE == 2 ? NB_OC * FS * 4 : 0);
-    constexpr int SB = NB_LC * CS * 2 > OUTB ? NB_LC * CS * 2 : OUTB;
-    __shared__ uint4 smem[SB / 16];
-    u16 *sA = reinterpret_cast<u16 *>(smem);
-    const int nbi = (d.Ni + NB_I - 1) / NB_I, nbj = (d.Nj + NB_J - 1) / NB_J;
-    const int b = blockIdx.x;
-    const int oi = NB_I * (b % nbi), oj = NB_J * ((b / nbi) % nbj), ok = NB_K * (b / (nbi * nbj));   // brick origin
-    {
-        constexpr int PER = CIN / 8;                      // 16-byte pieces per cell
-        constexpr int NIT = (NB_LC * PER + 255) / 256;
-        uint4 v[NIT];
+    static_assert(NB_I == 16 && NB_K == 4, "one 16-cell tile per row, four waves on four k rows");
+    using T = ConvT<CIN, NCO>;
+    constexpr int CS = T::CS, OS = T::OS, PER = CIN / 8;   // PER: 16-byte pieces per cell
+    constexpr int NIT = (NB_LC * PER + 255) / 256;
+    __shared__ uint4 sIn[NB_LC * CS / 8];
+    __shared__ uint4 sOut[MODE == 1 ? NB_OC * 2 : NB_OC * OS / 8];
+    u16 *sO = reinterpret_cast<u16 *>(sOut);
+    float *sF = reinterpret_cast<float *>(sOut);
+    const int nbi = (d.Ni + NB_I - 1) / NB_I, nbj = (d.Nj + NB_J - 1) / NB_J, nbk = (d.Nk + NB_K - 1) / NB_K;
+    const int run = brick_run(nbi * nbj * nbk), hi = d.lo + 16 * d.ntile;
+    const int b0 = (blockIdx.x & 7) * run, b1 = min(b0 + run, nbi * nbj * nbk), step = gridDim.x >> 3;
+    int b = b0 + (blockIdx.x >> 3);
+    auto origin = [&](int bb, int &oi, int &oj, int &ok) { oi = NB_I * (bb % nbi); oj = NB_J * ((bb / nbi) % nbj); ok = NB_K * (bb / (nbi * nbj)); };
+    uint4 v[NIT];
+    auto fetch = [&](int bb) {
+        int oi, oj, ok;
+        origin(bb, oi, oj, ok);
 #pragma unroll
         for (int it = 0; it < NIT; it++) {
             const int e = threadIdx.x + 256 * it, c = e / PER;
@@ -123,110 +216,70 @@ __global__ void __launch_bounds__(256) k_conv(NetDims d, const u16 *__restrict__
             v[it] = uint4{0u, 0u, 0u, 0u};
             if (c < NB_LC && p >= 0 && p < d.nc) v[it] = *reinterpret_cast<const uint4 *>(in + (size_t)p * NET_C + 8 * (e % PER));
         }
+    };
+    if (b >= b1) return;
+    fetch(b);
+    T cv;
+    cv.init(W);
+    for (; b < b1; b += step) {
 #pragma unroll
         for (int it = 0; it < NIT; it++) {
             const int e = threadIdx.x + 256 * it, c = e / PER;
-            if (c < NB_LC) smem[c * (CS / 8) + e % PER] = v[it];
+            if (c < NB_LC) sIn[c * (CS / 8) + e % PER] = v[it];
         }
-    }
-    __syncthreads();
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, row = lane & 15, kg = lane >> 4;
-    f32x4 acc[NB_J][NCO / 16];
+        __syncthreads();   // staged; and every wave has read the last brick's sOut
+        if (CIN == 32 && b + step < b1) fetch(b + step);
+        cv.run(reinterpret_cast<const u16 *>(sIn));
+        int oi, oj, ok;
+        origin(b, oi, oj, ok);
 #pragma unroll
-    for (int m = 0; m < NB_J; m++)
+        for (int q = 0; q < T::KT * NB_J * T::TW; q++) {
+            const int kt = q / (NB_J * T::TW), m = (q / T::TW) % NB_J, t = q % T::TW;
+            const int co = 16 * (cv.t0 + t) + cv.row, kk = cv.kr + kt, oc = (kk * NB_J + m) * NB_I + 4 * cv.kg;
+            const f32x4 x = cv.acc[kt][m][t];
+            if constexpr (MODE == 1) {
+                if (co < 8) {
+                    const float bb = bias[co];
 #pragma unroll
-        for (int t = 0; t < NCO / 16; t++) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // the K steps' weights (the same for every block, from L2) two steps ahead of their MFMAs
-    const u16 *wl = W + ((size_t)row) * NET_C + 8 * kg;
-    bf16x8 wn[2][NCO / 16];
-#pragma unroll
-    for (int q = 0; q < 2; q++)
-#pragma unroll
-        for (int t = 0; t < NCO / 16; t++) wn[q][t] = ld8(wl + ((size_t)q * NCO + 16 * t) * NET_C);
-    for (int st = 0; st < NSTEP; st++) {
-        const int tap = TPK == 1 ? st : TPK * st + kg;
-        const bool live = TPK == 1 || tap < NET_TAPS;   // K slots past the last tap: weights are zero there too
-        const int tp = live ? tap : 13;
-        bf16x8 bw[NCO / 16];
-        const int sn = st + 2 < NSTEP ? st + 2 : NSTEP - 1;
-#pragma unroll
-        for (int t = 0; t < NCO / 16; t++) {
-            bw[t] = wn[0][t];
-            wn[0][t] = wn[1][t];
-            wn[1][t] = ld8(wl + ((size_t)sn * NCO + 16 * t) * NET_C);
-        }
-        const int dx = tp % 3 - 1, dy = (tp / 3) % 3 - 1, dz = tp / 9 - 1;
-        const int c0 = (wave + 1 + dz) * (NB_LJ * NB_LI) + (1 + dy) * NB_LI + 1 + dx + row;
-#pragma unroll
-        for (int m = 0; m < NB_J; m++) {
-            bf16x8 a = *reinterpret_cast<const bf16x8 *>(sA + (size_t)(c0 + m * NB_LI) * CS + (TPK == 1 ? 8 * kg : 0));
-            if (!live) a = bf16x8{};
-#pragma unroll
-            for (int t = 0; t < NCO / 16; t++) acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bw[t], acc[m][t], 0, 0, 0);
-        }
-    }
-    __syncthreads();   // every wave is done with the staged input: the LDS takes the outputs
-    float *sF = reinterpret_cast<float *>(reinterpret_cast<char *>(smem) + (MODE == 2 ? NB_OC * OS * 2 : 0));
-    // D layout: lane holds cells 4*kg + r of the tile, channel 16*t + row
-#pragma unroll
-    for (int m = 0; m < NB_J; m++)
-#pragma unroll
-        for (int t = 0; t < NCO / 16; t++) {
-            const int co = 16 * t + row;
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int oc = (wave * NB_J + m) * NB_I + 4 * kg + r;
-                const float v = acc[m][t][r];
-                if (MODE == 0) {
-                    const float x = v + bias[co];
-                    sA[oc * OS + co] = f2bf(x > 0.f ? x : NET_LEAK * x);
-                } else if (MODE == 1) {
-                    if (co < 8) sF[oc * 8 + co] = v + bias[co];
-                } else {
-                    sF[oc * FS + co] = v;
+                    for (int r = 0; r < 4; r++) sF[(oc + r) * 8 + co] = x[r] + bb;
                 }
-            }
-        }
-    __syncthreads();
-    const int hi = d.lo + 16 * d.ntile;
-    auto cell = [&](int oc, int &p) {   // flattened index of output cell oc; false: not stored
-        const int i = oi + oc % NB_I, j = oj + (oc / NB_I) % NB_J, k = ok + oc / (NB_I * NB_J);
-        p = i + d.Ni * (j + d.Nj * k);
-        return i < d.Ni && j < d.Nj && k < d.Nk && p >= d.lo && p < hi;
-    };
-    if (MODE == 1) {
-        for (int e = threadIdx.x; e < NB_OC * 2; e += 256) {
-            int p;
-            if (cell(e >> 1, p)) *reinterpret_cast<uint4 *>(out + (size_t)p * 8 + 4 * (e & 1)) = smem[e];
-        }
-        return;
-    }
-    for (int e = threadIdx.x; e < NB_OC * 4; e += 256) {   // whole cells, 8 channels a thread
-        const int oc = e >> 2, q = e & 3;
-        int p;
-        const bool st = cell(oc, p);
-        uint4 *cellp = smem + oc * (OS / 8) + q;
-        if (MODE == 2) {
-            uint4 mk = {0u, 0u, 0u, 0u};
-            if (st) mk = *reinterpret_cast<const uint4 *>(mask + (size_t)p * NET_C + 8 * q);
-            const uint32_t mw[4] = {mk.x, mk.y, mk.z, mk.w};
-            uint32_t o[4];
+            } else {
+                const int i = oi + 4 * cv.kg, p = i + d.Ni * ((oj + m) + d.Nj * (ok + kk));
+                const bool rowin = oj + m < d.Nj && ok + kk < d.Nk;
+                const bool full = rowin && i + 3 < d.Ni && p >= d.lo && p + 3 < hi;
+                auto in1 = [&](int r) { return rowin && i + r < d.Ni && p + r >= d.lo && p + r < hi; };
+                const size_t pt = (size_t)co * d.ncs + p;
+                u16x4u h, mk;
+                if constexpr (MODE == 2) {
+                    if (full) mk = *reinterpret_cast<const u16x4u *>(maskT + pt);
+                    else
 #pragma unroll
-            for (int h = 0; h < 4; h++) {
-                float x = sF[oc * FS + 8 * q + 2 * h], y = sF[oc * FS + 8 * q + 2 * h + 1];
-                if (bf2f((u16)(mw[h] & 0xFFFFu)) <= 0.f) x = NET_LEAK * x;   // slope at the forward output
-                if (bf2f((u16)(mw[h] >> 16)) <= 0.f) y = NET_LEAK * y;
-                o[h] = (uint32_t)f2bf(x) | ((uint32_t)f2bf(y) << 16);
+                        for (int r = 0; r < 4; r++) mk.v[r] = in1(r) ? maskT[pt + r] : 0;
+                }
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    float y = x[r];
+                    if constexpr (MODE == 0) { y += bias[co]; y = y > 0.f ? y : NET_LEAK * y; }
+                    else if (bf2f(mk.v[r]) <= 0.f) y = NET_LEAK * y;   // slope at the forward output
+                    h.v[r] = f2bf(y);
+                    sO[(oc + r) * OS + co] = h.v[r];
+                }
+                if (full) *reinterpret_cast<u16x4u *>(actT_out + pt) = h;
+                else
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        if (in1(r)) actT_out[pt + r] = h.v[r];
             }
-            *cellp = uint4{o[0], o[1], o[2], o[3]};
         }
-        if (st) *reinterpret_cast<uint4 *>(act_out + (size_t)p * NET_C + 8 * q) = *cellp;
-    }
-    if (MODE == 2) __syncthreads();
-    for (int e = threadIdx.x; e < NB_OC * NET_C; e += 256) {   // rows of 16 cells per channel
-        const int oc = (e / (NB_I * NET_C)) * NB_I + e % NB_I, co = (e / NB_I) % NET_C;
-        int p;
-        if (cell(oc, p)) actT_out[(size_t)co * d.ncs + p] = sA[oc * OS + co];
+        __syncthreads();   // results in sOut; and every wave is done with sIn
+        constexpr int CH = MODE == 1 ? 2 : 4;   // 16-byte pieces per output cell
+        for (int e = threadIdx.x; e < NB_OC * CH; e += 256) {
+            const int oc = e / CH, q = e % CH;
+            const int i = oi + oc % NB_I, j = oj + (oc / NB_I) % NB_J, k = ok + oc / (NB_I * NB_J), p = i + d.Ni * (j + d.Nj * k);
+            if (i >= d.Ni || j >= d.Nj || k >= d.Nk || p < d.lo || p >= hi) continue;
+            if constexpr (MODE == 1) *reinterpret_cast<uint4 *>(out + (size_t)p * 8 + 4 * q) = sOut[e];
+            else *reinterpret_cast<uint4 *>(act_out + (size_t)p * NET_C + 8 * q) = sOut[oc * (OS / 8) + q];
+        }
     }
 }
 
@@ -441,154 +494,112 @@ __global__ void __launch_bounds__(256) k_features(int nc, int ncs, const R *__re
 }
 
 // ----------------------------------------------------------------- inference
-// One layer over a brick of NB_I x NB_J x NB_K output cells with its input (the
-// brick and one cell around it) staged once in LDS: every input cell comes from
-// L2/HBM about 2.5 times instead of once per tap, and the MFMA A operands are
-// LDS reads.  The layer's outputs are stored on a box [lo, lo + n) per axis only
-// (the last layer's box is the cells at least `halo` from the grid faces, each
-// earlier layer's box one cell wider on every side, so every stored output reads
-// stored inputs); staged cells off the grid are zeros and feed only outputs
-// that are not stored.  The first layer (CIN = 8) computes the features of its
-// staged cells from Gas and B itself (features_of, as k_features).  Per output
-// cell the operands, their K order, the bias and the activation are k_conv's,
-// so the stored values equal gam_net_forward's bit for bit.
-// Wave w of the block computes the brick's k row w: NB_J tiles of 16 cells (one
-// per j row).  The results go through LDS to leave as whole cells (64 bytes of
-// BF16 activations, or 32 bytes of FP32 output).
+// One layer on bricks, as k_conv, but the layer's outputs are stored on a box
+// [lo, lo + n) per axis only (the last layer's box is the cells at least `halo` from
+// the grid faces, each earlier layer's box one cell wider on every side, so every
+// stored output reads stored inputs); staged cells off the grid are zeros and feed
+// only outputs that are not stored.  The first layer (CIN = 8) computes the
+// features of its staged cells from Gas and B itself (as k_features).  Per
+// output cell the operands, their K order, the bias and the activation are
+// k_conv's, so the stored values equal gam_net_forward's bit for bit.
+// The last layer alone on 134^3 cells: 103 us with weights fetched per brick -> 78.
 struct InferBox { int lo[3], n[3], nb[3]; };
 
 template <int CIN, int NCO, int MODE, typename R>
-__global__ void __launch_bounds__(256) k_infer(NetDims d, InferBox bx, const u16 *__restrict__ in, const R *__restrict__ Gas,
-                                               const R *__restrict__ Bc, float gamma, float4 sc, float2 offs,
-                                               const u16 *__restrict__ W, const float *__restrict__ bias,
-                                               u16 *__restrict__ act_out, float *__restrict__ out) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CIN == 32 ? 2 : 4)))
+k_infer(NetDims d, InferBox bx, const u16 *__restrict__ in, const R *__restrict__ Gas, const R *__restrict__ Bc, float gamma,
+        float4 sc, float2 offs, const u16 *__restrict__ W, const float *__restrict__ bias, u16 *__restrict__ act_out,
+        float *__restrict__ out) {
     static_assert(CIN == 8 || CIN == 32, "8 or 32 input channels");
-    static_assert(NB_I == 16 && NB_K == 4, "one 16-cell tile per row, one k row per wave");
-    constexpr int TPK = CIN == 8 ? 4 : 1;
-    constexpr int NSTEP = (NET_TAPS + TPK - 1) / TPK;
-    constexpr int OB = MODE == 0 ? 64 : 32;                          // bytes per output cell
-    // a staged cell of 32 channels takes 80 bytes: consecutive cells of an A
-    // operand then start 5 x 16 bytes apart, so the lanes of a 16-byte LDS read
-    // fall on distinct banks (64 bytes apart, every fourth lane would share them)
-    constexpr int CS = CIN == 32 ? 40 : 8;                           // BF16 elements per staged cell
-    constexpr int SB = NB_LC * CS * 2 > NB_OC * OB ? NB_LC * CS * 2 : NB_OC * OB;
-    __shared__ uint4 smem[SB / 16];
-    u16 *sA = reinterpret_cast<u16 *>(smem);
-    const int b = blockIdx.x;
-    const int bi = b % bx.nb[0], bj = (b / bx.nb[0]) % bx.nb[1], bk = b / (bx.nb[0] * bx.nb[1]);
-    const int oi = bx.lo[0] + NB_I * bi, oj = bx.lo[1] + NB_J * bj, ok = bx.lo[2] + NB_K * bk;   // brick origin
-    const size_t nc = d.nc;
-    // stage the input: cell c of the staged box is (oi - 1, oj - 1, ok - 1) + (li, lj, lk).
-    // Every load of the thread is issued before the first LDS store.
-    auto cell_at = [&](int c, size_t &p) -> bool {
-        const int li = c % NB_LI, lj = (c / NB_LI) % NB_LJ, lk = c / (NB_LI * NB_LJ);
-        const int i = oi - 1 + li, j = oj - 1 + lj, k = ok - 1 + lk;
+    using T = ConvT<CIN, NCO>;
+    constexpr int CS = T::CS, OS = T::OS, PER = CIN == 8 ? 1 : 4;
+    constexpr int NIT = (NB_LC * PER + 255) / 256;
+    __shared__ uint4 sIn[NB_LC * CS / 8];
+    __shared__ uint4 sOut[MODE == 1 ? NB_OC * 2 : NB_OC * OS / 8];
+    u16 *sO = reinterpret_cast<u16 *>(sOut);
+    float *sF = reinterpret_cast<float *>(sOut);
+    const int nbrick = bx.nb[0] * bx.nb[1] * bx.nb[2], run = brick_run(nbrick);
+    const int b0 = (blockIdx.x & 7) * run, b1 = min(b0 + run, nbrick), step = gridDim.x >> 3;
+    int b = b0 + (blockIdx.x >> 3);
+    auto origin = [&](int bb, int &oi, int &oj, int &ok) {   // cell of the brick's box
+        oi = NB_I * (bb % bx.nb[0]); oj = NB_J * ((bb / bx.nb[0]) % bx.nb[1]); ok = NB_K * (bb / (bx.nb[0] * bx.nb[1]));
+    };
+    // staged cell c: (origin - 1) + (li, lj, lk)
+    auto cell_at = [&](int bb, int c, size_t &p) -> bool {
+        int oi, oj, ok;
+        origin(bb, oi, oj, ok);
+        const int i = bx.lo[0] + oi - 1 + c % NB_LI, j = bx.lo[1] + oj - 1 + (c / NB_LI) % NB_LJ, k = bx.lo[2] + ok - 1 + c / (NB_LI * NB_LJ);
         p = (size_t)i + (size_t)d.Ni * ((size_t)j + (size_t)d.Nj * k);
         return i >= 0 && i < d.Ni && j >= 0 && j < d.Nj && k >= 0 && k < d.Nk;
     };
-    if (CIN == 8) {
-        constexpr int NIT = (NB_LC + 255) / 256;
-        float q[NIT][8];
-        bool ok_[NIT];
+    uint4 v[CIN == 32 ? NIT : 1];
+    float q8[CIN == 8 ? NIT : 1][8];
+    bool live[NIT];
+    auto fetch = [&](int bb) {
 #pragma unroll
         for (int it = 0; it < NIT; it++) {
-            const int c = threadIdx.x + 256 * it;
+            const int e = threadIdx.x + 256 * it;
             size_t p = 0;
-            ok_[it] = c < NB_LC && cell_at(c, p);
-            if (ok_[it]) state_of<R>(p, nc, Gas, Bc, q[it]);
-        }
-#pragma unroll
-        for (int it = 0; it < NIT; it++) {
-            const int c = threadIdx.x + 256 * it;
-            if (c >= NB_LC) break;
-            uint4 v = {0u, 0u, 0u, 0u};
-            if (ok_[it]) {
-                float f[8];
-                features_calc(q[it], gamma, sc, offs, f);
-                v = pack8(f);
+            live[it] = e < NB_LC * PER && cell_at(bb, e / PER, p);
+            if constexpr (CIN == 8) {
+                if (live[it]) state_of<R>(p, d.nc, Gas, Bc, q8[it]);
+            } else {
+                v[it] = uint4{0u, 0u, 0u, 0u};
+                if (live[it]) v[it] = *reinterpret_cast<const uint4 *>(in + p * NET_C + 8 * (e % PER));
             }
-            smem[c] = v;
         }
-    } else {
-        constexpr int NIT = (NB_LC * 4 + 255) / 256;   // 4 x 16 bytes per cell, consecutive threads along i
-        uint4 v[NIT];
+    };
+    if (b >= b1) return;
+    fetch(b);
+    T cv;
+    cv.init(W);
+    for (; b < b1; b += step) {
 #pragma unroll
         for (int it = 0; it < NIT; it++) {
             const int e = threadIdx.x + 256 * it;
-            size_t p = 0;
-            v[it] = uint4{0u, 0u, 0u, 0u};
-            if (e < NB_LC * 4 && cell_at(e >> 2, p)) v[it] = *reinterpret_cast<const uint4 *>(in + p * NET_C + 8 * (e & 3));
+            if (e >= NB_LC * PER) break;
+            if constexpr (CIN == 8) {
+                uint4 x = {0u, 0u, 0u, 0u};
+                if (live[it]) {
+                    float f[8];
+                    features_calc(q8[it], gamma, sc, offs, f);
+                    x = pack8(f);
+                }
+                sIn[e] = x;
+            } else {
+                sIn[(e / PER) * (CS / 8) + e % PER] = v[it];
+            }
         }
+        __syncthreads();   // staged; and every wave has read the last brick's sOut
+        if (CIN == 32 && b + step < b1) fetch(b + step);
+        cv.run(reinterpret_cast<const u16 *>(sIn));
 #pragma unroll
-        for (int it = 0; it < NIT; it++) {
-            const int e = threadIdx.x + 256 * it;
-            if (e < NB_LC * 4) smem[(e >> 2) * (CS / 8) + (e & 3)] = v[it];
-        }
-    }
-    __syncthreads();
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, row = lane & 15, kg = lane >> 4;
-    f32x4 acc[NB_J][NCO / 16];
+        for (int q = 0; q < T::KT * NB_J * T::TW; q++) {
+            const int kt = q / (NB_J * T::TW), m = (q / T::TW) % NB_J, t = q % T::TW;
+            const int co = 16 * (cv.t0 + t) + cv.row, oc = ((cv.kr + kt) * NB_J + m) * NB_I + 4 * cv.kg;
+            const f32x4 x = cv.acc[kt][m][t];
+            if (MODE == 0 || co < 8) {
+                const float bb = bias[co];
 #pragma unroll
-    for (int m = 0; m < NB_J; m++)
-#pragma unroll
-        for (int t = 0; t < NCO / 16; t++) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // the K steps' weights (the same for every block, from L2) are loaded two
-    // steps ahead of their MFMAs, so their latency overlaps the two steps before
-    const u16 *wl = W + ((size_t)row) * NET_C + 8 * kg;
-    bf16x8 wn[2][NCO / 16];
-#pragma unroll
-    for (int q = 0; q < 2; q++)
-#pragma unroll
-        for (int t = 0; t < NCO / 16; t++) wn[q][t] = ld8(wl + ((size_t)q * NCO + 16 * t) * NET_C);
-    for (int st = 0; st < NSTEP; st++) {
-        const int tap = TPK == 1 ? st : TPK * st + kg;
-        const bool live = TPK == 1 || tap < NET_TAPS;   // K slots past the last tap: zero A (their weights are zero too)
-        const int tp = live ? tap : 13;                 // a staged cell for the dead slots
-        bf16x8 bw[NCO / 16];
-        const int sn = st + 2 < NSTEP ? st + 2 : NSTEP - 1;   // the step whose weights are fetched now
-#pragma unroll
-        for (int t = 0; t < NCO / 16; t++) {
-            bw[t] = wn[0][t];
-            wn[0][t] = wn[1][t];
-            wn[1][t] = ld8(wl + ((size_t)sn * NCO + 16 * t) * NET_C);
-        }
-        const int dx = tp % 3 - 1, dy = (tp / 3) % 3 - 1, dz = tp / 9 - 1;
-        const int c0 = (wave + 1 + dz) * (NB_LJ * NB_LI) + (1 + dy) * NB_LI + 1 + dx + row;
-#pragma unroll
-        for (int m = 0; m < NB_J; m++) {
-            bf16x8 a = *reinterpret_cast<const bf16x8 *>(sA + (size_t)(c0 + m * NB_LI) * CS + (TPK == 1 ? 8 * kg : 0));
-            if (!live) a = bf16x8{};
-#pragma unroll
-            for (int t = 0; t < NCO / 16; t++) acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bw[t], acc[m][t], 0, 0, 0);
-        }
-    }
-    __syncthreads();   // every wave is done with the staged input: the LDS takes the outputs
-    // D layout: lane holds cells 4*kg + r of the tile, channel 16*t + row
-#pragma unroll
-    for (int m = 0; m < NB_J; m++)
-#pragma unroll
-        for (int t = 0; t < NCO / 16; t++) {
-            const int co = 16 * t + row;
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int oc = (wave * NB_J + m) * NB_I + 4 * kg + r;
-                const float v = acc[m][t][r] + bias[co < (MODE == 0 ? NCO : 8) ? co : 0];
-                if (MODE == 0) {
-                    sA[oc * NET_C + co] = f2bf(v > 0.f ? v : NET_LEAK * v);
-                } else if (co < 8) {
-                    reinterpret_cast<float *>(smem)[oc * 8 + co] = v;
+                for (int r = 0; r < 4; r++) {
+                    const float y = x[r] + bb;
+                    if constexpr (MODE == 0) sO[(oc + r) * OS + co] = f2bf(y > 0.f ? y : NET_LEAK * y);
+                    else sF[(oc + r) * 8 + co] = y;
                 }
             }
         }
-    __syncthreads();
-    constexpr int CH = OB / 16;   // 16-byte chunks per output cell
-    for (int e = threadIdx.x; e < NB_OC * CH; e += 256) {
-        const int oc = e / CH, part = e % CH;
-        const int ii = oc % NB_I, jj = (oc / NB_I) % NB_J, kk = oc / (NB_I * NB_J);
-        if (NB_I * bi + ii >= bx.n[0] || NB_J * bj + jj >= bx.n[1] || NB_K * bk + kk >= bx.n[2]) continue;
-        const size_t p = (size_t)(oi + ii) + (size_t)d.Ni * ((size_t)(oj + jj) + (size_t)d.Nj * (ok + kk));
-        if (MODE == 0) *reinterpret_cast<uint4 *>(act_out + p * NET_C + 8 * part) = smem[e];
-        else *reinterpret_cast<uint4 *>(out + p * 8 + 4 * part) = smem[e];
+        __syncthreads();   // results in sOut; and every wave is done with sIn
+        int oi, oj, ok;
+        origin(b, oi, oj, ok);
+        constexpr int CH = MODE == 1 ? 2 : 4;   // 16-byte pieces per output cell
+        for (int e = threadIdx.x; e < NB_OC * CH; e += 256) {
+            const int oc = e / CH, part = e % CH;
+            const int ii = oi + oc % NB_I, jj = oj + (oc / NB_I) % NB_J, kk = ok + oc / (NB_I * NB_J);
+            if (ii >= bx.n[0] || jj >= bx.n[1] || kk >= bx.n[2]) continue;
+            const size_t p = (size_t)(bx.lo[0] + ii) + (size_t)d.Ni * ((size_t)(bx.lo[1] + jj) + (size_t)d.Nj * (bx.lo[2] + kk));
+            if constexpr (MODE == 0) *reinterpret_cast<uint4 *>(act_out + p * NET_C + 8 * part) = sOut[oc * (OS / 8) + part];
+            else *reinterpret_cast<uint4 *>(out + p * 8 + 4 * part) = sOut[e];
+        }
     }
 }
 
@@ -807,19 +818,19 @@ extern "C" int gam_net_set_features(gam_net *n, const float *feat) {
     return 0;
 }
 
-static dim3 conv_grid(const gam_net *n) {
+static dim3 conv_grid(const gam_net *n, int cin) {
     const NetDims &d = n->d;
-    return dim3((unsigned)(((d.Ni + NB_I - 1) / NB_I) * ((d.Nj + NB_J - 1) / NB_J) * ((d.Nk + NB_K - 1) / NB_K)));
+    return dim3(brick_blocks(cin, (long)((d.Ni + NB_I - 1) / NB_I) * ((d.Nj + NB_J - 1) / NB_J) * ((d.Nk + NB_K - 1) / NB_K)));
 }
 
 extern "C" int gam_net_forward(gam_net *n) {
     if (!n) return -1;
     const NetDims &d = n->d;
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_conv<8, 32, 0>), conv_grid(n), 256, 0, n->stream, d, (const u16 *)n->act[0], (const u16 *)n->Wf[0],
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_conv<8, 32, 0>), conv_grid(n, 8), 256, 0, n->stream, d, (const u16 *)n->act[0], (const u16 *)n->Wf[0],
                        (const float *)(n->w + boff(0)), (const u16 *)nullptr, n->act[1], n->actT[1], (float *)nullptr);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_conv<32, 32, 0>), conv_grid(n), 256, 0, n->stream, d, (const u16 *)n->act[1], (const u16 *)n->Wf[1],
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_conv<32, 32, 0>), conv_grid(n, 32), 256, 0, n->stream, d, (const u16 *)n->act[1], (const u16 *)n->Wf[1],
                        (const float *)(n->w + boff(1)), (const u16 *)nullptr, n->act[2], n->actT[2], (float *)nullptr);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_conv<32, 16, 1>), conv_grid(n), 256, 0, n->stream, d, (const u16 *)n->act[2], (const u16 *)n->Wf[2],
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_conv<32, 16, 1>), conv_grid(n, 32), 256, 0, n->stream, d, (const u16 *)n->act[2], (const u16 *)n->Wf[2],
                        (const float *)(n->w + boff(2)), (const u16 *)nullptr, (u16 *)nullptr, (u16 *)nullptr, n->out);
     NCHK(n, hipGetLastError());
     return 0;
@@ -842,19 +853,19 @@ extern "C" int gam_net_infer(gam_net *n, const void *Gas, const void *B, int pre
             bx[l].nb[a] = (bx[l].n[a] + nb[a] - 1) / nb[a];
         }
     }
-    auto grid = [](const InferBox &b) { return dim3((unsigned)(b.nb[0] * b.nb[1] * b.nb[2])); };
+    auto grid = [](int cin, const InferBox &b) { return dim3(brick_blocks(cin, (long)b.nb[0] * b.nb[1] * b.nb[2])); };
     if (precision)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_infer<8, 32, 0, float>), grid(bx[0]), 256, 0, n->stream, d, bx[0], (const u16 *)nullptr,
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_infer<8, 32, 0, float>), grid(8, bx[0]), 256, 0, n->stream, d, bx[0], (const u16 *)nullptr,
                            (const float *)Gas, (const float *)B, n->gamma, n->scales, n->offs, (const u16 *)n->Wf[0],
                            (const float *)(n->w + boff(0)), n->act[1], (float *)nullptr);
     else
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_infer<8, 32, 0, double>), grid(bx[0]), 256, 0, n->stream, d, bx[0], (const u16 *)nullptr,
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_infer<8, 32, 0, double>), grid(8, bx[0]), 256, 0, n->stream, d, bx[0], (const u16 *)nullptr,
                            (const double *)Gas, (const double *)B, n->gamma, n->scales, n->offs, (const u16 *)n->Wf[0],
                            (const float *)(n->w + boff(0)), n->act[1], (float *)nullptr);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_infer<32, 32, 0, float>), grid(bx[1]), 256, 0, n->stream, d, bx[1], (const u16 *)n->act[1],
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_infer<32, 32, 0, float>), grid(32, bx[1]), 256, 0, n->stream, d, bx[1], (const u16 *)n->act[1],
                        (const float *)nullptr, (const float *)nullptr, n->gamma, n->scales, n->offs, (const u16 *)n->Wf[1],
                        (const float *)(n->w + boff(1)), n->act[2], (float *)nullptr);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_infer<32, 16, 1, float>), grid(bx[2]), 256, 0, n->stream, d, bx[2], (const u16 *)n->act[2],
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_infer<32, 16, 1, float>), grid(32, bx[2]), 256, 0, n->stream, d, bx[2], (const u16 *)n->act[2],
                        (const float *)nullptr, (const float *)nullptr, n->gamma, n->scales, n->offs, (const u16 *)n->Wf[2],
                        (const float *)(n->w + boff(2)), (u16 *)nullptr, n->out);
     NCHK(n, hipGetLastError());
@@ -883,12 +894,12 @@ extern "C" int gam_net_backward(gam_net *n, const float *dout) {
     hipLaunchKernelGGL(k_dout, dim3((d.nc + 255) / 256), 256, 0, n->stream, d, dout, n->gr[0], n->grT[0]);
     // layer 2 (linear, 8 outputs padded to 16)
     wgrad(one, two, n->grT[0], n->actT[2], 2);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_conv<32, 32, 2>), conv_grid(n), 256, 0, n->stream, d, (const u16 *)n->gr[0], (const u16 *)n->Wb[2],
-                       (const float *)nullptr, (const u16 *)n->act[2], n->gr[1], n->grT[1], (float *)nullptr);
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_conv<32, 32, 2>), conv_grid(n, 32), 256, 0, n->stream, d, (const u16 *)n->gr[0], (const u16 *)n->Wb[2],
+                       (const float *)nullptr, (const u16 *)n->actT[2], n->gr[1], n->grT[1], (float *)nullptr);
     // layer 1
     wgrad(two, two, n->grT[1], n->actT[1], 1);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_conv<32, 32, 2>), conv_grid(n), 256, 0, n->stream, d, (const u16 *)n->gr[1], (const u16 *)n->Wb[1],
-                       (const float *)nullptr, (const u16 *)n->act[1], n->gr[0], n->grT[0], (float *)nullptr);
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_conv<32, 32, 2>), conv_grid(n, 32), 256, 0, n->stream, d, (const u16 *)n->gr[1], (const u16 *)n->Wb[1],
+                       (const float *)nullptr, (const u16 *)n->actT[1], n->gr[0], n->grT[0], (float *)nullptr);
     // layer 0 (input gradient not needed)
     wgrad(two, one, n->grT[0], n->actT[0], 0);
     NCHK(n, hipGetLastError());
