@@ -5,10 +5,7 @@
 // hand-written here; libgamera_net.so exports them (include/gamera_net.h).
 //
 // Layouts (nc = cells of the ghost-inclusive box, p = linear cell index, i fastest):
-//   activations  act[p][32]   BF16, channels last (A operand of the convolutions)
-//                actT[c][p]   BF16, channel-major copy (operand of the weight gradients),
-//                             rows of ncs >= nc elements (a multiple of 8, with a gap),
-//                             NET_PAD elements of zeros before row 0 and after row 31
+//   activations  act[p][32]   BF16, channels last
 //   weights      W[l][tap][co][ci] BF16 (ci = 32 padded), tap = dz*9 + dy*3 + dx;
 //                the first layer (8 input channels) packs 4 taps per K = 32:
 //                W0[g][co][4*8] with taps 4g..4g+3 (zero past tap 26)
@@ -38,7 +35,6 @@ typedef unsigned short u16;
 #define NET_C 32      // padded channel count of every activation
 #define NET_TAPS 27
 #define NET_G0 7      // K steps of the first layer: ceil(27 taps / 4)
-#define NET_PAD 64    // zero elements before and after a channel-major array
 #define NET_LEAK 0.125f
 
 // round-to-nearest-even FP32 -> BF16 (finite inputs)
@@ -55,7 +51,7 @@ __host__ __device__ inline float bf2f(u16 b) {
     return f;
 }
 
-struct NetDims { int Ni, Nj, Nk, nc, ncs, lo, ntile; int off[NET_TAPS]; };
+struct NetDims { int Ni, Nj, Nk, nc, lo, ntile; };
 
 __device__ __forceinline__ bf16x8 ld8(const u16 *p) {   // 16-byte aligned
     return *reinterpret_cast<const bf16x8 *>(p);
@@ -166,30 +162,39 @@ struct ConvT {
 // Bricks of a block: the launch's bricks in 8 runs, one per XCD, whose L2 then holds
 // the neighbours' shared cells.
 __device__ __forceinline__ int brick_run(int nbrick) { return (nbrick + 7) / 8; }
-static unsigned brick_blocks(int cin, long nbrick) {
-    const long all = (nbrick + 7) / 8 * 8;
-    return (unsigned)(cin == 32 ? std::min<long>(NB_STAY, all) : all);
-}
+static unsigned brick_blocks(long nbrick, long most) { return (unsigned)std::min((nbrick + 7) / 8 * 8, most); }
 
-struct alignas(2) u16x4u { u16 v[4]; };   // 4 cells of a channel, at element alignment
+// 8 BF16 gradients times the slope at the forward outputs m (1/8: exact, so before or after the rounding)
+__device__ __forceinline__ uint4 masked(const uint4 &x, const uint4 &m) {
+    const uint32_t xw[4] = {x.x, x.y, x.z, x.w}, mw[4] = {m.x, m.y, m.z, m.w};
+    uint32_t o[4];
+#pragma unroll
+    for (int h = 0; h < 4; h++) {
+        float l = bf2f((u16)(xw[h] & 0xFFFFu)), u = bf2f((u16)(xw[h] >> 16));
+        if (bf2f((u16)(mw[h] & 0xFFFFu)) <= 0.f) l = NET_LEAK * l;
+        if (bf2f((u16)(mw[h] >> 16)) <= 0.f) u = NET_LEAK * u;
+        o[h] = (uint32_t)f2bf(l) | ((uint32_t)f2bf(u) << 16);
+    }
+    return uint4{o[0], o[1], o[2], o[3]};
+}
 
 // Hidden activation: leaky ReLU, x > 0 ? x : x/8 (a slope that keeps every
 // unit trainable; 1/8 is exact in BF16 and FP32).
-// MODE 0: activation, write act_out (channels last) and actT_out (channel-major), NCO = 32
+// MODE 0: activation, write act_out, NCO = 32
 // MODE 1: linear output, write out[p][0..7] FP32 (NCO = 16, channels 8..15 padding)
 // MODE 2: backward data: multiply by the activation's slope at the forward
-//         output (maskT, channel-major, > 0: 1, else 1/8), write both BF16 layouts, NCO = 32
+//         output (mask > 0: 1, else 1/8), write act_out, NCO = 32
 // Neighbours are those of the flattened cell index (p + off), as at the box faces, whose
-// cells are never used; cells outside [lo, lo + 16 ntile) are not stored.  A lane holds
-// 4 cells of a channel, which go to the channel-major array as they are; whole cells
-// leave through LDS.
+// cells are never used; cells outside [lo, lo + 16 ntile) are not stored.  The results leave
+// through LDS as whole cells.
 // Per launch on a 104^3 grid, A operands from L2 / staged, weights per brick / as now:
-// hidden layer 230 / 151 / 94 us, first 111 / 84 / 62, last 182 / 70 / 43, backward
-// data 272 / 192 / 131.
+// hidden layer 230 / 151 / 69 us, first 111 / 84 / 49, last 182 / 70 / 43, backward
+// data 272 / 192 / 79.  Of that the channel-major copies that the weight gradients once
+// read were 25, 13, 0 and 52.
 template <int CIN, int NCO, int MODE>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CIN == 32 ? 2 : 4)))
 k_conv(NetDims d, const u16 *__restrict__ in, const u16 *__restrict__ W, const float *__restrict__ bias,
-       const u16 *__restrict__ maskT, u16 *__restrict__ act_out, u16 *__restrict__ actT_out, float *__restrict__ out) {
+       const u16 *__restrict__ mask, u16 *__restrict__ act_out, float *__restrict__ out) {
     static_assert(CIN == 8 || CIN == 32, "8 or 32 input channels");
     static_assert(NB_I == 16 && NB_K == 4, "one 16-cell tile per row, four waves on four k rows");
     using T = ConvT<CIN, NCO>;
@@ -244,31 +249,13 @@ k_conv(NetDims d, const u16 *__restrict__ in, const u16 *__restrict__ W, const f
                     for (int r = 0; r < 4; r++) sF[(oc + r) * 8 + co] = x[r] + bb;
                 }
             } else {
-                const int i = oi + 4 * cv.kg, p = i + d.Ni * ((oj + m) + d.Nj * (ok + kk));
-                const bool rowin = oj + m < d.Nj && ok + kk < d.Nk;
-                const bool full = rowin && i + 3 < d.Ni && p >= d.lo && p + 3 < hi;
-                auto in1 = [&](int r) { return rowin && i + r < d.Ni && p + r >= d.lo && p + r < hi; };
-                const size_t pt = (size_t)co * d.ncs + p;
-                u16x4u h, mk;
-                if constexpr (MODE == 2) {
-                    if (full) mk = *reinterpret_cast<const u16x4u *>(maskT + pt);
-                    else
-#pragma unroll
-                        for (int r = 0; r < 4; r++) mk.v[r] = in1(r) ? maskT[pt + r] : 0;
-                }
+                const float bb = MODE == 0 ? bias[co] : 0.f;
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
                     float y = x[r];
-                    if constexpr (MODE == 0) { y += bias[co]; y = y > 0.f ? y : NET_LEAK * y; }
-                    else if (bf2f(mk.v[r]) <= 0.f) y = NET_LEAK * y;   // slope at the forward output
-                    h.v[r] = f2bf(y);
-                    sO[(oc + r) * OS + co] = h.v[r];
+                    if constexpr (MODE == 0) { y += bb; y = y > 0.f ? y : NET_LEAK * y; }
+                    sO[(oc + r) * OS + co] = f2bf(y);
                 }
-                if (full) *reinterpret_cast<u16x4u *>(actT_out + pt) = h;
-                else
-#pragma unroll
-                    for (int r = 0; r < 4; r++)
-                        if (in1(r)) actT_out[pt + r] = h.v[r];
             }
         }
         __syncthreads();   // results in sOut; and every wave is done with sIn
@@ -278,145 +265,183 @@ k_conv(NetDims d, const u16 *__restrict__ in, const u16 *__restrict__ W, const f
             const int i = oi + oc % NB_I, j = oj + (oc / NB_I) % NB_J, k = ok + oc / (NB_I * NB_J), p = i + d.Ni * (j + d.Nj * k);
             if (i >= d.Ni || j >= d.Nj || k >= d.Nk || p < d.lo || p >= hi) continue;
             if constexpr (MODE == 1) *reinterpret_cast<uint4 *>(out + (size_t)p * 8 + 4 * q) = sOut[e];
-            else *reinterpret_cast<uint4 *>(act_out + (size_t)p * NET_C + 8 * q) = sOut[oc * (OS / 8) + q];
+            else {
+                uint4 x = sOut[oc * (OS / 8) + q];
+                if constexpr (MODE == 2) x = masked(x, *reinterpret_cast<const uint4 *>(mask + (size_t)p * NET_C + 8 * q));
+                *reinterpret_cast<uint4 *>(act_out + (size_t)p * NET_C + 8 * q) = x;
+            }
         }
     }
 }
 
 // Weight and bias gradients of one layer, dW[tap][co][ci] += sum_p g[p][co] *
 // a[p + off][ci] and db[co] += sum_p g[p][co]: per tap a GEMM with M = output
-// channels, N = input channels and K = cells.  A wave keeps the sums of the 9 taps
-// of one dz (up to 144 accumulator registers) while it walks its cells, 64 (two K
-// steps, a whole 128-byte line of each row) at a time: the gradient rows (A,
-// channel-major, 32 aligned bytes per lane) are loaded once for all 9 taps, the
-// activation rows (B) once per dy, 40 bytes per lane from which the three dx are taken
-// (whole dwords or v_alignbyte by one element).  So 64 cells are up to 76 MFMAs on 16
-// 16-byte and 6 8-byte loads; one tap per wave would
-// load 6 16-byte vectors for every 4 MFMAs and was bound by them.  The bias is one
-// more MFMA against ones, on the waves of the first dz.  The 4 waves of a block add up in
-// LDS and the block writes its sums to a workspace that k_wreduce adds in block
-// order, so the gradients do not depend on the order blocks finish in.  Cells outside the
-// computed range carry a zero gradient (never written, zero from allocation); the
-// arrays' zero padding covers the reads past either end.
-// Per launch on a 104^3 grid, layers 2 / 1 / 0: 463 / 813 / 435 us (one tap per wave,
-// FP32 atomics, and 38 us each for the bias) -> 187 / 231 / 119, and 18 for the sums.
-struct alignas(4) u32x4u { uint32_t v[4]; };   // loads at dword alignment
-struct alignas(4) u32x2u { uint32_t v[2]; };
-__device__ __forceinline__ bf16x8 bf8(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
-    const uint32_t r[4] = {a, b, c, d};
-    bf16x8 v;
-    memcpy(&v, r, 16);
-    return v;
+// channels, N = input channels and K = cells.  Both operands are staged channels
+// last, a brick of gradients and the activations one cell around it, and read with
+// the transposing LDS read (ds_read_b64_tr_b16: lane l of 16 gets column l of 4 rows of
+// 16): a row of 16 cells is half of a K step of any dx, a step is the rows j, j + 2, and a pair
+// of activation rows serves up to two steps and three k rows.  So a brick is
+// read from memory 2.5 times, not 9, and needs no channel-major copy of either array.
+// A wave keeps the 27 taps of one 16 x 16 tile (108 accumulator registers) on
+// KK of the brick's 4 k rows; the bias is one more MFMA against ones.  The two LDS buffers
+// alternate: the next brick's loads are in flight while this one's MFMAs run.
+// Per wave and brick (MT = NT = 2) 108 MFMAs on 112 8-byte reads: the LDS and the
+// matrix units are about equally busy.  The block's waves add up in LDS, and the
+// block writes its sums to a workspace that k_wreduce adds in a fixed order, so the
+// gradients do not depend on the order blocks finish in.  Cells outside the
+// computed range carry a zero gradient (never written, zero from allocation).
+// Per launch on a 104^3 grid, layers 2 / 1 / 0: 463 / 813 / 435 us with one tap per wave,
+// 187 / 231 / 119 with channel-major rows from L2 -> 55 / 77 / 52, and 5 for the sums (18 before).
+#define WG_BLOCKS 256   // one per CU: 2 waves per SIMD
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef bf16x4 __attribute__((address_space(3))) lds_bf16x4;
+__device__ __forceinline__ bf16x8 tr_rows(const u16 *a, const u16 *b) {   // 4 + 4 cells of a channel
+    const bf16x4 x = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4 *)a), y = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4 *)b);
+    return __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7);
 }
-#define WG_BLOCKS 170   // blocks per dz: 2 waves on each of the chip's 1024 SIMDs in all
 
 template <int MT, int NT>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
-k_wgrad(NetDims d, const u16 *__restrict__ gT, const u16 *__restrict__ aT, int steps,
-                                               float *__restrict__ ws) {
-    __shared__ float red[9 * MT * NT * 256 + MT * 16];
-    const int zi = blockIdx.x % 3, blk = blockIdx.x / 3;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, row = lane & 15, kg = lane >> 4;
-    const int A0 = d.lo & ~7, A1 = d.lo + 16 * d.ntile;
-    const int c0 = A0 + 64 * steps * (blk * 4 + wave), c1 = min(c0 + 64 * steps, A1);
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
+k_wgrad(NetDims d, const u16 *__restrict__ g, const u16 *__restrict__ act, float *__restrict__ ws) {
+    static_assert(NB_I == 16 && NB_J == 4 && NB_K == 4, "two K steps of two rows per k row");
+    constexpr int PA = 2 * NT, PG = 2 * MT;                   // 16-byte pieces per staged cell
+    constexpr int SA = NT == 2 ? 40 : 24, SG = MT == 2 ? 40 : 24;   // BF16 elements per staged cell: rows fall on distinct banks
+    constexpr int NA = NB_LC * PA, NG = NB_OC * PG, NIT = (NA + NG + 511) / 512;
+    constexpr int KS = 8 / (MT * NT), KK = NB_K / KS;         // waves per tile, k rows per wave
+    constexpr int NW = 27 * MT * NT * 256;                    // sums of a block
+    constexpr int BUF = (NB_LC * SA + NB_OC * SG) / 8;
+    constexpr int RED = (NW + MT * 16) / 4;
+    __shared__ uint4 smem[2 * BUF > RED ? 2 * BUF : RED];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, row = lane & 15, kg = lane >> 4;
+    const int mt = wave % MT, nt = (wave / MT) % NT, ks = wave / (MT * NT);
+    const int nbi = (d.Ni + NB_I - 1) / NB_I, nbj = (d.Nj + NB_J - 1) / NB_J, nb = nbi * nbj * ((d.Nk + NB_K - 1) / NB_K);
+    const int run = brick_run(nb), b0 = (blockIdx.x & 7) * run, b1 = min(b0 + run, nb), step = gridDim.x >> 3;
+    uint4 v[NIT];
+    auto fetch = [&](int b) {
+        const int oi = NB_I * (b % nbi), oj = NB_J * ((b / nbi) % nbj), ok = NB_K * (b / (nbi * nbj));
+#pragma unroll
+        for (int it = 0; it < NIT; it++) {
+            const int e = tid + 512 * it;
+            v[it] = uint4{0u, 0u, 0u, 0u};
+            if (e < NA) {          // as the convolutions: neighbours of the flattened index
+                const int c = e / PA, li = c % NB_LI, lj = (c / NB_LI) % NB_LJ, lk = c / (NB_LI * NB_LJ);
+                const int p = (oi - 1 + li) + d.Ni * ((oj - 1 + lj) + d.Nj * (ok - 1 + lk));
+                if (p >= 0 && p < d.nc) v[it] = *reinterpret_cast<const uint4 *>(act + (size_t)p * NET_C + 8 * (e % PA));
+            } else if (e < NA + NG) {
+                const int c = (e - NA) / PG, i = oi + c % NB_I, j = oj + (c / NB_I) % NB_J, k = ok + c / (NB_I * NB_J);
+                if (i < d.Ni && j < d.Nj && k < d.Nk)
+                    v[it] = *reinterpret_cast<const uint4 *>(g + ((size_t)i + (size_t)d.Ni * (j + (size_t)d.Nj * k)) * NET_C + 8 * ((e - NA) % PG));
+            }
+        }
+    };
+    auto stage = [&](uint4 *buf) {
+#pragma unroll
+        for (int it = 0; it < NIT; it++) {
+            const int e = tid + 512 * it;
+            if (e < NA) buf[(e / PA) * (SA / 8) + e % PA] = v[it];
+            else if (e < NA + NG) buf[NB_LC * SA / 8 + ((e - NA) / PG) * (SG / 8) + (e - NA) % PG] = v[it];
+        }
+    };
     const uint32_t o1 = 0x3F803F80u;   // two BF16 ones
-    const bf16x8 ones = bf8(o1, o1, o1, o1);
-    f32x4 acc[3][3][MT][NT], accb[MT];
+    const uint4 o4 = {o1, o1, o1, o1};
+    bf16x8 ones;
+    memcpy(&ones, &o4, 16);
+    f32x4 acc[27], accb = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int m = 0; m < MT; m++) {
-        accb[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int q = 0; q < 27; q++) acc[q] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int cell = 4 * kg + (row >> 2), ch = 4 * (row & 3);   // this lane's address in a transposing read
+    int b = b0 + (blockIdx.x >> 3);
+    if (b < b1) { fetch(b); stage(smem); }
+    for (int cur = 0; b < b1; b += step, cur ^= 1) {
+        __syncthreads();   // this brick staged; every wave is done with the other buffer
+        const bool more = b + step < b1;
+        if (more) fetch(b + step);
+        const u16 *sA = reinterpret_cast<const u16 *>(smem + cur * BUF) + ((KK * ks) * (NB_LJ * NB_LI) + cell) * SA + 16 * nt + ch;
+        const u16 *sG = reinterpret_cast<const u16 *>(smem + cur * BUF) + NB_LC * SA + ((KK * ks) * (NB_J * NB_I) + cell) * SG + 16 * mt + ch;
+        bf16x8 av[KK][2];   // rows (s, s + 2) of the gradients
 #pragma unroll
-        for (int q = 0; q < 9 * NT; q++) acc[q / (3 * NT)][(q / NT) % 3][m][q % NT] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-    for (int c = c0; c < c1; c += 64) {
-        const int pk = c + 16 * kg;                            // 16 cells of this lane group, 8 in each of two K steps
-        bf16x8 av[2][MT];                                      // A[m = co][k = cell]
+        for (int q = 0; q < 2 * KK; q++) {
+            const u16 *r = sG + ((q / 2) * NB_J + q % 2) * NB_I * SG;
+            av[q / 2][q % 2] = tr_rows(r, r + 2 * NB_I * SG);
+        }
+        if (nt == 0) {
 #pragma unroll
-        for (int m = 0; m < MT; m++)
-#pragma unroll
-            for (int h = 0; h < 2; h++) av[h][m] = ld8(gT + (size_t)(16 * m + row) * d.ncs + pk + 8 * h);
-        if (zi == 0) {
-#pragma unroll
-            for (int m = 0; m < MT; m++)
-#pragma unroll
-                for (int h = 0; h < 2; h++) accb[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[h][m], ones, accb[m], 0, 0, 0);
+            for (int q = 0; q < 2 * KK; q++) accb = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[q / 2][q % 2], ones, accb, 0, 0, 0);
         }
 #pragma unroll
-        for (int dy = 0; dy < 3; dy++) {
-            const int off = d.off[9 * zi + 3 * dy + 1];        // the tap dx = 0
-            const bool odd = (off + 1) & 1;                    // uniform: the wanted cells start at an odd element of u
+        for (int n = 0; n < (KK + 2) * 3; n++) {
+            const int pl = n / 3, dx = n % 3;   // staged plane: dz = pl - k row (0..2)
+            bf16x8 bv[4];                       // staged rows (x, x + 2): dy = x - s
 #pragma unroll
-            for (int n = 0; n < NT; n++) {
-                uint32_t u[10], sh[9];                         // cells pk + off - 1 (- 1 if odd) ..; moved by one element
-                const u16 *p = aT + (ptrdiff_t)(16 * n + row) * d.ncs + (pk + off - 1 - (odd ? 1 : 0));
-                const u32x4u x0 = *reinterpret_cast<const u32x4u *>(p), x1 = *reinterpret_cast<const u32x4u *>(p + 8);
-                const u32x2u y = *reinterpret_cast<const u32x2u *>(p + 16);
+            for (int x = 0; x < 4; x++) {
+                const u16 *r = sA + ((pl * NB_LJ + x) * NB_LI + dx) * SA;
+                bv[x] = tr_rows(r, r + 2 * NB_LI * SA);
+            }
 #pragma unroll
-                for (int q = 0; q < 4; q++) { u[q] = x0.v[q]; u[4 + q] = x1.v[q]; }
-                u[8] = y.v[0]; u[9] = y.v[1];
+            for (int k = 0; k < KK; k++) {
+                if (pl - k < 0 || pl - k > 2) continue;
 #pragma unroll
-                for (int q = 0; q < 9; q++) sh[q] = __builtin_amdgcn_alignbyte(u[q + 1], u[q], 2);
-#pragma unroll
-                for (int h = 0; h < 2; h++) {
-                    const uint32_t *a = u + 4 * h, *b = sh + 4 * h;
-                    bf16x8 bv[3];
-                    if (odd) { bv[0] = bf8(b[0], b[1], b[2], b[3]); bv[1] = bf8(a[1], a[2], a[3], a[4]); bv[2] = bf8(b[1], b[2], b[3], b[4]); }
-                    else { bv[0] = bf8(a[0], a[1], a[2], a[3]); bv[1] = bf8(b[0], b[1], b[2], b[3]); bv[2] = bf8(a[1], a[2], a[3], a[4]); }
-#pragma unroll
-                    for (int dx = 0; dx < 3; dx++)
-#pragma unroll
-                        for (int m = 0; m < MT; m++)
-                            acc[dy][dx][m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[h][m], bv[dx], acc[dy][dx][m][n], 0, 0, 0);
+                for (int q = 0; q < 6; q++) {
+                    const int tap = 9 * (pl - k) + 3 * (q % 3) + dx;
+                    acc[tap] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[k][q / 3], bv[q / 3 + q % 3], acc[tap], 0, 0, 0);
                 }
             }
         }
+        if (more) stage(smem + (cur ^ 1) * BUF);
     }
-    // D[i = co][j = ci]: lane holds co = 16m + 4kg + r, ci = 16n + row
-    for (int w = 0; w < 4; w++) {
-        if (wave == w) {
+    // D[i = co][j = ci]: lane holds co = 16 mt + 4 kg + r, ci = 16 nt + row
+    float *red = reinterpret_cast<float *>(smem);
+    for (int q = 0; q < KS; q++) {
+        __syncthreads();
+        if (ks != q) continue;
 #pragma unroll
-            for (int t = 0; t < 9; t++)
+        for (int t = 0; t < 27; t++)
 #pragma unroll
-                for (int m = 0; m < MT; m++)
+            for (int r = 0; r < 4; r++) {
+                float &x = red[((t * MT + mt) * 16 + 4 * kg + r) * (16 * NT) + 16 * nt + row];
+                x = q == 0 ? acc[t][r] : x + acc[t][r];
+            }
+        if (nt == 0 && row == 0) {
 #pragma unroll
-                    for (int n = 0; n < NT; n++)
-#pragma unroll
-                        for (int r = 0; r < 4; r++) {
-                            float &x = red[((t * MT + m) * 16 + 4 * kg + r) * (16 * NT) + 16 * n + row];
-                            x = w == 0 ? acc[t / 3][t % 3][m][n][r] : x + acc[t / 3][t % 3][m][n][r];
-                        }
-            if (row == 0) {
-#pragma unroll
-                for (int m = 0; m < MT; m++)
-#pragma unroll
-                    for (int r = 0; r < 4; r++) {
-                        float &x = red[9 * MT * NT * 256 + 16 * m + 4 * kg + r];
-                        x = w == 0 ? accb[m][r] : x + accb[m][r];
-                    }
+            for (int r = 0; r < 4; r++) {
+                float &x = red[NW + 16 * mt + 4 * kg + r];
+                x = q == 0 ? accb[r] : x + accb[r];
             }
         }
-        __syncthreads();
     }
-    // workspace of a block index: 27 taps of [co][ci], then the biases
-    float *out = ws + (size_t)blk * (27 * MT * NT * 256 + MT * 16);
-    for (int e = threadIdx.x; e < 9 * MT * NT * 256; e += 256) out[(size_t)zi * (9 * MT * NT * 256) + e] = red[e];
-    if (zi == 0 && threadIdx.x < MT * 16) out[27 * MT * NT * 256 + threadIdx.x] = red[9 * MT * NT * 256 + threadIdx.x];
+    __syncthreads();
+    // workspace of a block: 27 taps of [co][ci], then the biases
+    for (int e = tid; e < RED; e += 512) reinterpret_cast<uint4 *>(ws)[(size_t)blockIdx.x * RED + e] = smem[e];
 }
 
-// the blocks' sums, in block order, onto the unpadded parameter layout [tap][nco][nci], [nco]
+// the blocks' sums onto the unpadded parameter layout [tap][nco][nci], [nco]: 64 sums per
+// block, each in 16 runs of blocks added in order
 template <int MT, int NT>
 __global__ void __launch_bounds__(256) k_wreduce(const float *__restrict__ ws, int nblk, int nco, int nci, float *__restrict__ dW,
                                                  float *__restrict__ db) {
     constexpr int NW = 27 * MT * NT * 256, N = NW + MT * 16;
-    const int e = blockIdx.x * 256 + threadIdx.x;
-    if (e >= N) return;
+    __shared__ float part[16][64];
+    const int run = (nblk + 15) / 16, q = threadIdx.x & 15, r = threadIdx.x >> 4;   // 4 sums, blocks [r run, (r + 1) run)
+    const int e0 = blockIdx.x * 64 + 4 * q, b0 = r * run, b1 = min(b0 + run, nblk);
+    float4 s = {0.f, 0.f, 0.f, 0.f};
+    if (e0 < N) {
+#pragma unroll 8
+        for (int b = b0; b < b1; b++) {
+            const float4 x = *reinterpret_cast<const float4 *>(ws + (size_t)b * N + e0);
+            s.x += x.x; s.y += x.y; s.z += x.z; s.w += x.w;
+        }
+    }
+    part[r][4 * q] = s.x; part[r][4 * q + 1] = s.y; part[r][4 * q + 2] = s.z; part[r][4 * q + 3] = s.w;
+    __syncthreads();
+    const int e = blockIdx.x * 64 + threadIdx.x;
+    if (threadIdx.x >= 64 || e >= N) return;
     const int ci = e % (16 * NT), co = e < NW ? (e / (16 * NT)) % (16 * MT) : e - NW, tap = e / (MT * NT * 256);
     if (co >= nco || (e < NW && ci >= nci)) return;
-    float s = 0.f;
-#pragma unroll 10
-    for (int b = 0; b < nblk; b++) s += ws[(size_t)b * N + e];
-    if (e < NW) dW[((size_t)tap * nco + co) * nci + ci] += s;
-    else db[co] += s;
+    float t = 0.f;
+#pragma unroll
+    for (int k = 0; k < 16; k++) t += part[k][threadIdx.x];
+    if (e < NW) dW[((size_t)tap * nco + co) * nci + ci] += t;
+    else db[co] += t;
 }
 
 __device__ __forceinline__ uint4 pack8(const float (&f)[8]) {
@@ -425,19 +450,10 @@ __device__ __forceinline__ uint4 pack8(const float (&f)[8]) {
     for (int h = 0; h < 4; h++) o[h] = (uint32_t)f2bf(f[2 * h]) | ((uint32_t)f2bf(f[2 * h + 1]) << 16);
     return uint4{o[0], o[1], o[2], o[3]};
 }
-// 8 BF16 channels of cell p to the rows of a channel-major array
-__device__ __forceinline__ void put_rows(const uint4 &v, u16 *T, int ncs, int p) {
-    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-    for (int c = 0; c < 8; c++) T[(size_t)c * ncs + p] = (u16)(w[c / 2] >> (16 * (c & 1)));
-}
-
-// dL/dout (FP32 [nc][8]) -> BF16 gradient of the last layer, both layouts; zero
-// outside the computed cells, where the output is not defined.  The cell's
-// channels 8..31 are zeros (the buffer held another layer's gradient); the rows 8..15
-// that the weight gradient also reads only reach outputs it drops.  Whole 16-byte
-// stores: 76 -> 31 us on a 104^3 grid with one 2-byte store per channel before.
-__global__ void __launch_bounds__(256) k_dout(NetDims d, const float *__restrict__ dout, u16 *__restrict__ g, u16 *__restrict__ gT) {
+// dL/dout (FP32 [nc][8]) -> BF16 gradient of the last layer; zero outside the
+// computed cells, where the output is not defined.  The cell's channels 8..31 are
+// zeros (the buffer held another layer's gradient).
+__global__ void __launch_bounds__(256) k_dout(NetDims d, const float *__restrict__ dout, u16 *__restrict__ g) {
     const int p = blockIdx.x * 256 + threadIdx.x;
     if (p >= d.nc) return;
     uint4 v = {0u, 0u, 0u, 0u};
@@ -451,7 +467,6 @@ __global__ void __launch_bounds__(256) k_dout(NetDims d, const float *__restrict
     gp[0] = v;
 #pragma unroll
     for (int q = 1; q < 4; q++) gp[q] = uint4{0u, 0u, 0u, 0u};
-    put_rows(v, gT, d.ncs, p);
 }
 
 // state -> input features ((rho - rho0)/s_rho, v/s_v, (p - p0)/s_p, B/s_B) of cell p
@@ -480,17 +495,15 @@ __device__ __forceinline__ void features_of(size_t p, size_t n, const R *__restr
     features_calc(q, gamma, sc, off, f);
 }
 
-// the features, BF16, both layouts (channels 8..31 stay the zeros of the allocation)
+// the features, BF16 (channels 8..31 stay the zeros of the allocation)
 template <typename R>
-__global__ void __launch_bounds__(256) k_features(int nc, int ncs, const R *__restrict__ Gas, const R *__restrict__ B, float gamma,
-                                                  float4 sc, float2 off, u16 *__restrict__ act, u16 *__restrict__ actT) {
+__global__ void __launch_bounds__(256) k_features(int nc, const R *__restrict__ Gas, const R *__restrict__ B, float gamma,
+                                                  float4 sc, float2 off, u16 *__restrict__ act) {
     int p = blockIdx.x * 256 + threadIdx.x;
     if (p >= nc) return;
     float f[8];
     features_of<R>(p, nc, Gas, B, gamma, sc, off, f);
-    const uint4 v = pack8(f);
-    *reinterpret_cast<uint4 *>(act + (size_t)p * NET_C) = v;
-    put_rows(v, actT, ncs, p);
+    *reinterpret_cast<uint4 *>(act + (size_t)p * NET_C) = pack8(f);
 }
 
 // ----------------------------------------------------------------- inference
@@ -650,9 +663,12 @@ struct gam_net {
     // parameters: FP32 master, grads, Adam moments
     float *w = nullptr, *g = nullptr, *m = nullptr, *v = nullptr;
     u16 *Wf[3] = {}, *Wb[3] = {};
-    u16 *act[4] = {}, *actT[4] = {};     // 0 features, 1..2 hidden, 3 scratch gradient
-    u16 *gr[2] = {}, *grT[2] = {};       // gradient ping-pong
-    u16 *actT0[4] = {}, *grT0[2] = {};   // allocations of the channel-major arrays (NET_PAD before row 0)
+    u16 *act[3] = {}, *inf[2] = {};      // forward: 0 features, 1..2 hidden; inference's hidden
+    // A backward pass takes the last forward's activations, so inference writes inf once
+    // a forward has run.  Before the first one it writes act: the up to 15 cells past the
+    // forward's whole tiles, which no forward stores, then hold inferred values.
+    bool forwarded = false;
+    u16 *gr[2] = {};                     // gradient ping-pong
     float *out = nullptr;
     float *dbuf = nullptr;               // upstream gradient uploaded from the host
     float *ws = nullptr;                 // the weight-gradient blocks' sums (k_wgrad)
@@ -681,8 +697,7 @@ extern "C" int gam_net_destroy(gam_net *n) {
     void *bufs[] = {n->w, n->g, n->m, n->v, n->out, n->dbuf, n->ws};
     for (void *b : bufs) if (b) (void)hipFree(b);
     for (int l = 0; l < 3; l++) { (void)hipFree(n->Wf[l]); (void)hipFree(n->Wb[l]); }
-    for (int q = 0; q < 4; q++) { (void)hipFree(n->act[q]); (void)hipFree(n->actT0[q]); }
-    for (int q = 0; q < 2; q++) { (void)hipFree(n->gr[q]); (void)hipFree(n->grT0[q]); }
+    for (u16 *b : {n->act[0], n->act[1], n->act[2], n->inf[0], n->inf[1], n->gr[0], n->gr[1]}) (void)hipFree(b);
     if (n->done) (void)hipEventDestroy(n->done);
     if (n->own) (void)hipStreamDestroy(n->own);
     delete n;
@@ -693,18 +708,13 @@ extern "C" int gam_net_create(int Ni, int Nj, int Nk, gam_net **out) {
     if (!out || Ni < 8 || Nj < 8 || Nk < 8) return -1;   // the 3-layer stencil needs 3 cells around each used cell
     *out = nullptr;
     long nc = (long)Ni * Nj * Nk;
-    if ((nc + 24) * NET_C + 2 * NET_PAD > 0x7fffffffL) return -1;
+    if ((nc + 28) * NET_C > 0x7fffffffL) return -1;
     gam_net *n = new gam_net();
     NetDims &d = n->d;
     d.Ni = Ni; d.Nj = Nj; d.Nk = Nk; d.nc = (int)nc;
-    d.ncs = (int)(((nc + 7) / 8) * 8 + 16);   // channel-major row stride: 16-byte aligned rows, a gap between them
     const int O = Ni * Nj + Ni + 1;
     d.lo = O;
     d.ntile = (int)((nc - 2L * O) / 16);
-    for (int t = 0; t < NET_TAPS; t++) {
-        int dx = t % 3 - 1, dy = (t / 3) % 3 - 1, dz = t / 9 - 1;
-        d.off[t] = dx + Ni * (dy + Nj * dz);
-    }
     auto cleanup = [&](int c) { gam_net_destroy(n); return c; };
     if (hipStreamCreateWithFlags(&n->own, hipStreamNonBlocking) != hipSuccess) return cleanup(-2);
     n->stream = n->own;
@@ -719,16 +729,10 @@ extern "C" int gam_net_create(int Ni, int Nj, int Nk, gam_net **out) {
         if (hipMalloc(&n->Wb[l], (size_t)NET_TAPS * NET_C * NET_C * 2) != hipSuccess) return cleanup(-3);
         if (hipMemset(n->Wb[l], 0, (size_t)NET_TAPS * NET_C * NET_C * 2) != hipSuccess) return cleanup(-2);
     }
-    const size_t ab = (size_t)nc * NET_C * 2, abT = ((size_t)d.ncs * NET_C + 2 * NET_PAD) * 2;
-    for (int q = 0; q < 4; q++) {
-        if (hipMalloc(&n->act[q], ab) != hipSuccess || hipMalloc(&n->actT0[q], abT) != hipSuccess) return cleanup(-3);
-        if (hipMemset(n->act[q], 0, ab) != hipSuccess || hipMemset(n->actT0[q], 0, abT) != hipSuccess) return cleanup(-2);
-        n->actT[q] = n->actT0[q] + NET_PAD;
-    }
-    for (int q = 0; q < 2; q++) {
-        if (hipMalloc(&n->gr[q], ab) != hipSuccess || hipMalloc(&n->grT0[q], abT) != hipSuccess) return cleanup(-3);
-        if (hipMemset(n->gr[q], 0, ab) != hipSuccess || hipMemset(n->grT0[q], 0, abT) != hipSuccess) return cleanup(-2);
-        n->grT[q] = n->grT0[q] + NET_PAD;
+    const size_t ab = (size_t)nc * NET_C * 2;
+    for (u16 **p : {&n->act[0], &n->act[1], &n->act[2], &n->inf[0], &n->inf[1], &n->gr[0], &n->gr[1]}) {
+        if (hipMalloc(p, ab) != hipSuccess) return cleanup(-3);
+        if (hipMemset(*p, 0, ab) != hipSuccess) return cleanup(-2);
     }
     if (hipMalloc(&n->out, (size_t)nc * 8 * sizeof(float)) != hipSuccess) return cleanup(-3);
     if (hipMalloc(&n->dbuf, (size_t)nc * 8 * sizeof(float)) != hipSuccess) return cleanup(-3);
@@ -797,10 +801,10 @@ extern "C" int gam_net_set_offsets(gam_net *n, float rho0, float p0) {
 extern "C" int gam_net_features(gam_net *n, const void *Gas, const void *B, int precision) {
     if (!n || !Gas || !B) return -1;
     const int nb = (n->d.nc + 255) / 256;
-    if (precision) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_features<float>), dim3(nb), 256, 0, n->stream, n->d.nc, n->d.ncs, (const float *)Gas,
-                                      (const float *)B, n->gamma, n->scales, n->offs, n->act[0], n->actT[0]);
-    else hipLaunchKernelGGL(HIP_KERNEL_NAME(k_features<double>), dim3(nb), 256, 0, n->stream, n->d.nc, n->d.ncs, (const double *)Gas,
-                            (const double *)B, n->gamma, n->scales, n->offs, n->act[0], n->actT[0]);
+    if (precision) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_features<float>), dim3(nb), 256, 0, n->stream, n->d.nc, (const float *)Gas,
+                                      (const float *)B, n->gamma, n->scales, n->offs, n->act[0]);
+    else hipLaunchKernelGGL(HIP_KERNEL_NAME(k_features<double>), dim3(nb), 256, 0, n->stream, n->d.nc, (const double *)Gas,
+                            (const double *)B, n->gamma, n->scales, n->offs, n->act[0]);
     NCHK(n, hipGetLastError());
     return 0;
 }
@@ -808,30 +812,31 @@ extern "C" int gam_net_features(gam_net *n, const void *Gas, const void *B, int 
 extern "C" int gam_net_set_features(gam_net *n, const float *feat) {
     // host features [nc][8] FP32 (tests): rounded to BF16 like k_features
     if (!n || !feat) return -1;
-    const size_t nc = n->d.nc, ncs = n->d.ncs;
-    std::vector<u16> a(nc * NET_C, 0), aT(ncs * NET_C, 0);
+    const size_t nc = n->d.nc;
+    std::vector<u16> a(nc * NET_C, 0);
     for (size_t p = 0; p < nc; p++)
-        for (int c = 0; c < 8; c++) { u16 b = f2bf(feat[p * 8 + c]); a[p * NET_C + c] = b; aT[c * ncs + p] = b; }
+        for (int c = 0; c < 8; c++) a[p * NET_C + c] = f2bf(feat[p * 8 + c]);
     NCHK(n, hipMemcpyAsync(n->act[0], a.data(), a.size() * 2, hipMemcpyHostToDevice, n->stream));
-    NCHK(n, hipMemcpyAsync(n->actT[0], aT.data(), aT.size() * 2, hipMemcpyHostToDevice, n->stream));
     NCHK(n, hipStreamSynchronize(n->stream));
     return 0;
 }
 
-static dim3 conv_grid(const gam_net *n, int cin) {
+static unsigned conv_blocks(const gam_net *n, long most) {
     const NetDims &d = n->d;
-    return dim3(brick_blocks(cin, (long)((d.Ni + NB_I - 1) / NB_I) * ((d.Nj + NB_J - 1) / NB_J) * ((d.Nk + NB_K - 1) / NB_K)));
+    return brick_blocks((long)((d.Ni + NB_I - 1) / NB_I) * ((d.Nj + NB_J - 1) / NB_J) * ((d.Nk + NB_K - 1) / NB_K), most);
 }
+static dim3 conv_grid(const gam_net *n, int cin) { return dim3(conv_blocks(n, cin == 32 ? NB_STAY : 0x7fffffffL)); }
 
 extern "C" int gam_net_forward(gam_net *n) {
     if (!n) return -1;
     const NetDims &d = n->d;
+    n->forwarded = true;
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_conv<8, 32, 0>), conv_grid(n, 8), 256, 0, n->stream, d, (const u16 *)n->act[0], (const u16 *)n->Wf[0],
-                       (const float *)(n->w + boff(0)), (const u16 *)nullptr, n->act[1], n->actT[1], (float *)nullptr);
+                       (const float *)(n->w + boff(0)), (const u16 *)nullptr, n->act[1], (float *)nullptr);
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_conv<32, 32, 0>), conv_grid(n, 32), 256, 0, n->stream, d, (const u16 *)n->act[1], (const u16 *)n->Wf[1],
-                       (const float *)(n->w + boff(1)), (const u16 *)nullptr, n->act[2], n->actT[2], (float *)nullptr);
+                       (const float *)(n->w + boff(1)), (const u16 *)nullptr, n->act[2], (float *)nullptr);
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_conv<32, 16, 1>), conv_grid(n, 32), 256, 0, n->stream, d, (const u16 *)n->act[2], (const u16 *)n->Wf[2],
-                       (const float *)(n->w + boff(2)), (const u16 *)nullptr, (u16 *)nullptr, (u16 *)nullptr, n->out);
+                       (const float *)(n->w + boff(2)), (const u16 *)nullptr, (u16 *)nullptr, n->out);
     NCHK(n, hipGetLastError());
     return 0;
 }
@@ -853,19 +858,20 @@ extern "C" int gam_net_infer(gam_net *n, const void *Gas, const void *B, int pre
             bx[l].nb[a] = (bx[l].n[a] + nb[a] - 1) / nb[a];
         }
     }
-    auto grid = [](int cin, const InferBox &b) { return dim3(brick_blocks(cin, (long)b.nb[0] * b.nb[1] * b.nb[2])); };
+    u16 *h1 = n->forwarded ? n->inf[0] : n->act[1], *h2 = n->forwarded ? n->inf[1] : n->act[2];
+    auto grid = [](int cin, const InferBox &b) { return dim3(brick_blocks((long)b.nb[0] * b.nb[1] * b.nb[2], cin == 32 ? NB_STAY : 0x7fffffffL)); };
     if (precision)
         hipLaunchKernelGGL(HIP_KERNEL_NAME(k_infer<8, 32, 0, float>), grid(8, bx[0]), 256, 0, n->stream, d, bx[0], (const u16 *)nullptr,
                            (const float *)Gas, (const float *)B, n->gamma, n->scales, n->offs, (const u16 *)n->Wf[0],
-                           (const float *)(n->w + boff(0)), n->act[1], (float *)nullptr);
+                           (const float *)(n->w + boff(0)), h1, (float *)nullptr);
     else
         hipLaunchKernelGGL(HIP_KERNEL_NAME(k_infer<8, 32, 0, double>), grid(8, bx[0]), 256, 0, n->stream, d, bx[0], (const u16 *)nullptr,
                            (const double *)Gas, (const double *)B, n->gamma, n->scales, n->offs, (const u16 *)n->Wf[0],
-                           (const float *)(n->w + boff(0)), n->act[1], (float *)nullptr);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_infer<32, 32, 0, float>), grid(32, bx[1]), 256, 0, n->stream, d, bx[1], (const u16 *)n->act[1],
+                           (const float *)(n->w + boff(0)), h1, (float *)nullptr);
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_infer<32, 32, 0, float>), grid(32, bx[1]), 256, 0, n->stream, d, bx[1], (const u16 *)h1,
                        (const float *)nullptr, (const float *)nullptr, n->gamma, n->scales, n->offs, (const u16 *)n->Wf[1],
-                       (const float *)(n->w + boff(1)), n->act[2], (float *)nullptr);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_infer<32, 16, 1, float>), grid(32, bx[2]), 256, 0, n->stream, d, bx[2], (const u16 *)n->act[2],
+                       (const float *)(n->w + boff(1)), h2, (float *)nullptr);
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_infer<32, 16, 1, float>), grid(32, bx[2]), 256, 0, n->stream, d, bx[2], (const u16 *)h2,
                        (const float *)nullptr, (const float *)nullptr, n->gamma, n->scales, n->offs, (const u16 *)n->Wf[2],
                        (const float *)(n->w + boff(2)), (u16 *)nullptr, n->out);
     NCHK(n, hipGetLastError());
@@ -880,28 +886,26 @@ extern "C" void *gam_net_infer_event(gam_net *n) { return n ? (void *)n->done : 
 extern "C" int gam_net_backward(gam_net *n, const float *dout) {
     if (!n || !dout) return -1;
     const NetDims &d = n->d;
-    const int cells = d.lo + 16 * d.ntile - (d.lo & ~7);
-    const int steps = std::max(1, (cells + 64 * 4 * WG_BLOCKS - 1) / (64 * 4 * WG_BLOCKS));   // 64-cell steps per wave
-    const int nblk = (cells + 256 * steps - 1) / (256 * steps);
-    auto wgrad = [&](auto mt, auto nt, const u16 *gT, const u16 *aT, int l) {
+    const dim3 wb(conv_blocks(n, WG_BLOCKS));
+    auto wgrad = [&](auto mt, auto nt, const u16 *g, const u16 *a, int l) {
         constexpr int MT = decltype(mt)::value, NT = decltype(nt)::value;
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wgrad<MT, NT>), dim3(3 * nblk), 256, 0, n->stream, d, gT, aT, steps, n->ws);
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wreduce<MT, NT>), dim3((27 * MT * NT * 256 + MT * 16 + 255) / 256), 256, 0, n->stream,
-                           (const float *)n->ws, nblk, kCo[l], kCi[l], n->g + woff(l), n->g + boff(l));
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wgrad<MT, NT>), wb, 512, 0, n->stream, d, g, a, n->ws);
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_wreduce<MT, NT>), dim3((27 * MT * NT * 256 + MT * 16 + 63) / 64), 256, 0, n->stream,
+                           (const float *)n->ws, (int)wb.x, kCo[l], kCi[l], n->g + woff(l), n->g + boff(l));
     };
     const std::integral_constant<int, 1> one;
     const std::integral_constant<int, 2> two;
-    hipLaunchKernelGGL(k_dout, dim3((d.nc + 255) / 256), 256, 0, n->stream, d, dout, n->gr[0], n->grT[0]);
+    hipLaunchKernelGGL(k_dout, dim3((d.nc + 255) / 256), 256, 0, n->stream, d, dout, n->gr[0]);
     // layer 2 (linear, 8 outputs padded to 16)
-    wgrad(one, two, n->grT[0], n->actT[2], 2);
+    wgrad(one, two, n->gr[0], n->act[2], 2);
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_conv<32, 32, 2>), conv_grid(n, 32), 256, 0, n->stream, d, (const u16 *)n->gr[0], (const u16 *)n->Wb[2],
-                       (const float *)nullptr, (const u16 *)n->actT[2], n->gr[1], n->grT[1], (float *)nullptr);
+                       (const float *)nullptr, (const u16 *)n->act[2], n->gr[1], (float *)nullptr);
     // layer 1
-    wgrad(two, two, n->grT[1], n->actT[1], 1);
+    wgrad(two, two, n->gr[1], n->act[1], 1);
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_conv<32, 32, 2>), conv_grid(n, 32), 256, 0, n->stream, d, (const u16 *)n->gr[1], (const u16 *)n->Wb[1],
-                       (const float *)nullptr, (const u16 *)n->actT[1], n->gr[0], n->grT[0], (float *)nullptr);
+                       (const float *)nullptr, (const u16 *)n->act[1], n->gr[0], (float *)nullptr);
     // layer 0 (input gradient not needed)
-    wgrad(two, one, n->grT[0], n->actT[0], 0);
+    wgrad(two, one, n->gr[0], n->act[0], 0);
     NCHK(n, hipGetLastError());
     return 0;
 }
