@@ -670,7 +670,7 @@ extern "C" int gam_set_clock(gam_handle *h, const gam_clock *c) {
     DClock &d = *h->clk_host;
     d.t = c->t; d.dt = c->dt; d.dt0 = c->dt0; d.stime = c->stateTime; d.otime = c->oStateTime;
     d.ts = c->ts; d.status = c->status; d.dt0_after = c->dt0_after; d.ncpr = c->ncpr; d.cpr_pending = 0;
-    d.halt = 0;
+    d.halt = d.halted = 0;
     HIPCHK(h, hipMemcpy(h->clk, h->clk_host, sizeof(DClock), hipMemcpyHostToDevice));
     return 0;
 }
@@ -962,13 +962,29 @@ static int celldt(gam_handle *h, const void *Gas, const void *B) {
     return h->prec ? launch_celldt<float>(h, Gas, B) : launch_celldt<double>(h, Gas, B);
 }
 
+static bool all_periodic(const gam_handle *h) {
+    for (int f = 0; f < 6; f++) if (h->bct[f] != GAM_BC_PERIODIC) return false;
+    return true;
+}
+
+// Whether the BCs after a fused step are one pass over all ghosts (k_bc_b2f).
+static bool bc_one_pass(const gam_handle *h) { return !h->mp.do25D && all_periodic(h); }
+
+// Ghost layers that the update leaves out on either side: where k_bc_b2f follows, all
+// but the one that CalcDT reads.  Along k, and in the FP64 columns along j; rows stay whole:
+// FP64 256 x 256 x 4 block 64 -> 50 us, 128^3 236 -> 226 (238 with the i ghosts left
+// out as well, which moves the rows off their lines; so does j in FP32, one
+// cell per thread in order: 256^3 0.92 -> 0.99 ms).
+static int update_rim(const gam_handle *h, int fuse_dt) { return fuse_dt && bc_one_pass(h) && !h->ring.on ? h->gv.nG - 1 : 0; }
+
 // k_update's launch box: (i, j, column of update_kc cells in k); FP64: 2 waves per SIMD
-static int update_kc(const gam_handle *h) {
-    return h->prec ? 1 : col_len(h->gv.Nk, (long)(h->pack_share * h->gv.Ni * h->gv.Nj), UPDATE_KC, 2 * 65536);
+static int update_kc(const gam_handle *h, int rim) {
+    return h->prec ? 1 : col_len(h->gv.Nk - 2 * rim, (long)(h->pack_share * h->gv.Ni * (h->gv.Nj - 2 * rim)), UPDATE_KC, 2 * 65536);
 }
-static int update_blocks(const gam_handle *h) {
-    return tile_blocks(h->tile[ST_UPDATE], h->gv.Ni, h->gv.Nj, cdiv(h->gv.Nk, update_kc(h)));
+static int update_blocks(const gam_handle *h, int rim) {
+    return tile_blocks(h->tile[ST_UPDATE], h->gv.Ni, h->gv.Nj - (h->prec ? 0 : 2 * rim), cdiv(h->gv.Nk - 2 * rim, update_kc(h, rim)));
 }
+static int update_blocks_max(const gam_handle *h, const Tile &t) { return tile_blocks(t, h->gv.Ni, h->gv.Nj, h->gv.Nk); }
 
 // blocks of k_celldt_rows (DT box cells of the ring band), 0 without rings
 static int ring_dt_blocks(const gam_handle *h) {
@@ -1262,31 +1278,32 @@ static int advance_t(gam_handle *h, int fuse_dt) {
     }
     {
         StageTimer t(h, ST_UPDATE);
-        dim3 gr(update_blocks(h));
+        const int rim = update_rim(h, fuse_dt);
+        dim3 gr(update_blocks(h, rim));
         const Tile tu = h->tile[ST_UPDATE];
         const R *nGas = P<R>(h->Gas[S]), *nB = P<R>(h->B[S]), *Flx = P<R>(h->Flx);
         R *oGas = P<R>(h->Gas[O]), *oB = P<R>(h->B[O]);
-        const int skip = h->ring.on ? h->ring.nring + 3 : 0, kcu = update_kc(h);
+        const int skip = h->ring.on ? h->ring.nring + 3 : 0, kcu = update_kc(h, rim);
         // FP64: the k-column kernel; FP32 bulk: one cell per thread
         if constexpr (sizeof(R) == sizeof(double)) {
             if (m.doMHD) {
-                if (m.doBoris) PLAUNCH(h, (k_update_col<1, 1, R>), (b_update_col<1, 1, R>), gr, 256, g, tu, m, h->bgv, h->clk, nGas, nB, Flx, h->mag[O], oGas, oB, h->partial, skip, kcu);
-                else PLAUNCH(h, (k_update_col<0, 1, R>), (b_update_col<0, 1, R>), gr, 256, g, tu, m, h->bgv, h->clk, nGas, nB, Flx, h->mag[O], oGas, oB, h->partial, skip, kcu);
+                if (m.doBoris) PLAUNCH(h, (k_update_col<1, 1, R>), (b_update_col<1, 1, R>), gr, 256, g, tu, m, h->bgv, h->clk, nGas, nB, Flx, h->mag[O], oGas, oB, h->partial, skip, rim, kcu);
+                else PLAUNCH(h, (k_update_col<0, 1, R>), (b_update_col<0, 1, R>), gr, 256, g, tu, m, h->bgv, h->clk, nGas, nB, Flx, h->mag[O], oGas, oB, h->partial, skip, rim, kcu);
             } else {
-                PLAUNCH(h, (k_update_col<0, 0, R>), (b_update_col<0, 0, R>), gr, 256, g, tu, m, h->bgv, h->clk, nGas, nB, Flx, h->mag[O], oGas, oB, h->partial, skip, kcu);
+                PLAUNCH(h, (k_update_col<0, 0, R>), (b_update_col<0, 0, R>), gr, 256, g, tu, m, h->bgv, h->clk, nGas, nB, Flx, h->mag[O], oGas, oB, h->partial, skip, rim, kcu);
             }
         } else {
           if (m.doMHD) {
-            if (m.doBoris) PLAUNCH(h, (k_update<1, 1, R>), (b_update<1, 1, R>), gr, 256, g, tu, m, h->bgv, h->clk, nGas, nB, Flx, h->mag[O], oGas, oB, h->partial, skip);
-            else PLAUNCH(h, (k_update<0, 1, R>), (b_update<0, 1, R>), gr, 256, g, tu, m, h->bgv, h->clk, nGas, nB, Flx, h->mag[O], oGas, oB, h->partial, skip);
+            if (m.doBoris) PLAUNCH(h, (k_update<1, 1, R>), (b_update<1, 1, R>), gr, 256, g, tu, m, h->bgv, h->clk, nGas, nB, Flx, h->mag[O], oGas, oB, h->partial, skip, rim);
+            else PLAUNCH(h, (k_update<0, 1, R>), (b_update<0, 1, R>), gr, 256, g, tu, m, h->bgv, h->clk, nGas, nB, Flx, h->mag[O], oGas, oB, h->partial, skip, rim);
         } else {
-            PLAUNCH(h, (k_update<0, 0, R>), (b_update<0, 0, R>), gr, 256, g, tu, m, h->bgv, h->clk, nGas, nB, Flx, h->mag[O], oGas, oB, h->partial, skip);
+            PLAUNCH(h, (k_update<0, 0, R>), (b_update<0, 0, R>), gr, 256, g, tu, m, h->bgv, h->clk, nGas, nB, Flx, h->mag[O], oGas, oB, h->partial, skip, rim);
           }
         }
     }
     // CopyState State->oState is the buffer swap
     h->s = O;
-    h->fused_np = update_blocks(h);
+    h->fused_np = update_blocks(h, update_rim(h, fuse_dt));
     if (h->ring.on) {   // mhdgroup.F90:69-74; CalcDT then sees the averaged rings
         ring_average<R>(h);
         if (fuse_dt) {   // the ring band's CFL minima after k_update's
@@ -1308,11 +1325,6 @@ static int advance_t(gam_handle *h, int fuse_dt) {
 }
 static int advance(gam_handle *h, int fuse_dt) {
     return h->prec ? advance_t<float>(h, fuse_dt) : advance_t<double>(h, fuse_dt);
-}
-
-static bool all_periodic(const gam_handle *h) {
-    for (int f = 0; f < 6; f++) if (h->bct[f] != GAM_BC_PERIODIC) return false;
-    return true;
 }
 
 // BCs on State, in the reference's order (INI, OUTI, INJ, OUTJ, INK, OUTK);
@@ -1543,7 +1555,7 @@ extern "C" int gam_set_ring(gam_handle *h, int nring, const int *nch) {
     h->ring.on = 1;
     h->ring.nring = nring;
     for (int r = 0; r < GAM_RING_MAX; r++) h->ring.nch[r] = r < nring ? nch[r] : 0;
-    return ensure_partial(h, update_blocks(h) + ring_dt_blocks(h));
+    return ensure_partial(h, update_blocks_max(h, h->tile[ST_UPDATE]) + ring_dt_blocks(h));
 }
 
 extern "C" int gam_get_ring(gam_handle *h, int *nring, int *nch) {
@@ -1559,10 +1571,10 @@ template <typename R>
 static int bcs_t(gam_handle *h, bool shell) {
     const int S = h->s;
     const GVT<R> &g = view<R>(h);
-    if (shell && !h->mp.do25D && all_periodic(h)) {
+    if (shell && bc_one_pass(h)) {
         StageTimer t(h, ST_BC);
         PLAUNCH(h, (k_bc_b2f<R>), (b_bc_b2f<R>), grid1(bc_shell_count(bc_shell(g.Ni, g.Nj, g.Nk, g.Nip, g.Njp, g.Nkp, g.nG, 7, 0))),
-                256, g, h->clk, P<R>(h->Gas[S]), h->mag[S], P<R>(h->B[S]));
+                256, g, h->clk, P<R>(h->Gas[S]), h->mag[S], P<R>(h->B[S]), P<R>(h->Gas[1 - S]));
         HIPCHK(h, hipGetLastError());
         return 0;
     }
@@ -2032,7 +2044,7 @@ extern "C" int gam_set_tile(gam_handle *h, int stage, int ti, int tj, int tk, in
     if (rc) return rc;
     const Tile t = {ti, tj, tk, fast};
     if (stage == ST_UPDATE) {   // one block minimum per update block, then the ring band's
-        rc = ensure_partial(h, tile_blocks(t, h->gv.Ni, h->gv.Nj, cdiv(h->gv.Nk, update_kc(h))) + ring_dt_blocks(h));
+        rc = ensure_partial(h, update_blocks_max(h, t) + ring_dt_blocks(h));
         if (rc) return rc;
     }
     h->tile[stage] = t;

@@ -37,6 +37,7 @@ struct DClock {
     double limDT0, limCPR;
     int ts, status, dt0_after, fixedTimestep, doCPR, halt;
     int cpr_pending, ncpr;   // CalcDT asked for a CPR repair this step; repairs so far
+    int halted, pad;         // CalcDT halted in this step: its BCs do not run (b_bc_b2f)
 };
 
 // Per-cell / per-face quantities the stencil kernels read, computed once per

@@ -1313,11 +1313,12 @@ __device__ __forceinline__ void b_update(const unsigned vb, GVT<R> g, Tile t, MP
                                                 const R *__restrict__ nGas, const R *__restrict__ nB,
                                                 const R *__restrict__ Flx, const double *__restrict__ magNew,
                                                 R *__restrict__ oGas, R *__restrict__ oB,
-                                                double *__restrict__ partial, int skip_nb) {
+                                                double *__restrict__ partial, int skip_nb, int rim) {
     if (clk->halt) return;
     double dtl = GAM_HUGE;
     int i, j, k;
-    if (tile_pos(vb, t, g.Ni, g.Nj, g.Nk, i, j, k)) {
+    if (tile_pos(vb, t, g.Ni, g.Nj, g.Nk - 2 * rim, i, j, k)) {
+        k += rim;
         const int idx = ci(g, i, j, k);
         const size_t nc = g.nc;
         R U[5];   // the update computes in the bulk type (FP64 step: double)
@@ -1366,8 +1367,8 @@ __global__ void __launch_bounds__(256) k_update(GVT<R> g, Tile t, MP m, BGV bg, 
                                                 const R *__restrict__ nGas, const R *__restrict__ nB,
                                                 const R *__restrict__ Flx, const double *__restrict__ magNew,
                                                 R *__restrict__ oGas, R *__restrict__ oB,
-                                                double *__restrict__ partial, int skip_nb) {
-    b_update<BORIS, MHD, R>(blockIdx.x, g, t, m, bg, clk, nGas, nB, Flx, magNew, oGas, oB, partial, skip_nb);
+                                                double *__restrict__ partial, int skip_nb, int rim) {
+    b_update<BORIS, MHD, R>(blockIdx.x, g, t, m, bg, clk, nGas, nB, Flx, magNew, oGas, oB, partial, skip_nb, rim);
 }
 
 // k_update walking kc <= UPDATE_KC cells up a k column per thread, reading each K
@@ -1378,11 +1379,12 @@ __device__ __forceinline__ void b_update_col(const unsigned vb, GVT<R> g, Tile t
                                                 const R *__restrict__ nGas, const R *__restrict__ nB,
                                                 const R *__restrict__ Flx, const double *__restrict__ magNew,
                                                 R *__restrict__ oGas, R *__restrict__ oB,
-                                                double *__restrict__ partial, int skip_nb, int kc) {
+                                                double *__restrict__ partial, int skip_nb, int rim, int kc) {
     if (clk->halt) return;
     double dtl = GAM_HUGE;
     int i, j, kb;
-    if (tile_pos(vb, t, g.Ni, g.Nj, cdiv(g.Nk, kc), i, j, kb)) {
+    if (tile_pos(vb, t, g.Ni, g.Nj - 2 * rim, cdiv(g.Nk - 2 * rim, kc), i, j, kb)) {
+        j += rim;
         const size_t nc = g.nc;
         const int a0 = g.nG;
         const bool act_ij = i >= a0 && i < a0 + g.Nip && j >= a0 && j < a0 + g.Njp;
@@ -1392,8 +1394,8 @@ __device__ __forceinline__ void b_update_col(const unsigned vb, GVT<R> g, Tile t
         bool haveF = false;
 #pragma unroll 1
         for (int kk = 0; kk < kc; kk++) {
-            const int k = kb * kc + kk;
-            if (k >= g.Nk) break;
+            const int k = rim + kb * kc + kk;
+            if (k >= g.Nk - rim) break;
             const int idx = ci(g, i, j, k);
             double U[5], Bn[3] = {0, 0, 0};
 #pragma unroll
@@ -1447,8 +1449,8 @@ __global__ void __launch_bounds__(256) k_update_col(GVT<R> g, Tile t, MP m, BGV 
                                                 const R *__restrict__ nGas, const R *__restrict__ nB,
                                                 const R *__restrict__ Flx, const double *__restrict__ magNew,
                                                 R *__restrict__ oGas, R *__restrict__ oB,
-                                                double *__restrict__ partial, int skip_nb, int kc) {
-    b_update_col<BORIS, MHD, R>(blockIdx.x, g, t, m, bg, clk, nGas, nB, Flx, magNew, oGas, oB, partial, skip_nb, kc);
+                                                double *__restrict__ partial, int skip_nb, int rim, int kc) {
+    b_update_col<BORIS, MHD, R>(blockIdx.x, g, t, m, bg, clk, nGas, nB, Flx, magNew, oGas, oB, partial, skip_nb, rim, kc);
 }
 
 // Stand-alone CellDT min over the DT box (CalcDT without the fused update)
@@ -1482,6 +1484,7 @@ __global__ void __launch_bounds__(256) k_celldt(GVT<R> g, MP m, BGV bg, const DC
 // when advance != 0, then CalcDT's checks and clamps (step.F90:103-166).
 __device__ __forceinline__ void clock_advance(DClock *clk, double dtMin, int advance, int calc) {
     clk->cpr_pending = 0;
+    clk->halted = 0;
     if (advance) {
         clk->otime = clk->stime;
         clk->stime = clk->stime + clk->dt;
@@ -1510,7 +1513,7 @@ __device__ __forceinline__ void clock_advance(DClock *clk, double dtMin, int adv
     if (clk->dt0 > GAM_TINY && dt > (10.0 * clk->dt0)) dt = 10.0 * clk->dt0;
     clk->dt = dt;
     clk->status = status;
-    if (status) clk->halt = 1;   // the reference stops here (step.F90:138-154); the host decides
+    if (status) clk->halt = clk->halted = 1;   // the reference stops here (step.F90:138-154); the host decides
     // console-output dt0 capture (output.F90:57-59) at the configured cadence
     if (clk->dt0_after > 0 && clk->ts >= clk->dt0_after && clk->dt0 < GAM_TINY) clk->dt0 = clk->dt;
 }
@@ -1523,7 +1526,10 @@ __device__ __forceinline__ void b_dtfinal(const unsigned vb, DClock *clk, DClock
                                           int advance, int calc) {
     static_assert(sizeof(DClock) % sizeof(double) == 0 && sizeof(DClock) / sizeof(double) <= 64, "one word per lane");
     constexpr unsigned NW = sizeof(DClock) / sizeof(double);
-    if (clk->halt) return;
+    if (clk->halt) {   // in an earlier step
+        if (threadIdx.x == 0) clk->halted = 0;
+        return;
+    }
 #ifdef GAM_EMU
     if (threadIdx.x != 0) return;
     double dtMin = GAM_HUGE;
@@ -1733,16 +1739,28 @@ __global__ void __launch_bounds__(256) k_bc(GVT<R> g, const DClock *__restrict__
 // no thread writes those, so the pass needs none of its own results.  (Bxyz of the active
 // cells: see k_b2f_shell.)  Two launches before: 0.063 + 0.100 ms at 256^3 FP64,
 // 6.8 + 3.8 us on a 32x32x4 box -> 0.145 ms and 8-10 us, and one launch less.
+// nGas: Gas n.  The update before this pass skips the ghost cells that it fills (rim);
+// in the step that halts, whose BCs do not run, it writes the update's values there.
 template <typename R>
 __device__ __forceinline__ void b_bc_b2f(const unsigned vb, GVT<R> g, const DClock *__restrict__ clk, R *__restrict__ Gas,
-                                         double *__restrict__ mag, R *__restrict__ B) {
+                                         double *__restrict__ mag, R *__restrict__ B, const R *__restrict__ nGas) {
     b_bc<R>(vb, g, clk, 0, 7, Gas, mag, (R *)nullptr);
     const BcShell sh = bc_shell(g.Ni, g.Nj, g.Nk, g.Nip, g.Njp, g.Nkp, g.nG, 7, 0);
     int i, j, k;
-    if (clk->halt || !bc_shell_pos(sh, (long)vb * blockDim.x + threadIdx.x, i, j, k)) return;
+    if ((clk->halt && !clk->halted) || !bc_shell_pos(sh, (long)vb * blockDim.x + threadIdx.x, i, j, k)) return;
     if (i >= g.Ni || j >= g.Nj || k >= g.Nk) return;
     const int a0 = g.nG;
     const size_t nc = g.nc, nf = g.nf;
+    if (clk->halted) {   // no BCs: what the update would have left in the ghost cells
+        const int c = ci(g, i, j, k);
+        double b[3];
+        cell_bxyz(g, mag, i, j, k, b);
+#pragma unroll
+        for (int v = 0; v < 5; v++) Gas[nc * v + c] = nGas[nc * v + c];
+#pragma unroll
+        for (int x = 0; x < 3; x++) B[nc * x + c] = R(b[x]);
+        return;
+    }
     const int ic = pmap_c(i, a0, g.Nip), jc = pmap_c(j, a0, g.Njp), kc = pmap_c(k, a0, g.Nkp);
     // the lower and upper face of the pair along its normal
     const int il = pmap_f(i, a0, g.Nip), iu = pmap_f(i + 1, a0, g.Nip);
@@ -1759,8 +1777,8 @@ __device__ __forceinline__ void b_bc_b2f(const unsigned vb, GVT<R> g, const DClo
 }
 template <typename R>
 __global__ void __launch_bounds__(256) k_bc_b2f(GVT<R> g, const DClock *__restrict__ clk, R *__restrict__ Gas,
-                                                double *__restrict__ mag, R *__restrict__ B) {
-    b_bc_b2f<R>(blockIdx.x, g, clk, Gas, mag, B);
+                                                double *__restrict__ mag, R *__restrict__ B, const R *__restrict__ nGas) {
+    b_bc_b2f<R>(blockIdx.x, g, clk, Gas, mag, B, nGas);
 }
 
 // One face's non-periodic BC, restating bcs.F90: zeroGrad_{i,o}bc{I,J,K}

@@ -136,7 +136,33 @@ def test_large_block_of_periods(mkw):
                 assert relerr(y[act], x[act]) <= tol
 
 
-EMU_EXPR = {"all": "one_step and (thin or 25d) or volumes", "asan": "one_step and 25d or volumes", "cols": "one_step and not ragged"}
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("n", [(9, 40, 2), (17, 6, 30)])
+def test_ghosts_of_a_halted_step(n, precision):
+    """A periodic fused step whose CalcDT halts leaves the ghost cells that its update
+    skips as the separate calls leave them: the same copies and sums, the same bits."""
+    from kaiju_amd.gamera import GamApp
+    say(f"[halt] {n} precision {precision}")
+    out = []
+    for fused in (True, False):
+        with GamApp(configs.blast_wave(n, precision=precision)) as app:
+            app.InitModel()
+            assert app.steps(2) == 0
+            st = app.get_state(0)
+            gas, c = st["Gas"], tuple(app.nG + q // 2 for q in n)
+            gas[c + (1,)] = 1e12 * gas[c + (0,)]
+            gas[c + (4,)] += 0.5 * 1e24 * gas[c + (0,)]
+            app.put_state(0, st["time"], gas, st["magFlux"], st["Bxyz"])
+            ts = app.Model.ts
+            assert (app.steps(3) if fused else app.stepGamera(fused=False)) != 0
+            assert app.Model.ts == ts + 1
+            out.append(app.get_state(0))
+    for q in ("Gas", "magFlux", "Bxyz"):
+        assert np.array_equal(out[0][q], out[1][q], equal_nan=True), q
+
+
+EMU_EXPR = {"all": "one_step and (thin or 25d) or volumes or halted", "asan": "one_step and 25d or volumes or halted", "cols": "one_step and not ragged"}
 
 
 @pytest.mark.parametrize("kind", list(EMU_EXPR))
