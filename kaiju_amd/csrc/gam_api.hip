@@ -2082,11 +2082,11 @@ extern "C" int gam_stage_bytes(gam_handle *h, int stage, double *bytes) {
         const double S = h->mp.do25D ? G : (double)b2f_shell_count(g.Ni, g.Nj, g.Nk, g.Nip, g.Njp, g.Nkp);
         b = S * 3; d = S * (3 + 9 + 3 + 1); break;
     }
-    case ST_MOM2FACE: b = G * (3 + 1 + 9); break;                                 // VdV, vol -> Vf (9)
-    case ST_EMF_I: case ST_EMF_J: case ST_EMF_K: {   // Vf (dT1), rho ; face, bn, bh (dT1, dT2), Te, Teb, edge -> E
+    case ST_MOM2FACE: b = G * (3 + 1 + (emf_cols(h) ? 3 : 9)); break;            // VdV, vol -> Vf (9, K faces 3)
+    case ST_EMF_I: case ST_EMF_J: case ST_EMF_K: {   // Vf (dT1) or VdV and vol, rho ; face, bn, bh (dT1, dT2), Te, Teb, edge -> E
         const int e = stage - ST_EMF_I;
         const double nEd = (double)(g.Nip + (e != 0)) * (g.Njp + (e != 1)) * (g.Nkp + (e != 2));
-        b = G * (3 + 1) + nEd * (2 + 2 + 2 + 6 + 4 + 1 + 1); break;
+        b = G * (3 + 1 + (e != 1 && emf_cols(h))) + nEd * (2 + 2 + 2 + 6 + 4 + 1 + 1); break;
     }
     case ST_FLUX_I: b = (G * (5 + 5 + 3 + 3 + 1)) + nI * (9 + 1 + 1 + 8); d = h->bgv.on ? nI * 4 : 0; break;
     case ST_FLUX_J: b = (G * (5 + 5 + 3 + 3 + 1)) + nJ * (9 + 1 + 1 + 8); d = h->bgv.on ? nJ * 4 : 0; break;
@@ -2094,7 +2094,12 @@ extern "C" int gam_stage_bytes(gam_handle *h, int stage, double *bytes) {
     case ST_CT: d = F * (3 + 3); b = G * 3; break;
     case ST_UPDATE:   // Gas n, fluxes (8 per direction), di/dj/dk -> Gas, Bxyz (b) ; magFlux new, xfc, xyzcc, vol (d)
         b = G * (5 + 24 + 3 + 5 + 3 + (h->mp.doBoris ? 3 : 0)); d = F * (3 + 9) + G * (3 + 1);
-        if (h->bgv.on) d += G * (3 + 3); break;                                  // dpB0, B0
+        if (h->bgv.on) d += G * (3 + 3);                                         // dpB0, B0
+        if (const int rim = update_rim(h, 1)) {   // the fused step's box
+            const double f = (1.0 - 2.0 * rim / g.Nk) * (h->prec ? 1.0 : 1.0 - 2.0 * rim / g.Nj);
+            b *= f; d *= f;
+        }
+        break;
     case ST_BC: b = 2.0 * (G - nA) * 5; d = 2.0 * (F - nE) * 3; break;
     case ST_CELLDT: b = G * (5 + 3 + 3); break;
     default: b = 0;

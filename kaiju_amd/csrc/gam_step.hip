@@ -6,12 +6,14 @@
 //                                                    mhdgroup.F90:25-31,445-616
 //   k_b2f       (G)   H.Bxyz = bFlux2Fld(H.magFlux)  gridutils.F90:281-301,648-680
 //   k_vf        (G)   Mom2Face for the 3 sweeps      fields.F90:110-179,235-285
-//   k_emf<d>    (E)   edge EMFs, one direction each  fields.F90:186-226,288-517
+//   k_emf<d>, k_emf_jcol, k_emf_col (E)  edge EMFs, one direction each
+//                                                    fields.F90:186-226,288-517
 //   k_flux, k_flux_col (I)  interface fluxes, 3 launches  stress.F90:84-128,204-599
 //   k_ct        (F)   O.magFlux = E2Flux(S.magFlux)  fields.F90:18-51
 //   k_update    (G)   Flux2Deltas + Reynolds + Bxyz + Maxwell/Boris + CellDT min
 //                                                    stress.F90:152-194, mhdgroup.F90:79-442,
 //                                                    gridutils.F90:49-106
+// (small blocks: k_b2f and k_vf, and the EMFs and fluxes, in one launch each)
 //   k_dtfinal   (1)   time update + CalcDT checks    gamapp.F90:112-114, step.F90:58-168
 //   k_bc_b2f    (F)   periodic ghost fill and the ghosts' Bxyz = bFlux2Fld
 //                                                    bcs.F90:279-450, gamapp.F90:89

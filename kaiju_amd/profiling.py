@@ -30,7 +30,8 @@ STAGE_OF = [
     ("k_predict", "predictor"), ("k_bc_b2f", "bcs"), ("k_b2f_vf", "mom2face"), ("k_emf_flux", "flux_i"), ("k_b2f_shell", "bflux_post"), ("k_b2f_rows", "ring"),
     ("k_b2f", "bflux_half"), ("k_ring_", "ring"), ("k_pole_e", "ring"), ("k_fix_e", "ring"),
     ("k_celldt_rows", "celldt"), ("k_bc_wind", "bcs"), ("k_wind_", "bcs"),
-    ("k_vf", "mom2face"), ("k_emf_jcol", "emf_j"), ("k_emf<0", "emf_i"), ("k_emf<1", "emf_j"), ("k_emf<2", "emf_k"),
+    ("k_vf", "mom2face"), ("k_emf_jcol", "emf_j"), ("k_emf<0", "emf_i"), ("k_emf<2", "emf_k"),
+    ("k_emf_col<0", "emf_i"), ("k_emf_col<2", "emf_k"),
     ("k_flux<0", "flux_i"), ("k_flux_col<1", "flux_j"), ("k_flux_col<2", "flux_k"),
     ("k_ct", "ct_update"), ("k_update", "update"),
     ("k_dtfinal", "dt_final"), ("k_bc", "bcs"), ("k_celldt", "celldt"),
@@ -169,13 +170,13 @@ BF16_PEAK_TFLOPS = 2500.0
 # per network kernel: multiply-adds per computed cell and per tap (real channels:
 # 8 -> 32 -> 32 -> 8); the backward-data launches alternate between the output
 # layer's (8 -> 32) and the hidden layer's (32 -> 32) and are averaged
-NET_MACS = {"k_conv<32, 0, 4>": 32 * 8, "k_conv<32, 0, 1>": 32 * 32, "k_conv<16, 1, 1>": 8 * 32,
-            "k_conv<32, 2, 1>": (8 * 32 + 32 * 32) / 2, "k_wgrad<32, 2>": 32 * 32, "k_wgrad<16, 2>": 8 * 32,
-            "k_wgrad<32, 1>": 32 * 8}
-NET_ROLE = {"k_conv<32, 0, 4>": "forward, layer 1 (8 -> 32, 4 taps per K)", "k_conv<32, 0, 1>": "forward, layer 2 (32 -> 32)",
-            "k_conv<16, 1, 1>": "forward, layer 3 (32 -> 8)", "k_conv<32, 2, 1>": "backward data, layers 3 and 2",
-            "k_wgrad<32, 2>": "weight gradient, layer 2", "k_wgrad<16, 2>": "weight gradient, layer 3",
-            "k_wgrad<32, 1>": "weight gradient, layer 1"}
+NET_MACS = {"k_conv<8, 32, 0>": 32 * 8, "k_conv<32, 32, 0>": 32 * 32, "k_conv<32, 16, 1>": 8 * 32,
+            "k_conv<32, 32, 2>": (8 * 32 + 32 * 32) / 2, "k_wgrad<2, 2>": 32 * 32, "k_wgrad<1, 2>": 8 * 32,
+            "k_wgrad<2, 1>": 32 * 8}
+NET_ROLE = {"k_conv<8, 32, 0>": "forward, layer 1 (8 -> 32, 4 taps per K)", "k_conv<32, 32, 0>": "forward, layer 2 (32 -> 32)",
+            "k_conv<32, 16, 1>": "forward, layer 3 (32 -> 8)", "k_conv<32, 32, 2>": "backward data, layers 3 and 2",
+            "k_wgrad<2, 2>": "weight gradient, layer 2", "k_wgrad<1, 2>": "weight gradient, layer 3",
+            "k_wgrad<2, 1>": "weight gradient, layer 1"}
 # inference layers (k_infer): MACs per stored cell, role, and the layer's stored
 # box, the active N^3 block widened by this many cells on every side
 NET_INFER = {"k_infer<8, 32, 0, double>": (32 * 8, "inference, features + layer 1 (FP64 state)", 2),
