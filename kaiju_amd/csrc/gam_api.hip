@@ -1241,7 +1241,7 @@ static int advance_t(gam_handle *h, int fuse_dt) {
     const MP &m = h->mp;
     const int S = h->s, O = 1 - h->s;
     { StageTimer t(h, ST_PREDICT);
-      PLAUNCH(h, (k_predict<R>), (b_predict<R>), grid1(g.nf), 256, g, m, h->clk, P<R>(h->Gas[S]), P<R>(h->Gas[O]),
+      PLAUNCH(h, (k_predict<R>), (b_predict<R>), dim3((m.doMHD ? 3 * xcd_blocks(g.nf) : 0) + xcd_blocks(g.nc)), 256, g, m, h->clk, P<R>(h->Gas[S]), P<R>(h->Gas[O]),
               h->mag[S], h->mag[O], P<R>(h->hGas), P<R>(h->hmag), wkt<R>(h)); }
     const bool merge = merged(h);
     if (merge && m.doMHD) {

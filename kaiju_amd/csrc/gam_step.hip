@@ -191,35 +191,40 @@ static inline int col_len(int L, long cols, int most, long lanes) {
 // sets the clock's trap and pdt/odt (mhdgroup.F90:25-31,459): every thread forms
 // them from the clock, one stores them (a thread that reads the stored otime
 // forms the same odt).
+// Bound by memory: 9 + 11 arrays read and 9 + 18 written, once each.  With all 47 in
+// flight at once (a thread per point, face and cell) it reached 4.8 TB/s; the three
+// face components and the cells one after the other, each XCD on a run of its own, keep
+// 6 and 29 in flight.  ms at 256^3 FP64 / FP32 / 128^3 FP64: 1.51 / 0.87 / 0.185 ->
+// 1.30 / 0.70 / 0.162; faces together 1.33 / 0.73 / 0.168, nontemporal loads of the old state
+// no gain, 2 or 4 points per thread slower.
+__host__ __device__ __forceinline__ unsigned xcd_blocks(int n) { return (unsigned)(cdiv(cdiv(n, 256), 8) * 8); }
 template <typename R>
 __device__ __forceinline__ void b_predict(const unsigned vb, GVT<R> g, MP m, DClock *clk,
                                                  const R *__restrict__ Gas, const R *__restrict__ oGas,
                                                  const double *__restrict__ mag, const double *__restrict__ omag,
                                                  R *__restrict__ hGas, R *__restrict__ hmag, WKT<R> w) {
-    int idx = vb * blockDim.x + threadIdx.x;
-    if (idx >= g.nf || clk->halt) return;
+    const unsigned nfb = m.doMHD ? xcd_blocks(g.nf) : 0, d = nfb ? vb / nfb : 3, ncb = xcd_blocks(g.nc);
+    const bool cells = d >= 3;
+    const unsigned lb = cells ? vb - 3 * nfb : vb - d * nfb, per = (cells ? ncb : nfb) / 8;
+    const int idx = (int)(((lb & 7) * per + (lb >> 3)) * 256 + threadIdx.x);   // a run per XCD
+    if (idx >= (cells ? g.nc : g.nf) || clk->halt) return;
     double otime = clk->otime;
     const double stime = clk->stime, dt = clk->dt;
     if (fabs(otime - stime) < GAM_TINY) otime = stime - dt;
     const double odt = stime - otime, pdt = 0.5 * dt;
-    if (idx == 0) { clk->otime = otime; clk->odt = odt; clk->pdt = pdt; }
+    if (cells && idx == 0) { clk->otime = otime; clk->odt = odt; clk->pdt = pdt; }
     const int nf = g.nf, nc = g.nc;
-    if (m.doMHD) {
-#pragma unroll
-        for (int d = 0; d < 3; d++) {
-            double mn = mag[(size_t)nf * d + idx];
-            double hm = ab2(pdt, mn, omag[(size_t)nf * d + idx], odt);
-            const R hmR = R(hm);
-            hmag[(size_t)nf * d + idx] = hmR;
-            R fa = rmax(g.face[(size_t)nf * d + idx], R(GAM_TINY));
-            w.bh[(size_t)nf * d + idx] = hmR / fa;
-            w.bn[(size_t)nf * d + idx] = (m.doLFMLim ? R(mn) : hmR) / fa;
-        }
+    if (!cells) {
+        const double mn = mag[(size_t)nf * d + idx];
+        const double hm = ab2(pdt, mn, omag[(size_t)nf * d + idx], odt);
+        const R hmR = R(hm);
+        hmag[(size_t)nf * d + idx] = hmR;
+        const R fa = rmax(g.face[(size_t)nf * d + idx], R(GAM_TINY));
+        w.bh[(size_t)nf * d + idx] = hmR / fa;
+        w.bn[(size_t)nf * d + idx] = (m.doLFMLim ? R(mn) : hmR) / fa;
+        return;
     }
-    int i, j, k;
-    decode_f(g, idx, i, j, k);
-    if (i >= g.Ni || j >= g.Nj || k >= g.Nk) return;
-    int c = ci(g, i, j, k);
+    const int c = idx;
     R Q[5], oQ[5], W[5], oW[5], pW[5], pQ[5];
 #pragma unroll
     for (int v = 0; v < 5; v++) { Q[v] = Gas[(size_t)nc * v + c]; oQ[v] = oGas[(size_t)nc * v + c]; }
