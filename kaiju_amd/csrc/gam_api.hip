@@ -967,15 +967,16 @@ static bool all_periodic(const gam_handle *h) {
     return true;
 }
 
-// Whether the BCs after a fused step are one pass over all ghosts (k_bc_b2f).
-static bool bc_one_pass(const gam_handle *h) { return !h->mp.do25D && all_periodic(h); }
+// Whether the BCs after a fused step are one pass over all ghosts (k_bc_b2f).  Not with
+// a ring average, whose field fix (launch_ring_bfix) follows the ghosts' bFlux2Fld.
+static bool bc_one_pass(const gam_handle *h) { return !h->mp.do25D && !h->ring.on && all_periodic(h); }
 
 // Ghost layers that the update leaves out on either side: where k_bc_b2f follows, all
 // but the one that CalcDT reads.  Along k, and in the FP64 columns along j; rows stay whole:
 // FP64 256 x 256 x 4 block 64 -> 50 us, 128^3 236 -> 226 (238 with the i ghosts left
 // out as well, which moves the rows off their lines; so does j in FP32, one
 // cell per thread in order: 256^3 0.92 -> 0.99 ms).
-static int update_rim(const gam_handle *h, int fuse_dt) { return fuse_dt && bc_one_pass(h) && !h->ring.on ? h->gv.nG - 1 : 0; }
+static int update_rim(const gam_handle *h, int fuse_dt) { return fuse_dt && bc_one_pass(h) ? h->gv.nG - 1 : 0; }
 
 // k_update's launch box: (i, j, column of update_kc cells in k); FP64: 2 waves per SIMD
 static int update_kc(const gam_handle *h, int rim) {
