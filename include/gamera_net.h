@@ -46,9 +46,9 @@ int  gam_net_forward(gam_net *n);
 /* Inference only: features of the device state and the three layers in one
  * call, each layer's input staged in LDS per brick.  The output is stored on
  * the cells at least `halo` (>= 3) cells from the grid faces and equals
- * gam_net_forward's there bit for bit; elsewhere it keeps its old values, and
- * the activations kept for gam_net_backward are not all rewritten (train
- * through gam_net_features + gam_net_forward). */
+ * gam_net_forward's there bit for bit; elsewhere it keeps its old values.  The
+ * activations of the last gam_net_forward, which gam_net_backward takes, stay
+ * as they are (train through gam_net_features + gam_net_forward). */
 int  gam_net_infer(gam_net *n, const void *Gas, const void *Bxyz, int precision, int halo);
 /* The hipEvent_t gam_net_infer records after its last kernel (the net's
  * lifetime): hand it to gam_set_correction_wait so that a step on another

@@ -13,8 +13,8 @@
 // A convolution is an implicit GEMM: M = 16 consecutive cells per MFMA, N = 16
 // output channels per tile, K = 32 input channels of one tap per MFMA (of four
 // taps in the first layer).  Output
-// cells cover [lo, lo + 16*ntile) with lo = Ni*Nj + Ni + 1, so every tap's
-// neighbour p + off stays inside the array; cells near the box faces read
+// cells cover [lo, nc - lo) with lo = Ni*Nj + Ni + 1, the cells whose every tap's
+// neighbour p + off lies inside the array; cells near the box faces read
 // wrapped neighbours and are never used (the correction is read on the active
 // box plus one layer only, 4 ghost layers deep).
 #include <hip/hip_runtime.h>
@@ -51,7 +51,7 @@ __host__ __device__ inline float bf2f(u16 b) {
     return f;
 }
 
-struct NetDims { int Ni, Nj, Nk, nc, lo, ntile; };
+struct NetDims { int Ni, Nj, Nk, nc, lo, hi; };   // computed cells [lo, hi)
 
 __device__ __forceinline__ bf16x8 ld8(const u16 *p) {   // 16-byte aligned
     return *reinterpret_cast<const bf16x8 *>(p);
@@ -185,7 +185,7 @@ __device__ __forceinline__ uint4 masked(const uint4 &x, const uint4 &m) {
 // MODE 2: backward data: multiply by the activation's slope at the forward
 //         output (mask > 0: 1, else 1/8), write act_out, NCO = 32
 // Neighbours are those of the flattened cell index (p + off), as at the box faces, whose
-// cells are never used; cells outside [lo, lo + 16 ntile) are not stored.  The results leave
+// cells are never used; cells outside [lo, hi) are not stored.  The results leave
 // through LDS as whole cells.
 // Per launch on a 104^3 grid, A operands from L2 / staged, weights per brick / as now:
 // hidden layer 230 / 151 / 69 us, first 111 / 84 / 49, last 182 / 70 / 43, backward
@@ -205,7 +205,7 @@ k_conv(NetDims d, const u16 *__restrict__ in, const u16 *__restrict__ W, const f
     u16 *sO = reinterpret_cast<u16 *>(sOut);
     float *sF = reinterpret_cast<float *>(sOut);
     const int nbi = (d.Ni + NB_I - 1) / NB_I, nbj = (d.Nj + NB_J - 1) / NB_J, nbk = (d.Nk + NB_K - 1) / NB_K;
-    const int run = brick_run(nbi * nbj * nbk), hi = d.lo + 16 * d.ntile;
+    const int run = brick_run(nbi * nbj * nbk);
     const int b0 = (blockIdx.x & 7) * run, b1 = min(b0 + run, nbi * nbj * nbk), step = gridDim.x >> 3;
     int b = b0 + (blockIdx.x >> 3);
     auto origin = [&](int bb, int &oi, int &oj, int &ok) { oi = NB_I * (bb % nbi); oj = NB_J * ((bb / nbi) % nbj); ok = NB_K * (bb / (nbi * nbj)); };
@@ -263,7 +263,7 @@ k_conv(NetDims d, const u16 *__restrict__ in, const u16 *__restrict__ W, const f
         for (int e = threadIdx.x; e < NB_OC * CH; e += 256) {
             const int oc = e / CH, q = e % CH;
             const int i = oi + oc % NB_I, j = oj + (oc / NB_I) % NB_J, k = ok + oc / (NB_I * NB_J), p = i + d.Ni * (j + d.Nj * k);
-            if (i >= d.Ni || j >= d.Nj || k >= d.Nk || p < d.lo || p >= hi) continue;
+            if (i >= d.Ni || j >= d.Nj || k >= d.Nk || p < d.lo || p >= d.hi) continue;
             if constexpr (MODE == 1) *reinterpret_cast<uint4 *>(out + (size_t)p * 8 + 4 * q) = sOut[e];
             else {
                 uint4 x = sOut[oc * (OS / 8) + q];
@@ -457,7 +457,7 @@ __global__ void __launch_bounds__(256) k_dout(NetDims d, const float *__restrict
     const int p = blockIdx.x * 256 + threadIdx.x;
     if (p >= d.nc) return;
     uint4 v = {0u, 0u, 0u, 0u};
-    if (p >= d.lo && p < d.lo + 16 * d.ntile) {
+    if (p >= d.lo && p < d.hi) {
         float f[8];
 #pragma unroll
         for (int c = 0; c < 8; c++) f[c] = dout[(size_t)p * 8 + c];
@@ -664,10 +664,7 @@ struct gam_net {
     float *w = nullptr, *g = nullptr, *m = nullptr, *v = nullptr;
     u16 *Wf[3] = {}, *Wb[3] = {};
     u16 *act[3] = {}, *inf[2] = {};      // forward: 0 features, 1..2 hidden; inference's hidden
-    // A backward pass takes the last forward's activations, so inference writes inf once
-    // a forward has run.  Before the first one it writes act: the up to 15 cells past the
-    // forward's whole tiles, which no forward stores, then hold inferred values.
-    bool forwarded = false;
+                                         // (a backward pass takes the last forward's)
     u16 *gr[2] = {};                     // gradient ping-pong
     float *out = nullptr;
     float *dbuf = nullptr;               // upstream gradient uploaded from the host
@@ -712,9 +709,8 @@ extern "C" int gam_net_create(int Ni, int Nj, int Nk, gam_net **out) {
     gam_net *n = new gam_net();
     NetDims &d = n->d;
     d.Ni = Ni; d.Nj = Nj; d.Nk = Nk; d.nc = (int)nc;
-    const int O = Ni * Nj + Ni + 1;
-    d.lo = O;
-    d.ntile = (int)((nc - 2L * O) / 16);
+    d.lo = Ni * Nj + Ni + 1;
+    d.hi = d.nc - d.lo;
     auto cleanup = [&](int c) { gam_net_destroy(n); return c; };
     if (hipStreamCreateWithFlags(&n->own, hipStreamNonBlocking) != hipSuccess) return cleanup(-2);
     n->stream = n->own;
@@ -830,7 +826,6 @@ static dim3 conv_grid(const gam_net *n, int cin) { return dim3(conv_blocks(n, ci
 extern "C" int gam_net_forward(gam_net *n) {
     if (!n) return -1;
     const NetDims &d = n->d;
-    n->forwarded = true;
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_conv<8, 32, 0>), conv_grid(n, 8), 256, 0, n->stream, d, (const u16 *)n->act[0], (const u16 *)n->Wf[0],
                        (const float *)(n->w + boff(0)), (const u16 *)nullptr, n->act[1], (float *)nullptr);
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_conv<32, 32, 0>), conv_grid(n, 32), 256, 0, n->stream, d, (const u16 *)n->act[1], (const u16 *)n->Wf[1],
@@ -858,7 +853,7 @@ extern "C" int gam_net_infer(gam_net *n, const void *Gas, const void *B, int pre
             bx[l].nb[a] = (bx[l].n[a] + nb[a] - 1) / nb[a];
         }
     }
-    u16 *h1 = n->forwarded ? n->inf[0] : n->act[1], *h2 = n->forwarded ? n->inf[1] : n->act[2];
+    u16 *h1 = n->inf[0], *h2 = n->inf[1];
     auto grid = [](int cin, const InferBox &b) { return dim3(brick_blocks((long)b.nb[0] * b.nb[1] * b.nb[2], cin == 32 ? NB_STAY : 0x7fffffffL)); };
     if (precision)
         hipLaunchKernelGGL(HIP_KERNEL_NAME(k_infer<8, 32, 0, float>), grid(8, bx[0]), 256, 0, n->stream, d, bx[0], (const u16 *)nullptr,

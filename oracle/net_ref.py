@@ -49,15 +49,15 @@ def bf16(x: np.ndarray) -> np.ndarray:
 
 
 def geometry(Ni: int, Nj: int, Nk: int):
-    """(tap offsets, lo, ntile) of the GPU kernels for a ghost-inclusive box."""
+    """(tap offsets, lo, hi) for a ghost-inclusive box: the computed cells [lo, hi) are
+    those whose 27 neighbours lie inside the flattened array."""
     nc = Ni * Nj * Nk
     O = Ni * Nj + Ni + 1
-    ntile = (nc - 2 * O) // 16
     off = []
     for t in range(TAPS):
         dx, dy, dz = t % 3 - 1, (t // 3) % 3 - 1, t // 9 - 1
         off.append(dx + Ni * (dy + Nj * dz))
-    return np.array(off), O, ntile
+    return np.array(off), O, nc - O
 
 
 def conv(a: np.ndarray, W: np.ndarray, off, rng):
@@ -72,8 +72,8 @@ class NetRef:
     def __init__(self, Ni, Nj, Nk, w: np.ndarray, bf: bool = True):
         self.dims = (Ni, Nj, Nk)
         self.nc = Ni * Nj * Nk
-        self.off, self.lo, self.ntile = geometry(Ni, Nj, Nk)
-        self.rng = np.arange(self.lo, self.lo + 16 * self.ntile)
+        self.off, self.lo, self.hi = geometry(Ni, Nj, Nk)
+        self.rng = np.arange(self.lo, self.hi)
         self.bf = bf
         self.layers = [((bf16(W) if bf else W), b) for W, b in unpack(w)]
 

@@ -76,3 +76,84 @@ def test_inference_leaves_the_forward_activations():
         G.free()
         Bd.free()
     assert np.array_equal(grads[0], grads[1])
+
+
+def _random_state(seed, nc):
+    rng = np.random.default_rng(seed)
+    gas = np.concatenate([rng.uniform(1.0, 2.0, size=(1, nc)), rng.normal(size=(3, nc)), rng.uniform(5.0, 9.0, size=(1, nc))])
+    return gas, rng.normal(size=(3, nc))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dims", [(21, 18, 17), (17, 9, 11), (16, 12, 8)])
+def test_forward_depends_on_its_own_input_only(dims):
+    """A forward pass after other passes and inferences on another state gives the bits
+    that it gives on a new net, on every cell, and so do its gradients; inference (halo 3, the
+    narrowest) gives the forward's output on its box whatever ran before it."""
+    from kaiju_amd.gamera import DeviceArray
+    from kaiju_amd.net import GamNet, init_params
+    nc = int(np.prod(dims))
+    dout = np.random.default_rng(4).normal(size=(nc, 8)).astype(np.float32)
+    say(f"[net] order of calls {dims}")
+    st = []
+    for s in (1, 2):
+        gas, B = _random_state(s, nc)
+        st.append((DeviceArray.of(gas, np.float64), DeviceArray.of(B, np.float64)))
+    box = tuple(slice(3, n - 3) for n in reversed(dims))
+    got = []
+    for other_first in (False, True):
+        with GamNet(*dims) as net:
+            net.set_params(init_params(2, out_scale=1.0))
+            if other_first:
+                g, b = (a.ptr for a in st[0])
+                net.infer(g, b, 0, 3)
+                net.features_from_device(g, b, 0)
+                net.forward()
+                net.infer(g, b, 0, 3)
+            g, b = (a.ptr for a in st[1])
+            net.features_from_device(g, b, 0)
+            net.forward()
+            out = net.get_output()
+            net.zero_grad()
+            net.backward_host(dout)
+            got.append((out, net.get_act(1), net.get_act(2), net.get_params()[1]))
+            net.infer(g, b, 0, 3)
+            o = net.get_output().reshape(*reversed(dims), 8)
+            assert np.array_equal(o[box], out.reshape(*reversed(dims), 8)[box])
+    for a in st:
+        for x in a:
+            x.free()
+    for x, y in zip(*got):
+        assert np.array_equal(x, y)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dims", [(8, 8, 8), (17, 9, 11), (16, 12, 8)])
+def test_every_cell_with_all_its_neighbours_is_computed(dims):
+    """The output and the gradient reach the last cell whose 27 neighbours lie in the
+    array: its output is the reference's (the FP32 sums of the layers reorder 27 x 32 terms,
+    the hidden BF16 roundings flip: 2e-2 of the largest output), and the last layer's
+    bias gradient is the cell's BF16 upstream gradient, exactly."""
+    from kaiju_amd.net import GamNet, init_params
+    nc = int(np.prod(dims))
+    rng = np.random.default_rng(8)
+    w = init_params(2, out_scale=1.0)
+    feat, dout = rng.normal(size=(nc, 8)).astype(np.float32), np.zeros((nc, 8), np.float32)
+    first = dims[0] * dims[1] + dims[0] + 1
+    last = nc - first - 1
+    dout[last] = rng.normal(size=8)
+    ref = net_ref.NetRef(*dims, w)
+    want = ref.forward(feat)
+    say(f"[net] last cell {last} of {dims}")
+    with GamNet(*dims) as net:
+        net.set_params(w)
+        net.set_features(feat)
+        net.forward()
+        out = net.get_output()
+        net.zero_grad()
+        net.backward_host(dout)
+        grad = net.get_params()[1]
+    assert ref.rng[0] == first and ref.rng[-1] == last
+    assert np.abs(out[last] - want[last]).max() <= 2e-2 * np.abs(want).max()
+    assert np.abs(out[last]).max() > 0
+    assert np.array_equal(grad[-8:].astype(np.float64), net_ref.bf16(dout[last]))
