@@ -81,7 +81,8 @@ struct gam_handle {
     int npart = 0;             // blocks of the 1-D CellDT launch
     int pcap = 0;              // capacity of partial (block minima / sums)
     DClock *clk = nullptr;      // device
-    DClock *clk_host = nullptr; // pinned; equals *clk once the stream's work is done (k_dtfinal writes both)
+    DClock *clk_host = nullptr; // pinned; equals *clk after each call, once its stream's work is done: the host writes both, and
+                                 // every sequence of kernels that changes the clock ends with k_dtfinal, which copies it
     std::string err;
     bool timing = false;
     std::vector<PendingEv> pending;

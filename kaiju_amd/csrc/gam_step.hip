@@ -1534,7 +1534,7 @@ __device__ __forceinline__ void b_dtfinal(const unsigned vb, DClock *clk, DClock
     static_assert(sizeof(DClock) % sizeof(double) == 0 && sizeof(DClock) / sizeof(double) <= 64, "one word per lane");
     constexpr unsigned NW = sizeof(DClock) / sizeof(double);
     if (clk->halt) {   // in an earlier step
-        if (threadIdx.x == 0) clk->halted = 0;
+        if (threadIdx.x == 0) clk->halted = host->halted = 0;
         return;
     }
 #ifdef GAM_EMU

@@ -21,19 +21,23 @@ def _cxx():
     return os.environ.get("CXX") or shutil.which("g++") or "g++"
 
 
-def build(asan: bool = False) -> str:
+def build(asan: bool = False, defs: tuple = (), main: str = "") -> str:
+    """The emulation library; defs: macros ("NAME=value") of another build of it.  main: a
+    source of this folder that includes gam_api.hip, built as a program instead."""
     os.makedirs(OUT, exist_ok=True)
-    lib = os.path.join(OUT, "libgamera_emu_asan.so" if asan else "libgamera_emu.so")
-    if os.path.exists(lib) and os.path.getmtime(lib) >= max(os.path.getmtime(s) for s in SRCS):
-        return lib
-    cmd = [_cxx(), "-std=c++17", "-O1", "-g", "-fPIC", "-shared", "-DGAM_EMU", "-ffp-contract=off",
-           "-fno-fast-math", "-x", "c++", "-I", os.path.join(ROOT, "include"), "-I", CSRC, "-I", HERE,
-           os.path.join(CSRC, "gam_api.hip"), "-o", lib + ".tmp"]
+    name = "".join([main[:-4] if main else "libgamera_emu", "_asan" if asan else "", *("_" + d.replace("=", "_") for d in defs)])
+    out = os.path.join(OUT, name if main else name + ".so")
+    src = os.path.join(HERE, main) if main else os.path.join(CSRC, "gam_api.hip")
+    if os.path.exists(out) and os.path.getmtime(out) >= max(os.path.getmtime(s) for s in SRCS + [src]):
+        return out
+    cmd = [_cxx(), "-std=c++17", "-O1", "-g", "-fPIC", *([] if main else ["-shared"]), "-DGAM_EMU", *("-D" + d for d in defs),
+           "-ffp-contract=off", "-fno-fast-math", "-x", "c++", "-I", os.path.join(ROOT, "include"), "-I", CSRC, "-I", HERE,
+           src, "-o", out + ".tmp"]
     if asan:
         cmd[1:1] = ["-fsanitize=address", "-fno-omit-frame-pointer"]
     subprocess.run(cmd, check=True)
-    os.replace(lib + ".tmp", lib)
-    return lib
+    os.replace(out + ".tmp", out)
+    return out
 
 
 def asan_runtime() -> str:
