@@ -1246,15 +1246,15 @@ static int advance_t(gam_handle *h, int fuse_dt) {
       PLAUNCH(h, (k_predict<R>), (b_predict<R>), dim3((m.doMHD ? 3 * xcd_blocks(g.nf) : 0) + xcd_blocks(g.nc)), 256, g, m, h->clk, P<R>(h->Gas[S]), P<R>(h->Gas[O]),
               h->mag[S], h->mag[O], P<R>(h->hGas), P<R>(h->hmag), wkt<R>(h)); }
     const bool merge = merged(h);
+    // a halted block's kernels return at once, and a recorded step has not run: Vf stays as it is
+    if (m.doMHD && !h->rec && !h->capturing && !h->clk_host->halt) h->vf_partial = true;
     if (merge && m.doMHD) {
         launch_b2f_vf<R>(h);
-        h->vf_partial = true;
     } else {
         { StageTimer t(h, ST_BHALF); launch_b2f<R, R>(h, ST_BHALF, P<R>(h->hmag), h->hB); }
         if (m.doMHD) {
             StageTimer t(h, ST_MOM2FACE);
             launch_vf<R>(h, emf_cols(h) ? VF_K : VF_NEEDED);
-            h->vf_partial = true;
         }
     }
     if (h->corr && h->corr_wait) HIPCHK(h, hipStreamWaitEvent(h->stream, h->corr_wait, 0));
@@ -1978,7 +1978,7 @@ extern "C" int gam_graph_launch(gam_graph *g, int replays) {
     }
     hipError_t e;
     for (gam_handle *h : g->hs)
-        if (replays > 0 && h->mp.doMHD) h->vf_partial = true;
+        if (replays > 0 && h->mp.doMHD && !h->clk_host->halt) h->vf_partial = true;
     for (int r = 0; r < replays; r++)
         if ((e = hipGraphLaunch(g->exec, g->stream)) != hipSuccess) return gfail(g, -2, "hipGraphLaunch", e);
     return 0;
