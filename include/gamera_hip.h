@@ -271,7 +271,11 @@ int  gam_get_work(gam_handle *h, int which, double *out);
 
 /* --- instrumentation ------------------------------------------------------ */
 /* Per-stage HIP-event timers, like the reference's Tic/Toc clocks
- * (base/clocks.F90:84-182).  Stage ids are listed by gam_stage_name. */
+ * (base/clocks.F90:84-182).  Stage ids are listed by gam_stage_name.  While they
+ * are on every stage has a launch of its own; a small block's step otherwise runs
+ * bflux_half with mom2face, and the EMFs with the fluxes, in one launch each, and
+ * takes less time than the stages' sum.  A periodic 3D block's bcs hold its
+ * bflux_post. */
 int  gam_set_timing(gam_handle *h, int enable);
 int  gam_get_timing(gam_handle *h, int stage, double *ms_total, int64_t *launches);
 const char *gam_stage_name(int stage);
@@ -282,14 +286,19 @@ int  gam_stage_bytes(gam_handle *h, int stage, double *bytes);
 
 /* --- launch tuning --------------------------------------------------------- */
 /* No counterpart in the reference (its loops are OpenMP over k,j with i
- * vectorised).  The stencil stages (bflux_half, bflux_post, mom2face, emf,
- * flux_i, flux_j, flux_k, update) launch 256-thread blocks that each cover
+ * vectorised).  The stencil stages (bflux_half, bflux_post, mom2face, emf_i,
+ * emf_j, emf_k, flux_i, flux_j, flux_k, update) launch 256-thread blocks that each cover
  * a ti x tj x tk brick of their index box; 'fast' (0 i, 1 j, 2 k) is the axis
  * along which consecutive bricks of one XCD follow each other, and fast = 3
  * gives each block 256 consecutive points of the box in i-fastest order.
  * Adding 4 to fast keeps the hardware's block order (block b to XCD b % 8)
  * instead of giving each XCD one contiguous run of bricks.  Results do not
- * depend on the tile; only speed does.  gam_set_tile returns -1 for other
+ * depend on the tile; only speed does.  A tile applies where its stage has a
+ * launch of its own: in graphs, under stage timers and in the steps of larger
+ * blocks.  A small block's merged launches (bflux_half, mom2face, emf and flux;
+ * hydro: flux) and a periodic 3D block's bflux_post take none, nor do emf_i and
+ * emf_k of a block below the size of the column kernels in a packed graph that
+ * reaches it.  gam_set_tile returns -1 for other
  * stages, ti*tj*tk != 256 or fast outside 0..7.  tile4 receives {ti, tj, tk, fast}. */
 int  gam_set_tile(gam_handle *h, int stage, int ti, int tj, int tk, int fast);
 int  gam_get_tile(gam_handle *h, int stage, int *tile4);

@@ -8,6 +8,10 @@ with the library's stage timers over a few real steps, each stage keeping its
 fastest, and the block's State/oState/clock are restored afterwards -- tuning
 changes no result, only speed (the launch brick never changes a bit of the
 output; tests check this).  Results are cached per (shape, precision, scheme).
+
+The stage timers time every stage's own launch.  Those are what a captured graph replays and
+what a large block steps with; a small block outside a graph runs some stages in merged
+launches, which take no brick (``gam_set_tile``), so for it tuning changes little.
 """
 from __future__ import annotations
 
@@ -17,14 +21,16 @@ from typing import Dict, Optional, Tuple
 
 LINEAR, NOXCD = 3, 4
 
-# candidate bricks per stage (ti, tj, tk, fast); index 0 is the library default
+# candidate bricks per stage (ti, tj, tk, fast); index 0 is the library default (emf_i and
+# emf_k: of their one-edge-per-thread kernels; the last ones are those of the columns that
+# large blocks walk)
 CANDIDATES: Dict[str, list] = {
     "bflux_half": [(256, 1, 1, LINEAR | NOXCD), (256, 1, 1, LINEAR), (64, 4, 1, NOXCD), (32, 4, 2, 2)],
     "bflux_post": [(256, 1, 1, LINEAR | NOXCD), (256, 1, 1, LINEAR), (64, 4, 1, NOXCD), (32, 4, 2, 2)],
     "mom2face": [(256, 1, 1, LINEAR), (256, 1, 1, LINEAR | NOXCD), (16, 4, 4, 0), (32, 4, 2, 2)],
-    "emf_i": [(64, 1, 4, NOXCD), (64, 1, 4, 2), (32, 2, 4, 2), (256, 1, 1, LINEAR | NOXCD)],
+    "emf_i": [(64, 1, 4, NOXCD), (64, 1, 4, 2), (32, 2, 4, 2), (256, 1, 1, LINEAR | NOXCD), (64, 4, 1, NOXCD), (64, 4, 1, 0)],
     "emf_j": [(256, 1, 1, LINEAR | NOXCD), (32, 1, 8, 2), (64, 1, 4, 2), (32, 2, 4, NOXCD)],
-    "emf_k": [(32, 8, 1, 1), (64, 4, 1, 1), (32, 8, 1, 1 | NOXCD), (256, 1, 1, LINEAR | NOXCD)],
+    "emf_k": [(32, 8, 1, 1), (64, 4, 1, 1), (32, 8, 1, 1 | NOXCD), (256, 1, 1, LINEAR | NOXCD), (256, 1, 1, LINEAR)],
     "flux_i": [(256, 1, 1, LINEAR | NOXCD), (256, 1, 1, LINEAR), (32, 8, 1, 0), (64, 4, 1, NOXCD)],
     "flux_j": [(256, 1, 1, LINEAR), (256, 1, 1, LINEAR | NOXCD), (64, 1, 4, 0), (64, 4, 1, 0)],
     "flux_k": [(256, 1, 1, LINEAR), (256, 1, 1, LINEAR | NOXCD), (64, 4, 1, 0), (64, 1, 4, 0)],

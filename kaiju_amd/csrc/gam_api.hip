@@ -304,6 +304,14 @@ static bool tiled_stage(int st) {
     return st == ST_BHALF || st == ST_BPOST || st == ST_MOM2FACE || st == ST_EMF_I || st == ST_EMF_J ||
            st == ST_EMF_K || st == ST_FLUX_I || st == ST_FLUX_J || st == ST_FLUX_K || st == ST_UPDATE;
 }
+static double zones(const gam_handle *h) { return (double)h->gv.Nip * h->gv.Njp * h->gv.Nkp; }
+#ifndef EMF_COL_MIN
+#define EMF_COL_MIN 4e6   // zones from which the I and K edges walk columns (emf_cols)
+#endif
+// I edges: 64 x 4 bricks, whose rows share the j stencils of the face velocities
+static Tile emf_col_tile(const gam_handle *h, int ED) {
+    return ED == 0 ? Tile{64, 4, 1, h->prec ? 0 : TILE_NOXCD} : Tile{256, 1, 1, TILE_LINEAR};
+}
 static void default_tiles(gam_handle *h) {
     // measured best on MI355X for the 256^3 blast wave (ms per launch, stage
     // timers): emf bricks halve their HBM traffic against row-shaped blocks; the
@@ -314,6 +322,8 @@ static void default_tiles(gam_handle *h) {
     h->tile[ST_EMF_I] = {64, 1, 4, TILE_NOXCD};
     h->tile[ST_EMF_J] = {256, 1, 1, TILE_LINEAR | TILE_NOXCD};
     h->tile[ST_EMF_K] = {32, 8, 1, 1};
+    if (zones(h) >= EMF_COL_MIN)
+        for (int ed : {0, 2}) h->tile[ST_EMF_I + ed] = emf_col_tile(h, ed);
     h->tile[ST_UPDATE] = {256, 1, 1, TILE_LINEAR | TILE_NOXCD};
     h->tile[ST_FLUX_I] = {256, 1, 1, TILE_LINEAR | TILE_NOXCD};
     h->tile[ST_FLUX_J] = {256, 1, 1, TILE_LINEAR};   // columns: 64 x 4 bricks within 2%
@@ -1066,14 +1076,8 @@ static void launch_flux(gam_handle *h, int d) {
 // only).  Each of its columns starts with 7 more face velocities, so a launch must have
 // the lanes for long ones.  k_vf and the two EMFs, separate / folded in: 256^3 2.85 /
 // 2.30 ms (FP64), 1.44 / 1.19 (FP32); 9.4 M zones of FP32 0.92 / 0.79; 128^3 0.405 /
-// 0.406 (FP64), so the line lies between the last two.  The launch's own tile choice
-// (gam_set_tile) applies to the separate kernel only.
-#ifndef EMF_COL_MIN
-#define EMF_COL_MIN 4e6
-#endif
-static bool emf_cols(const gam_handle *h) {
-    return h->pack_share * h->gv.Nip * (double)h->gv.Njp * h->gv.Nkp >= EMF_COL_MIN;
-}
+// 0.406 (FP64), so the line lies between the last two.
+static bool emf_cols(const gam_handle *h) { return h->pack_share * zones(h) >= EMF_COL_MIN; }
 
 template <int ED, int RM, int BO, typename R>
 static void launch_emf(gam_handle *h) {
@@ -1086,8 +1090,8 @@ static void launch_emf(gam_handle *h) {
             const int n[3] = {g.Nip + (ED != 0), g.Njp + (ED != 1), g.Nkp + (ED != 2)};
             const int T2 = (ED + 2) % 3, kc = flux_col_kc(n[T2], (long)(h->pack_share * n[0] * n[3 - T2]));
             const int ns = cdiv(n[T2], kc);
-            // I edges: 64 x 4 bricks, whose rows share the j stencils of the face velocities
-            const Tile tl = ED == 0 ? Tile{64, 4, 1, sizeof(R) == sizeof(float) ? 0 : TILE_NOXCD} : Tile{256, 1, 1, TILE_LINEAR};
+            // in columns only as one of several packed blocks: its own tile is the edge kernel's
+            const Tile tl = zones(h) >= EMF_COL_MIN ? h->tile[st] : emf_col_tile(h, ED);
             const dim3 gr((unsigned)tile_blocks(tl, n[0], T2 == 1 ? ns : n[1], T2 == 2 ? ns : n[2]));
             PLAUNCH(h, (k_emf_col<ED, RM, BO, R>), (b_emf_col<ED, RM, BO, R>), gr, 256, g, tl, h->mp, h->bgv, h->clk,
                     P<R>(h->wk[W_VDV]), P<R>(h->hGas), w.bn, w.bh, P<R>(h->E), h->corr, h->corr_scale, kc);
@@ -1847,7 +1851,6 @@ extern "C" int gam_graph_create_packed(gam_handle *const *hs, int n, int nsteps,
             return fail(h, -1, "gam_graph_create_packed: periodic MHD blocks only (no ring average, no correction)");
     }
     std::vector<std::vector<std::unique_ptr<PackRec>>> recs(n);
-    auto zones = [](const gam_handle *h) { return (double)h->gv.Nip * h->gv.Njp * h->gv.Nkp; };
     double all = 0.0;
     for (int q = 0; q < n; q++) all += zones(hs[q]);
     for (int q = 0; q < n; q++) {

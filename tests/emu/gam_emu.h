@@ -125,9 +125,13 @@ template <class F> inline void emu_launch_now(dim3 g, dim3 b, const F &f) {
             }
 }
 
+// set: sees the grid of every launch
+inline void (*emu_on_launch)(dim3) = nullptr;
+
 // The kernel arguments are evaluated once, at the launch, as HIP does; a
 // recorded launch keeps those values.
 template <class F, class... A> inline void emu_launch(dim3 g, dim3 b, F f, A... args) {
+    if (emu_on_launch) emu_on_launch(g);
     auto run = [g, b, f, args...]() { emu_launch_now(g, b, [&]() { f(args...); }); };
     if (emu_capture) emu_capture->push_back(run);
     else run();
