@@ -1075,8 +1075,11 @@ static void launch_flux(gam_handle *h, int d) {
 // Whether the I and K edges form their face velocities themselves (k_emf_col; speed
 // only).  Each of its columns starts with 7 more face velocities, so a launch must have
 // the lanes for long ones.  k_vf and the two EMFs, separate / folded in: 256^3 2.85 /
-// 2.30 ms (FP64), 1.44 / 1.19 (FP32); 9.4 M zones of FP32 0.92 / 0.79; 128^3 0.405 /
-// 0.406 (FP64), so the line lies between the last two.
+// 2.30 ms (FP64), 1.44 / 1.19 (FP32).  A whole step, separate / folded in, around the line,
+// FP64 and FP32 bulk: cubes of 128 cells 0.96 and 0.96, 144 0.96 and 0.95, 152 1.01 and
+// 0.97, 160 (4.1 M zones) 0.98 and 0.96, 168 1.02 and 1.02, 176 1.04 and 1.03, 192 1.02 and 1.03;
+// 4 cells deep, where the columns are 4 or 5 edges, 1.06 at 2 and at 4 M zones.  The rounds of
+// blocks that a size happens to fill count as much as the size: one line serves both.
 static bool emf_cols(const gam_handle *h) { return h->pack_share * zones(h) >= EMF_COL_MIN; }
 
 template <int ED, int RM, int BO, typename R>
@@ -1190,7 +1193,7 @@ static void launch_b2f(gam_handle *h, int st, const TM *mag, void *B) {
     launch_ring_bfix<R>(h, B);
 }
 
-// Mom2Face of the predictor state (FP64: 3 waves per SIMD, FP32: 5)
+// Mom2Face of the predictor state; columns for 4 waves per SIMD (resident: FP64 3, FP32 5)
 template <typename R>
 static void launch_vf(gam_handle *h, int what) {
     const GVT<R> &g = view<R>(h);

@@ -48,9 +48,10 @@ __global__ void k_fill(double *p, size_t n, double v) {
 // and the face triad (init.F90:873-906, doQuadFT = F).  POINTS: the sums point by
 // point, as the reference takes them; else through the moments of the area (the
 // same rule, other roundings).  FP32 bulk keeps the point sums here and in
-// k_volume: its step reads face and cell centres through differences rounded to
-// FP32 (k_b2f_coef), where the last bits of the FP64 centres flip single
-// roundings, and in a low-beta field those reach magFlux at 5e-9.  Bound by FP64
+// k_volume so that its results keep their bits, not for accuracy: its step reads face
+// and cell centres through differences rounded to FP32 (k_b2f_coef), where the last
+// bits of the FP64 centres flip single roundings (5e-9 of magFlux after a step of
+// a low-beta field, below FP32's own error).  Bound by FP64
 // issue (the square root): 0.75 -> 0.45 ms per launch at 128^3.
 template <bool POINTS>
 __global__ void __launch_bounds__(256) k_faces(GVw g, int d) {

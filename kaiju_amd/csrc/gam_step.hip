@@ -933,9 +933,11 @@ __global__ void __launch_bounds__(256) k_flux(GVT<R> g, Tile t, MP m, BGV bg, co
 // rings private to the thread (no barrier): in registers they cost the FP64
 // kernel its second wave per SIMD.  The next interface's points are loaded ahead
 // of this one's flux arithmetic and land during it; where the FP64 flux itself
-// needs the registers (Boris, background, correction: they would spill), after
-// it.  Bound by VALU issue, 1430 (FP64) and 1250 (FP32) vector instructions per
-// interface, 0.6 ms at 256^3.  Measured there, ms per launch j / k: FP32 bulk
+// needs the registers (Boris, background, correction), after it: Boris then still
+// spills up to 88 bytes per lane.  1430 (FP64) and 1250 (FP32) vector instructions per
+// interface take 0.61 and 0.53 ms at 256^3 at full issue: FP32 is bound by that, FP64 by
+// the latency of its loads and divisions as much, which two waves per SIMD do not hide.
+// Measured there, ms per launch j / k: FP32 bulk
 // 0.79 / 0.91 (one interface per thread, no windows) -> 0.64 / 0.65; FP64 1.37 / 1.46
 // (two interfaces along i per thread) -> 1.24 / 1.26.
 template <int DN, int RM, int BORIS, int MHD, int BG, typename R, int CORR = 0>
@@ -1034,8 +1036,8 @@ __global__ void __launch_bounds__(256) FLUX_COL_WAVES k_flux_col(GVT<R> g, Tile 
 // another writes.  Launched one by one each leaves most of the chip idle and waits for
 // the last block of the one before; together their blocks run side by side.
 // Block ranges first[q] .. first[q + 1] - 1 run body q over 256-point rows.
-// Bound by latency: six launches of 6-17 us on a 45x38x51 FP64 block (8CENT, Boris)
-// become one of 46 us, a step of it 176 -> 138 us; of a 32x32x4 box 133 -> 91 us.
+// Bound by latency: six launches of 9-17 us on a 45x38x51 FP64 block (8CENT, Boris)
+// become one of 46 us, a step among others 143 -> 108 us; of a 32x32x4 box 88 -> 45 us.
 struct MergeRanges { unsigned first[7]; };
 #define MERGE_TILE Tile{256, 1, 1, TILE_LINEAR | TILE_NOXCD}
 template <typename R>

@@ -25,9 +25,10 @@ import json
 import sys
 from collections import defaultdict
 
-# kernel-name prefix -> stage name used by the library's stage timers
+# kernel-name prefix -> stage name used by the library's stage timers (a small block's merged
+# launches: the stages they hold)
 STAGE_OF = [
-    ("k_predict", "predictor"), ("k_bc_b2f", "bcs"), ("k_b2f_vf", "mom2face"), ("k_emf_flux", "flux_i"), ("k_b2f_shell", "bflux_post"), ("k_b2f_rows", "ring"),
+    ("k_predict", "predictor"), ("k_bc_b2f", "bcs"), ("k_b2f_vf", "bflux_half+mom2face"), ("k_emf_flux", "emf+flux"), ("k_b2f_shell", "bflux_post"), ("k_b2f_rows", "ring"),
     ("k_b2f", "bflux_half"), ("k_ring_", "ring"), ("k_pole_e", "ring"), ("k_fix_e", "ring"),
     ("k_celldt_rows", "celldt"), ("k_bc_wind", "bcs"), ("k_wind_", "bcs"),
     ("k_vf", "mom2face"), ("k_emf_jcol", "emf_j"), ("k_emf<0", "emf_i"), ("k_emf<2", "emf_k"),
