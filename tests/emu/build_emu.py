@@ -30,7 +30,7 @@ def build(asan: bool = False, defs: tuple = (), main: str = "") -> str:
     src = os.path.join(HERE, main) if main else os.path.join(CSRC, "gam_api.hip")
     if os.path.exists(out) and os.path.getmtime(out) >= max(os.path.getmtime(s) for s in SRCS + [src]):
         return out
-    cmd = [_cxx(), "-std=c++17", "-O1", "-g", "-fPIC", *([] if main else ["-shared"]), "-DGAM_EMU", *("-D" + d for d in defs),
+    cmd = [_cxx(), "-std=c++17", *(["-O0"] if main else ["-O1", "-g", "-shared"]), "-fPIC", "-DGAM_EMU", *("-D" + d for d in defs),
            "-ffp-contract=off", "-fno-fast-math", "-x", "c++", "-I", os.path.join(ROOT, "include"), "-I", CSRC, "-I", HERE,
            src, "-o", out + ".tmp"]
     if asan:
